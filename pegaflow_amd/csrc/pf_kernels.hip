@@ -241,6 +241,9 @@ __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units
     c_u64* far_table =
         reinterpret_cast<c_u64*>(reinterpret_cast<uint64_t>(up->far_table) + (paged ? bias : 0));
     const uint64_t far_table_off = up->far_table_off;
+    // What segment 1 adds to a position's place in the table and to its base.
+    const uint32_t seg1_entries = up->far_table_step;
+    const uint64_t seg1_bytes = seg1_entries != 0 ? 0 : frag_bytes;
     const uint32_t tiles_per_frag = up->tiles_per_frag;
     const bool vec_ok = up->vec_ok != 0;
     const bool ids16 = up->ids16 != 0;
@@ -263,7 +266,8 @@ __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units
       const uint64_t near_addr = near_base + id * block_stride + (seg ? kv_stride : 0) + off;
       uint64_t far_addr;
       if (paged) {
-        far_addr = far_table[pos] + far_table_off + (seg ? frag_bytes : 0) + off;
+        far_addr = far_table[pos + (seg ? seg1_entries : 0)] + far_table_off +
+                   (seg ? seg1_bytes : 0) + off;
       } else {
         far_addr = (seg ? far_base1 : far_base0) + static_cast<uint64_t>(pos) * far_stride + off;
       }
@@ -332,14 +336,8 @@ __device__ __forceinline__ void block_tiles_copy(UnitPtr up, uint32_t row, uint3
   const uint64_t id = ids[pos];
   const uint64_t near_addr =
       up->near_base + id * up->block_stride + (seg ? up->kv_stride : 0) + off;
-  uint64_t far_addr;
-  if (up->far_table != nullptr) {
-    c_u64* far_table = reinterpret_cast<c_u64*>(reinterpret_cast<uint64_t>(up->far_table));
-    far_addr = far_table[pos] + up->far_table_off + (seg ? frag_bytes : 0) + off;
-  } else {
-    far_addr = (seg ? up->far_base[1] : up->far_base[0]) +
-               static_cast<uint64_t>(pos) * up->far_stride + off;
-  }
+  const uint64_t far_addr = (seg ? up->far_base[1] : up->far_base[0]) +
+                            static_cast<uint64_t>(pos) * up->far_stride + off;
   const uint64_t dst = TO_FAR ? far_addr : near_addr;
   const uint64_t src = TO_FAR ? near_addr : far_addr;
   const uint64_t left = frag_bytes - off;

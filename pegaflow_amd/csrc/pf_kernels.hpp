@@ -13,8 +13,11 @@ namespace pf {
 //
 // Fragment f = (segment s, list position i) covers
 //   near: near_base + ids[i]*block_stride + s*kv_stride          [frag_bytes]
-//   far : far_table ? far_table[i] + far_table_off + s*frag_bytes
+//   far : far_table ? far_table[i + s*far_table_step] + far_table_off
+//                       + (far_table_step ? 0 : s*frag_bytes)
 //                   : far_base[s] + i*far_stride                 [frag_bytes]
+// far_table_step = 0: segment 1 lies right behind segment 0; otherwise it has
+// bases of its own, far_table_step entries further on in the table.
 struct BlockUnit {
   uint64_t near_base;
   uint64_t block_stride;
@@ -31,7 +34,7 @@ struct BlockUnit {
   uint32_t tiles_per_frag;    // ceil(frag_bytes / tile_bytes)
   uint32_t vec_ok;            // every address and stride is 16-byte aligned
   uint32_t ids16;             // the id list holds 16-bit ids (zero-copy form only)
-  uint32_t reserved;
+  uint32_t far_table_step;    // entries between a position's bases of segment 0 and 1; 0 = one base
 };
 
 // Bytes one workgroup moves per tile for the given unroll (256 lanes x 16 B x U).

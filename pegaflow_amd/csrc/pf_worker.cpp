@@ -1,5 +1,6 @@
 #include "pf_worker.hpp"
 
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 
@@ -14,6 +15,12 @@ namespace {
 // The workers move KV beside a running model: a task whose dense layers add up
 // to this much is staged whatever the size of its layers (see run()).
 constexpr uint64_t kWorkerStagedCallBytes = 8ull << 20;
+// Layers whose blocks come from several saves are staged piece by piece when
+// the pieces lie in host memory in runs of this length on average: every run
+// is a link copy of its own, which costs ~22 us beyond its bytes behind a
+// kernel on the same stream (8 MiB: 146 us at link rate, so 50 of 57 GB/s).
+// Shorter runs cross with the zero-copy kernel, which does not care.
+constexpr uint64_t kStagedPieceRunBytes = 8ull << 20;
 }  // namespace
 
 bool build_copy_descs(const std::vector<LayerTransferData>& layers, std::vector<CopyDesc>* out,
@@ -116,9 +123,12 @@ namespace {
 // Storage for one task's block-ID form.
 struct BlockForm {
   std::vector<pf_layer_blocks> layers;
+  std::vector<SecondSegmentTable> second;  // one per entry of `layers`, or empty
   std::vector<std::vector<uint32_t>> ids;
   std::vector<std::vector<uint64_t>> page_host;
   std::vector<std::vector<uint64_t>> page_dev;
+  std::vector<std::vector<uint64_t>> page2_host;
+  std::vector<std::vector<uint64_t>> page2_dev;
   // Page tables of host images, one per distinct page list, so that the
   // layers of a page-first task pass the very same table.
   std::vector<const void*> image_pages;
@@ -128,20 +138,83 @@ struct BlockForm {
   uint64_t total_bytes = 0;
 };
 
+// A maximal run of list positions whose segments follow one another in host
+// memory without a gap.
+struct Piece {
+  size_t layer;  // index in the form
+  size_t first, count;
+  MappedPinnedPtr seg[2];
+};
+
+// Split layers that are not uniform into pieces, in host address order, if that
+// makes them worth staging: the order lets the pieces of one save cross the
+// link in one copy (its layers lie one behind the other).  Replaces those
+// layers of the form; the others follow unchanged.
+void stage_in_pieces(BlockForm* form, std::vector<Piece>* pieces, uint64_t staged_min_bytes) {
+  uint64_t bytes = 0;
+  std::vector<std::pair<const uint8_t*, uint64_t>> spans;
+  spans.reserve(pieces->size() * 2);
+  for (const Piece& p : *pieces) {
+    const pf_kv_layout& layout = form->layers[p.layer].layout;
+    for (uint32_t s = 0; s < (layout.split ? 2u : 1u); ++s) {
+      const uint64_t len = p.count * layout.segment_bytes;
+      spans.emplace_back(p.seg[s].host, len);
+      bytes += len;
+    }
+  }
+  if (bytes < staged_min_bytes) return;
+  std::sort(spans.begin(), spans.end());
+  uint64_t runs = spans.empty() ? 0 : 1;
+  for (size_t i = 1; i < spans.size(); ++i) {
+    runs += spans[i - 1].first + spans[i - 1].second != spans[i].first;
+  }
+  if (runs == 0 || bytes / runs < kStagedPieceRunBytes) return;
+  std::sort(pieces->begin(), pieces->end(),
+            [](const Piece& a, const Piece& b) { return a.seg[0].host < b.seg[0].host; });
+  std::vector<pf_layer_blocks> split;
+  std::vector<bool> replaced(form->layers.size(), false);
+  split.reserve(pieces->size() + form->layers.size());
+  for (const Piece& p : *pieces) {
+    replaced[p.layer] = true;
+    pf_layer_blocks lb = form->layers[p.layer];
+    const uint64_t frag = lb.layout.segment_bytes;
+    lb.block_ids += p.first;
+    lb.n_blocks = p.count;
+    lb.page_host = lb.page_host_device = nullptr;
+    for (uint32_t s = 0; s < (lb.layout.split ? 2u : 1u); ++s) {
+      lb.host[s] = p.seg[s].host;
+      lb.host_device[s] = reinterpret_cast<uint64_t>(p.seg[s].device);
+      lb.host_len[s] = p.count * frag;
+    }
+    lb.host_stride = frag;
+    split.push_back(lb);
+  }
+  std::vector<SecondSegmentTable> second(split.size());
+  for (size_t i = 0; i < form->layers.size(); ++i) {
+    if (replaced[i]) continue;
+    split.push_back(form->layers[i]);
+    second.push_back(form->second[i]);
+  }
+  form->layers = std::move(split);
+  form->second = std::move(second);
+}
+
 // Express the task through block ids: per layer either a uniform-stride host
-// image or a per-block base table.  Returns false when some layer fits
-// neither form (e.g. K and V of each block in unrelated allocations); the
-// caller then falls back to per-fragment descriptors.  Errors are reported
-// through *err with *failed = true.
+// image, the dense pieces it consists of, or per-block base tables.  Errors are
+// reported through *err with a false return.  `staged_min_bytes`: from how many
+// bytes on a task of pieces is staged (UINT64_MAX = never).
 bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begin, size_t end,
-                   BlockForm* out, bool* failed, std::string* err) {
-  *failed = false;
+                   uint64_t staged_min_bytes, BlockForm* out, std::string* err) {
   const size_t n_layers = end - begin;
   out->layers.resize(n_layers);
+  out->second.resize(n_layers);
   out->ids.resize(n_layers);
   out->page_host.resize(n_layers);
   out->page_dev.resize(n_layers);
+  out->page2_host.resize(n_layers);
+  out->page2_dev.resize(n_layers);
   out->layer_table.assign(n_layers, -1);
+  std::vector<Piece> pieces;
   for (size_t li = 0; li < n_layers; ++li) {
     const LayerTransferData& layer = all_layers[begin + li];
     pf_layer_blocks& lb = out->layers[li];
@@ -172,7 +245,6 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
       }
       if (!im.pages || im.pages->size() != n_im) {
         *err = "layer " + layer.layer_name + ": host image has a page list of the wrong length";
-        *failed = true;
         return false;
       }
       size_t ti = 0;
@@ -204,14 +276,12 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
       if (tb.block_idx >= layer.layout.num_blocks()) {
         *err = "layer " + layer.layer_name + ": block " + std::to_string(tb.block_idx) +
                " out of range (" + std::to_string(layer.layout.num_blocks()) + " blocks)";
-        *failed = true;
         return false;
       }
       ids[i] = static_cast<uint32_t>(tb.block_idx);
       const RawBlock* raw = tb.block.raw;
       if (!raw || !raw->segment_mapped_ptr(0, &k[i])) {
         *err = "layer " + layer.layer_name + ": host block has no segment 0";
-        *failed = true;
         return false;
       }
       k[i] = k[i].add(tb.block.offset);
@@ -255,12 +325,35 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
       lb.host_stride = stride;
       continue;
     }
-    // Per-block bases: needs V right behind K when split.
-    bool table_ok = true;
-    for (size_t i = 0; table_ok && split && i < n; ++i) {
-      table_ok = v[i].host == k[i].host + frag && v[i].device == k[i].device + frag;
+    // Blocks of several saves: K and V of a block usually lie apart.
+    bool v_behind_k = true;
+    for (size_t i = 0; v_behind_k && split && i < n; ++i) {
+      v_behind_k = v[i].host == k[i].host + frag && v[i].device == k[i].device + frag;
     }
-    if (!table_ok) return false;
+    if (!v_behind_k) {
+      for (size_t i = 0; i < n; ++i) {
+        if (i != 0) {
+          Piece& last = pieces.back();
+          if (k[i].host == last.seg[0].host + last.count * frag &&
+              k[i].device == last.seg[0].device + last.count * frag &&
+              v[i].host == last.seg[1].host + last.count * frag &&
+              v[i].device == last.seg[1].device + last.count * frag) {
+            ++last.count;
+            continue;
+          }
+        }
+        pieces.push_back({li, i, 1, {k[i], v[i]}});
+      }
+      std::vector<uint64_t>& vh = out->page2_host[li];
+      std::vector<uint64_t>& vd = out->page2_dev[li];
+      vh.resize(n);
+      vd.resize(n);
+      for (size_t i = 0; i < n; ++i) {
+        vh[i] = reinterpret_cast<uint64_t>(v[i].host);
+        vd[i] = reinterpret_cast<uint64_t>(v[i].device);
+      }
+      out->second[li] = {vh.data(), vd.data()};
+    }
     std::vector<uint64_t>& ph = out->page_host[li];
     std::vector<uint64_t>& pd = out->page_dev[li];
     ph.resize(n);
@@ -272,7 +365,7 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
     lb.page_host = ph.data();
     lb.page_host_device = pd.data();
     lb.page_offset = 0;
-    lb.page_len = frag * (split ? 2 : 1);
+    lb.page_len = frag * (split && v_behind_k ? 2 : 1);
   }
   for (size_t li = 0; li < n_layers; ++li) {
     const int ti = out->layer_table[li];
@@ -280,6 +373,7 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
     out->layers[li].page_host = out->image_page_host[ti].data();
     out->layers[li].page_host_device = out->image_page_dev[ti].data();
   }
+  if (!pieces.empty()) stage_in_pieces(out, &pieces, staged_min_bytes);
   return true;
 }
 
@@ -718,6 +812,10 @@ void GpuWorkerPool::run(Worker* w, bool is_load, NumaNode numa, std::promise<Tas
   // transfers are staged (their link crossing needs no compute unit, so model
   // kernels beside them keep their rate), small and scattered ones go zero-copy.
   const int path = mode_ == TransferMode::ZeroCopy ? PF_PATH_ZEROCOPY : PF_PATH_AUTO;
+  const uint64_t staged_min_bytes =
+      path == PF_PATH_ZEROCOPY ? UINT64_MAX
+      : options_.auto_staged_min_bytes != 0 ? options_.auto_staged_min_bytes
+                                             : kWorkerStagedCallBytes;
 
   for (;;) {
     std::unique_ptr<Task> task;
@@ -777,25 +875,22 @@ void GpuWorkerPool::run(Worker* w, bool is_load, NumaNode numa, std::promise<Tas
       const size_t end = (begin == 0 || !xfer)
                              ? (begin + first_part < n_layers ? begin + first_part : n_layers)
                              : n_layers;
-      bool done_fast = false;
       if (xfer) {
         BlockForm form;
-        bool failed = false;
         const auto t_convert = std::chrono::steady_clock::now();
-        const bool converted = to_block_form(task->layers, begin, end, &form, &failed, &err);
+        const bool converted = to_block_form(task->layers, begin, end, staged_min_bytes, &form, &err);
         res.convert_ms += since(t_convert);
         if (converted) {
-          st = is_load ? xfer->load(form.layers.data(), form.layers.size(), path, stream)
-                       : xfer->save(form.layers.data(), form.layers.size(), path, stream);
+          st = is_load ? xfer->load(form.layers.data(), form.layers.size(), path, stream,
+                                    form.second.data())
+                       : xfer->save(form.layers.data(), form.layers.size(), path, stream,
+                                    form.second.data());
           if (st != PF_OK) err = last_error();
           res.bytes += form.total_bytes;
-          done_fast = true;
-        } else if (failed) {
+        } else {
           st = PF_ERR_STORAGE;
-          done_fast = true;
         }
-      }
-      if (!done_fast) {
+      } else {
         std::vector<CopyDesc> copies;
         uint64_t total = 0;
         const auto t_convert = std::chrono::steady_clock::now();

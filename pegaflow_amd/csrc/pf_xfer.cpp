@@ -50,10 +50,13 @@ struct LayerPlan {
   uint64_t host_stride = 0;
   const uint64_t* page_dev = nullptr;  // device-visible page bases, host array
   const uint64_t* page_host = nullptr; // host addresses of the same pages
+  const uint64_t* page2_dev = nullptr; // bases of segment 1 when it does not follow segment 0
   uint64_t page_offset = 0;
   bool staged = false;
   bool dense = false;           // uniform host image at the fragment's own stride
   bool vec_ok = false;
+  bool ids_owner = false;       // this plan fills its id list's region of the slab
+  bool table_owner = false;     // ... and its page table's
   uint64_t ids_slab_off = 0;    // byte offset of the id list inside the slab
   uint64_t table_slab_off = 0;  // byte offset of the page table inside the slab
   uint64_t order_slab_off = 0;  // byte offset of the row order inside the slab (staged loads)
@@ -224,8 +227,8 @@ int Xfer::last_kernel_ms(float* out_ms, uint32_t* out_launches) {
   return PF_OK;
 }
 
-int Xfer::plan_layer(const pf_layer_blocks& in, size_t index, int path, LayerPlan* out,
-                     bool* skip) {
+int Xfer::plan_layer(const pf_layer_blocks& in, const SecondSegmentTable& second, size_t index,
+                     int path, LayerPlan* out, bool* skip) {
   LayerPlan& p = *out;
   p.src_index = index;
   p.name = in.layer_name ? in.layer_name : ("#" + std::to_string(index));
@@ -267,22 +270,26 @@ int Xfer::plan_layer(const pf_layer_blocks& in, size_t index, int path, LayerPla
       return fail(PF_ERR_INVALID_ARGUMENT,
                   "layer %s: page_host and page_host_device must both be set", p.name.c_str());
     }
+    const bool apart = p.n_seg == 2 && second.host != nullptr && second.device != nullptr;
+    const uint64_t slice = p.frag_bytes * (apart ? 1 : p.n_seg);
     uint64_t need = 0;
-    if (__builtin_add_overflow(in.page_offset, p.frag_bytes * p.n_seg, &need) ||
-        need > in.page_len) {
+    if (__builtin_add_overflow(in.page_offset, slice, &need) || need > in.page_len) {
       return fail(PF_ERR_INVALID_ARGUMENT,
                   "layer %s: page slice [%llu, +%llu) exceeds page length %llu", p.name.c_str(),
                   static_cast<unsigned long long>(in.page_offset),
-                  static_cast<unsigned long long>(p.frag_bytes * p.n_seg),
+                  static_cast<unsigned long long>(slice),
                   static_cast<unsigned long long>(in.page_len));
     }
     for (uint64_t i = 0; i < p.n_blocks; ++i) {
-      if (in.page_host[i] == 0 || in.page_host_device[i] == 0) {
+      if (in.page_host[i] == 0 || in.page_host_device[i] == 0 ||
+          (apart && (second.host[i] == 0 || second.device[i] == 0))) {
         return fail(PF_ERR_INVALID_ARGUMENT, "layer %s: page %llu has a null base",
                     p.name.c_str(), static_cast<unsigned long long>(i));
       }
-      far_aligned = far_aligned && aligned16(in.page_host_device[i]);
+      far_aligned = far_aligned && aligned16(in.page_host_device[i]) &&
+                    (!apart || aligned16(second.device[i]));
     }
+    if (apart) p.page2_dev = second.device;
     far_aligned = far_aligned && aligned16(in.page_offset);
     p.page_dev = in.page_host_device;
     p.page_host = in.page_host;
@@ -323,7 +330,8 @@ int Xfer::plan_layer(const pf_layer_blocks& in, size_t index, int path, LayerPla
   // A fragment size that is not a multiple of 16 is fine for the vector path
   // (the kernel copies the tail bytewise) as long as every fragment START is
   // aligned, which the stride checks above guarantee.
-  p.vec_ok = near_aligned && far_aligned && (p.n_seg == 1 || !paged || aligned16(p.frag_bytes));
+  p.vec_ok = near_aligned && far_aligned &&
+             (p.n_seg == 1 || !paged || p.page2_dev != nullptr || aligned16(p.frag_bytes));
 
   const bool dense = !paged && in.host_stride == p.frag_bytes;
   p.dense = dense;
@@ -636,10 +644,10 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
 }
 
 int Xfer::run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save,
-              hipStream_t s) {
+              hipStream_t s, const SecondSegmentTable* second) {
   began_ = false;
   staging_oom_ = false;
-  int st = run_impl(layers, n_layers, path, save, s);
+  int st = run_impl(layers, n_layers, path, save, s, second);
   if (st != PF_OK && !began_ && staging_oom_ && path == PF_PATH_AUTO) {
     // The device has no memory left for a staging slot (slots allocated on
     // first use, or grown for an oversized block).  Nothing is enqueued yet,
@@ -654,7 +662,7 @@ int Xfer::run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool s
     }
     (void)hipGetLastError();
     began_ = false;
-    st = run_impl(layers, n_layers, PF_PATH_ZEROCOPY, save, s);
+    st = run_impl(layers, n_layers, PF_PATH_ZEROCOPY, save, s, second);
   }
   if (st != PF_OK && began_) {
     // Something was already enqueued, possibly on the side stream, which the
@@ -731,7 +739,7 @@ FillPlan plan_staged_fills(const std::vector<FillLayer>& layers, uint64_t slot_b
 }
 
 int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save,
-                   hipStream_t s) {
+                   hipStream_t s, const SecondSegmentTable* second) {
   if (!timing_in_place_) timing_used_ = 0;
   if (n_layers == 0) return PF_OK;
   if (!layers) return fail(PF_ERR_INVALID_ARGUMENT, "layers must not be null");
@@ -748,7 +756,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   for (uint64_t li = 0; li < n_layers; ++li) {
     LayerPlan p;
     bool skip = false;
-    int st = plan_layer(layers[li], li, path, &p, &skip);
+    int st = plan_layer(layers[li], second ? second[li] : SecondSegmentTable(), li, path, &p, &skip);
     if (st != PF_OK) return st;
     if (!skip) plans.push_back(std::move(p));
   }
@@ -850,12 +858,15 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     slab_bytes = unit_refs.size() * sizeof(BlockUnit);
     slab_bytes = (slab_bytes + 255) & ~255ull;
     order_bytes = 0;
+    // Plans whose id list is in the slab: a call of many layers (times the
+    // pieces of a layer) has few distinct lists, so only these are compared.
+    std::vector<size_t> id_owners;
     for (size_t pi = 0; pi < plans.size(); ++pi) {
       LayerPlan& p = plans[pi];
       p.ordered = p.order_owner = p.order_shared = false;
-      // Layers that pass the very same id array share one upload.
+      // Layers that pass the same ids share one upload.
       bool shared = false;
-      for (size_t pj = 0; pj < pi; ++pj) {
+      for (size_t pj : id_owners) {
         if (plans[pj].n_blocks == p.n_blocks &&
             (plans[pj].ids == p.ids ||
              std::memcmp(plans[pj].ids, p.ids, p.n_blocks * sizeof(uint32_t)) == 0)) {
@@ -864,7 +875,9 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
           break;
         }
       }
+      p.ids_owner = !shared;
       if (!shared) {
+        id_owners.push_back(pi);
         p.ids_slab_off = slab_bytes;
         slab_bytes += (p.n_blocks * id_bytes + 255) & ~255ull;
       }
@@ -873,7 +886,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (!save && p.staged && p.n_blocks > 1 && p.layer_bytes >= kRowOrderFromBytes) {
         p.ordered = true;
         for (size_t pj = 0; pj < pi; ++pj) {
-          if (plans[pj].ordered && plans[pj].ids_slab_off == p.ids_slab_off &&
+          if (plans[pj].order_owner && plans[pj].ids_slab_off == p.ids_slab_off &&
               plans[pj].units == p.units) {
             p.order_slab_off = plans[pj].order_slab_off;
             p.order_shared = true;
@@ -889,7 +902,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (p.page_dev) {
         bool tshared = false;
         for (size_t pj = 0; pj < pi; ++pj) {
-          if (plans[pj].page_dev == p.page_dev && plans[pj].n_blocks == p.n_blocks) {
+          if (plans[pj].page_dev == p.page_dev && plans[pj].page2_dev == p.page2_dev &&
+              plans[pj].n_blocks == p.n_blocks) {
             p.table_slab_off = plans[pj].table_slab_off;
             tshared = true;
             break;
@@ -897,8 +911,9 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         }
         if (!tshared) {
           p.table_slab_off = slab_bytes;
-          slab_bytes += (p.n_blocks * sizeof(uint64_t) + 255) & ~255ull;
+          slab_bytes += (p.n_blocks * sizeof(uint64_t) * (p.page2_dev ? 2 : 1) + 255) & ~255ull;
         }
+        p.table_owner = !tshared;
       }
     }
   };
@@ -935,6 +950,12 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   const uint64_t slab_dev = in_args ? 0 : reinterpret_cast<uint64_t>(slab->dev);
   for (size_t pi = 0; pi < plans.size(); ++pi) {
     LayerPlan& p = plans[pi];
+    if (p.page_dev && p.table_owner) {
+      uint64_t* table = reinterpret_cast<uint64_t*>(slab_host + p.table_slab_off);
+      std::memcpy(table, p.page_dev, p.n_blocks * sizeof(uint64_t));
+      if (p.page2_dev) std::memcpy(table + p.n_blocks, p.page2_dev, p.n_blocks * sizeof(uint64_t));
+    }
+    if (!p.ids_owner) continue;
     if (ids16) {
       uint16_t* narrow = reinterpret_cast<uint16_t*>(slab_host + p.ids_slab_off);
       for (uint64_t i = 0; i < p.n_blocks; ++i) narrow[i] = static_cast<uint16_t>(p.ids[i]);
@@ -942,9 +963,6 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (p.n_blocks & 1) narrow[p.n_blocks] = 0;
     } else {
       std::memcpy(slab_host + p.ids_slab_off, p.ids, p.n_blocks * sizeof(uint32_t));
-    }
-    if (p.page_dev) {
-      std::memcpy(slab_host + p.table_slab_off, p.page_dev, p.n_blocks * sizeof(uint64_t));
     }
   }
 
@@ -996,6 +1014,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (p.page_dev) {
         u.far_table = reinterpret_cast<const uint64_t*>(slab_dev + p.table_slab_off);
         u.far_table_off = p.page_offset;
+        u.far_table_step = p.page2_dev ? static_cast<uint32_t>(p.n_blocks) : 0;
       } else {
         u.far_base[0] = p.host_dev[0];
         u.far_base[1] = p.host_dev[1];

@@ -137,6 +137,13 @@ struct XferProfile {
   double device_ms = 0;         // first command -> last command
 };
 
+// Host bases of segment 1 of a paged layer, one per list position, for images
+// whose K and V of a block lie apart; null = segment 1 follows segment 0.
+struct SecondSegmentTable {
+  const uint64_t* host = nullptr;
+  const uint64_t* device = nullptr;  // device-visible
+};
+
 class Xfer {
  public:
   explicit Xfer(const pf_xfer_config* cfg) {
@@ -223,14 +230,18 @@ class Xfer {
     side_owned_ = side == nullptr;
   }
 
-  int run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save, hipStream_t s);
+  // `second`: null, or n_layers entries.
+  int run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save, hipStream_t s,
+          const SecondSegmentTable* second = nullptr);
   int run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save,
-               hipStream_t s);
-  int save(const pf_layer_blocks* layers, uint64_t n_layers, int path, hipStream_t s) {
-    return run(layers, n_layers, path, true, s);
+               hipStream_t s, const SecondSegmentTable* second);
+  int save(const pf_layer_blocks* layers, uint64_t n_layers, int path, hipStream_t s,
+           const SecondSegmentTable* second = nullptr) {
+    return run(layers, n_layers, path, true, s, second);
   }
-  int load(const pf_layer_blocks* layers, uint64_t n_layers, int path, hipStream_t s) {
-    return run(layers, n_layers, path, false, s);
+  int load(const pf_layer_blocks* layers, uint64_t n_layers, int path, hipStream_t s,
+           const SecondSegmentTable* second = nullptr) {
+    return run(layers, n_layers, path, false, s, second);
   }
 
   void set_layer_events(pf_event_t* events, uint64_t n) {
@@ -288,7 +299,8 @@ class Xfer {
   bool plan_page_pack(const std::vector<LayerPlan>& plans, bool save, PagePack* out);
   int run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uint64_t n_layers,
                     bool save, hipStream_t s);
-  int plan_layer(const pf_layer_blocks& in, size_t index, int path, LayerPlan* out, bool* skip);
+  int plan_layer(const pf_layer_blocks& in, const SecondSegmentTable& second, size_t index,
+                 int path, LayerPlan* out, bool* skip);
   int ensure_slot(Slot& sl, uint64_t bytes);
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,

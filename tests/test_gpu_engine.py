@@ -1064,3 +1064,50 @@ def test_engine_load_profile_and_staging_report(gpu):
     register(z, "kernel-as-reference", zlayers, mode=TransferMode.KERNEL)
     assert z.staging_bytes == 0
     z.close()
+
+
+@pytest.mark.parametrize("seg,turns,n_layers,paths", [
+    (4096, (3, 1, 2), 2, ("zerocopy",)),                 # small: per-block bases of K and V
+    (1000, (5, 1, 9), 3, ("zerocopy",)),                 # off 16-byte boundaries, pool padding
+    (1000, (4000, 1, 3999), 2, ("zerocopy",)),           # 32 MB in padded images: no long runs
+    (32768, (1,) * 160, 1, ("zerocopy",)),               # 10 MiB in one-block saves
+    (32768, (150, 149, 1), 2, ("staged", "zerocopy")),   # a last piece of one 64 KiB block
+    (16384, (600, 599), 3, ("staged",)),
+    (1040, (9000, 8000), 1, ("staged",)),
+], ids=lambda v: "x".join(map(str, v[:3])) if isinstance(v, tuple) else str(v))
+def test_load_of_blocks_from_several_saves(gpu, seg, turns, n_layers, paths):
+    """A prefix whose blocks were stored by several saves: K and V of its blocks
+    lie in as many buffers.  Every byte of the cache is compared, and the load
+    takes the block-ID forms, not descriptors."""
+    n = sum(turns)
+    nb = 2 * n + 3
+    rng = np.random.default_rng(seg + n)
+    e = PegaEngine(pool_size=(4 * n_layers * n * max(seg, 1024)) + (8 << 20))
+    caches = [random_bytes(rng, 2 * nb * seg) for _ in range(n_layers)]
+    devs = [DeviceBuffer(c.nbytes) for c in caches]
+    for d, c in zip(devs, caches):
+        d.copy_from_host(c)
+    names = [f"l{i}" for i in range(n_layers)]
+    e.register_context_layer_batch("t", "ns", 0, 0, 0, 1, 1, names, [d.ptr for d in devs],
+                                   [c.nbytes for c in caches], [nb] * n_layers, [seg] * n_layers,
+                                   [nb * seg] * n_layers, [2] * n_layers)
+    hashes = [i.to_bytes(8, "little") for i in range(n)]
+    ids = rng.permutation(nb)
+    src, dst = ids[:n], ids[n:2 * n]
+    at = 0
+    for t in turns:
+        e.batch_save_kv_blocks("t", 0, 0, 0, [LayerSave(m, src[at:at + t].tolist(), hashes[at:at + t])
+                                              for m in names])
+        at += t
+    hits, lease = e.query_prefix("t", hashes)
+    assert hits == n
+    res = e.batch_load_kv_blocks_multi_layer("t", 0, 0, [names], lease, [dst.tolist()]).wait()
+    assert set(res.paths) <= set(paths) and res.bytes == 2 * n * seg * n_layers
+    assert res.zero_copy_launches or "staged" in res.paths
+    for d, c in zip(devs, caches):
+        want = c.reshape(2, nb, seg).copy()
+        want[:, dst] = want[:, src]
+        assert np.array_equal(d.copy_to_host(), want.reshape(-1))
+    e.close()
+    for d in devs:
+        d.close()
