@@ -578,7 +578,8 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   }
 
   // Before anything of this call is on `s`: the check wants the stream idle.
-  if (use_side_stream(chunks.size())) {
+  const bool on_side = use_side_stream(chunks.size(), n * pack.page_bytes);
+  if (on_side) {
     const int side_status = ensure_side_stream(s);
     if (side_status != PF_OK) return side_status;
   }
@@ -586,7 +587,7 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   const Clock::time_point t_enqueue = Clock::now();
   prof_mark_begin(s);
   PF_HIP(hipMemcpyAsync(slab->dev, slab->host, slab_bytes, hipMemcpyHostToDevice, s));
-  hipStream_t side = use_side_stream(chunks.size()) ? side_ : s;
+  hipStream_t side = on_side ? side_ : s;
   if (side != s) {
     PF_HIP(hipEventRecord(fork_, s));
     PF_HIP(hipStreamWaitEvent(side, fork_, 0));
@@ -1028,10 +1029,13 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   // ---- 4. enqueue ---------------------------------------------------------
   // A second stream pays off when the link copies of one fill can overlap the
   // gather of the next: count the fills.
-  size_t staged_units = 0;
-  for (size_t ge : group_end) staged_units += ge != 0 ? 1 : 0;
+  size_t fills = 0;
+  for (size_t ge : group_end) fills += ge != 0 ? 1 : 0;
+  uint64_t staged_bytes = 0;
+  for (const LayerPlan& p : plans) staged_bytes += p.staged ? p.layer_bytes : 0;
+  const bool on_side = use_side_stream(fills, staged_bytes);
   // Before anything of this call is on `s`: the check wants the stream idle.
-  if (use_side_stream(staged_units)) {
+  if (on_side) {
     const int side_status = ensure_side_stream(s);
     if (side_status != PF_OK) return side_status;
   }
@@ -1062,7 +1066,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   };
   // With kernel timing on, the DMA copies run on the caller's stream too, so
   // that every timed kernel executes alone (a measurement mode: no overlap).
-  hipStream_t side = use_side_stream(staged_units) ? side_ : s;
+  hipStream_t side = on_side ? side_ : s;
   bool side_used = false;
   auto fork_side = [&]() -> int {
     if (side_used || side == s) return PF_OK;

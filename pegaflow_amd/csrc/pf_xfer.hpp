@@ -101,6 +101,8 @@ struct FillPlan {
 };
 FillPlan plan_staged_fills(const std::vector<FillLayer>& layers, uint64_t slot_bytes,
                            uint64_t group_cap, bool may_split, uint64_t max_unit_blocks);
+// Average fill from which on the link copies of a call go to a side stream.
+constexpr uint64_t kSideStreamFillBytes = 64ull << 20;
 constexpr int kDefaultUnroll = 4;
 // Zero-copy launches are capped to a few workgroups: the host link, not the
 // GPU, is the bound, and every workgroup that stays resident for the length of
@@ -346,17 +348,22 @@ class Xfer {
   bool timing_ = false;
   bool timing_in_place_ = false;
   bool began_ = false;  // the current call has enqueued work
-  uint32_t copy_stream_ = 0;  // 0 = by unit count, 1 = side stream, 2 = caller's stream
-  // A second stream pays off only when the copy of one unit can overlap the
-  // gather of the next.  Measured on MI355X (Llama layer shape, one call then
-  // a synchronise): a single unit of 4 / 16 / 64 / 312 MiB moves at 33.6 /
-  // 48.7 / 54.3 / 56.0 GB/s in order on the caller's stream against 24.8 /
-  // 44.4 / 52.8 / 55.6 GB/s with the hand-off to a side stream; from two
-  // units on the side stream wins (56.6 against 55.8 GB/s at 32 units).
-  bool use_side_stream(size_t staged_units) const {
+  uint32_t copy_stream_ = 0;  // 0 = by number and size of the fills, 1 = side stream, 2 = caller's stream
+  // A second stream pays off only when the copy of one fill can overlap the
+  // gather of the next, and only when the fills are large.  Its cross-stream
+  // waits cost the submitting thread ~30 us per fill instead of 7, and with
+  // many short fills under way the runtime deals their copies to whichever
+  // engine is idle when they are enqueued, some of which move 12 GB/s.  Measured
+  // on MI355X, calls back to back / one call then a synchronise, GB/s, side
+  // stream against in order: 32 loads of 20 MB with layer events 44.4 / 53.3
+  // against 52.4 / 51.6; fills of 41 MB with zero-copy layers between them 35.5
+  // / 54.4 against 54.2 / 53.6; 8 saves of 21 MB 39.1 / 51.3 against 52.0 /
+  // 50.9; from 64 MB fills on it is the faster one both ways (55.2 / 54.9
+  // against 54.7 / 54.4; 131 MB 56.0 / 55.8 against 55.4 / 55.2).
+  bool use_side_stream(size_t fills, uint64_t staged_bytes) const {
     if ((timing_ && !timing_in_place_) || copy_stream_ == 2) return false;
     if (copy_stream_ == 1) return true;
-    return staged_units > 1;
+    return fills > 1 && staged_bytes / fills >= kSideStreamFillBytes;
   }
   std::vector<std::pair<hipEvent_t, hipEvent_t>> timing_pool_;
   size_t timing_used_ = 0;
