@@ -31,10 +31,17 @@ struct BlockUnit {
   uint64_t far_table_off;
   uint32_t n_blocks;
   uint32_t n_seg;             // fragments per block: 1 or 2
-  uint32_t tiles_per_frag;    // ceil(frag_bytes / tile_bytes)
-  uint32_t vec_ok;            // every address and stride is 16-byte aligned
+  uint32_t tiles_per_frag;    // ceil(frag_bytes / tile_bytes); kUnitChunks: 16-byte chunks of one
+  uint32_t form;              // UnitForm
   uint32_t ids16;             // the id list holds 16-bit ids (zero-copy form only)
   uint32_t far_table_step;    // entries between a position's bases of segment 0 and 1; 0 = one base
+};
+
+// How a unit's fragments are cut up.
+enum UnitForm : uint32_t {
+  kUnitAny = 0,     // tiles of one fragment, no alignment assumed
+  kUnitVec = 1,     // tiles of one fragment, every address and stride 16-byte aligned
+  kUnitChunks = 2,  // zero-copy only: 16-byte chunks of consecutive fragments share a tile
 };
 
 // Bytes one workgroup moves per tile for the given unroll (256 lanes x 16 B x U).

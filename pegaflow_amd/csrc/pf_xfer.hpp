@@ -304,6 +304,7 @@ class Xfer {
   int plan_layer(const pf_layer_blocks& in, const SecondSegmentTable& second, size_t index,
                  int path, LayerPlan* out, bool* skip);
   int ensure_slot(Slot& sl, uint64_t bytes);
+  uint32_t chunks_per_fragment(const LayerPlan& p, const BlockUnit& u) const;
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
                      uint64_t min_frag_bytes, bool to_far, hipStream_t s);

@@ -115,6 +115,35 @@ def test_unaligned_and_odd_sizes_match_oracle(backends, stream, direction):
     host.close()
 
 
+@pytest.mark.parametrize("direction", ["h2d", "d2h"])
+@pytest.mark.parametrize("n, slot", [(70, 2080), (1300, 2080), (1300, 4128), (70, 16416), (9, 70000)])
+def test_rows_of_any_size_and_alignment(backends, stream, n, slot, direction):
+    """Row per wavefront (rows of at most 2 KiB) and row per workgroup, every alignment of both sides modulo 16,
+    sizes from one byte to a byte below, at and above a tile: only the fragments'
+    bytes change."""
+    rng = np.random.default_rng(n + slot)
+    top = slot - 32
+    sizes = rng.integers(1, top + 1, size=n)
+    edges = [1, 15, 16, 17, 31, 32, 33, 1023, 1024, 1025, top - 1, top]
+    sizes[:len(edges[:n])] = edges[:n]
+    rows = [(i * slot + i % 16, i * slot + (i // 16 + i) % 16, int(size)) for i, size in enumerate(sizes)]
+    total = slot * n
+    dev0, host0 = random_bytes(rng, total), random_bytes(rng, total)
+    exp_dev, exp_host = _oracle_expect(dev0, host0, rows, host_is_src=(direction == "h2d"))
+    host = PinnedMemory(total)
+    dev = DeviceBuffer(total)
+    for b in backends:
+        host.as_numpy()[:] = host0
+        dev.copy_from_host(dev0)
+        descs = [CopyDesc(dev.ptr + d, host.host_ptr + h, host.device_ptr + h, s) for d, h, s in rows]
+        getattr(b, direction)(descs, stream)
+        stream.synchronize()
+        assert np.array_equal(dev.copy_to_host(), exp_dev), b.name
+        assert np.array_equal(host.as_numpy(), exp_host), b.name
+    dev.close()
+    host.close()
+
+
 @pytest.mark.parametrize("n", [4096, 16385, 40001])
 def test_shuffled_4k_fragments(backends, stream, n):
     """Shape of the reference's transfer bench (benches/transfer_h2d.rs):

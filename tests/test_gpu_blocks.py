@@ -169,6 +169,38 @@ def test_save_load_matches_oracle(name, path, xfer, stream):
         case.close()
 
 
+# Zero-copy units cut into 16-byte chunks: the smallest fragment that has one,
+# fragments around the sizes where another form takes over (16 bytes, 8 KiB on
+# the 16-byte grid), segments of 1023, 1024 and 1025 chunks (a tile holds 1024)
+# and a last tile with chunks for one wavefront only; aligned and not, dense and
+# padded.
+CHUNKS = {
+    "15_bytes_no_chunk": dict(num_blocks=40, seg=15, segments=2),
+    "16_bytes": dict(num_blocks=300, seg=16, segments=2, n_ids=257),
+    "17_bytes": dict(num_blocks=300, seg=17, segments=2, n_ids=255),
+    "1023_chunks": dict(num_blocks=40, seg=528, segments=1, n_ids=31),
+    "1024_chunks": dict(num_blocks=40, seg=512, segments=2, n_ids=32),
+    "1025_chunks": dict(num_blocks=30, seg=656, segments=1, n_ids=25),
+    "one_wave_in_the_last_tile": dict(num_blocks=80, seg=272, segments=2, n_ids=64),
+    "padded_odd": dict(num_blocks=60, seg=1332, segments=2, pad_to=512),
+    "off_grid_base": dict(num_blocks=60, seg=1040, segments=2, base_off=7),
+    "below_8k": dict(num_blocks=20, seg=8176, segments=2),
+    "at_8k": dict(num_blocks=20, seg=8192, segments=2),
+    "off_grid_40k": dict(num_blocks=12, seg=40003, segments=2, base_off=1),
+}
+
+
+@pytest.mark.parametrize("name, path", [
+    (name, path) for name in sorted(CHUNKS) for path in (ZC, ST)
+    if path == ZC or "pad_to" not in CHUNKS[name]])  # the staged path needs a dense host image
+def test_chunked_units_match_oracle(name, path, xfer, stream):
+    case = Case(np.random.default_rng(zlib.crc32(name.encode())), **CHUNKS[name])
+    try:
+        _roundtrip(case, xfer, stream, path)
+    finally:
+        case.close()
+
+
 def _random_case_kwargs(rng):
     """A valid layout drawn at random: contiguous or split, dense / strided /
     interleaved, aligned or not, fragment sizes with and without a 16-byte
