@@ -86,7 +86,9 @@ __device__ __forceinline__ void store16_sc1_nt(__amdgpu_buffer_rsrc_t tile, uint
 // the load of its value to be open from then on, and starts the next tile (or
 // unit) by waiting for everything in flight, the stores of this one included
 // (a link trip per unit: 72 x 2 fragments of 12 096 bytes of two layers saved in
-// 66.3 us instead of 64.5).
+// 66.3 us instead of 64.5).  For saves: the stores of a load go to HBM, where
+// letting the first of them out before the last load is back is worth more
+// (fragments of 1000 bytes loaded at 55.1 GB/s, with this wait at 53.0).
 __device__ __forceinline__ void wait_for_loads() {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt 0; expcnt and lgkmcnt as they are
 }
@@ -140,11 +142,10 @@ __device__ __forceinline__ void copy_tile_vec(uint64_t dst, uint64_t src, uint32
       const uint32_t idx = lane + k * LANES;
       v[k] = __builtin_nontemporal_load(s + (k + 1 < K || idx < nvec ? idx : nvec - 1));
     }
-    wait_for_loads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const uint32_t idx = lane + k * LANES;
-      if (k + 1 < K || idx < nvec) store16_sc1_nt(tile, idx * 16u, v[k]);
+      // Lanes past the tile's end: dropped by the descriptor's range check.
+      store16_sc1_nt(tile, (lane + k * LANES) * 16u, v[k]);
     }
   });
   // Fewer than 16 trailing bytes (fragment size not a multiple of 16).
@@ -202,7 +203,7 @@ __device__ __forceinline__ void copy_tile_any(uint64_t dst, uint64_t src, uint32
     for (int k = 0; k < K; ++k) {
       v[k] = load16_any(src + chunk_start(lane + k * LANES, bytes, mis));
     }
-    wait_for_loads();
+    if (!ALIGN_SRC) wait_for_loads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const uint32_t i = lane + k * LANES;
@@ -346,9 +347,9 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
 // tile is full.  The block id of a lane's chunk is a vector load; it costs a
 // trip to the id list before the data loads can start, which the other
 // workgroups cover.  Measured on MI355X, 25 MB in 16 layers of K and V, save /
-// load in GB/s: fragments of 1000 bytes 47.9 / 41.4 -> 51.9 / 55.3, 1 KiB 54.8 /
-// 39.1 -> 55.7 / 55.4, 4112 bytes 52.2 / 44.4 -> 54.7 / 54.9, 100 004 bytes
-// (tile form with the chunks of copy_tile_any) 44.6 / 52.1 -> 52.3 / 54.7.
+// load in GB/s: fragments of 1000 bytes 47.9 / 41.4 -> 52.3 / 55.1, 1 KiB 54.8 /
+// 39.1 -> 56.1 / 55.8, 4112 bytes 52.2 / 44.4 -> 56.1 / 55.9, 100 004 bytes
+// (tile form with the chunks of copy_tile_any) 44.6 / 52.1 -> 52.8 / 54.8.
 template <int U, bool TO_FAR>
 __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t grid_x) {
   const uint32_t frag_bytes = static_cast<uint32_t>(f.frag_bytes);
@@ -390,17 +391,17 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
       for (int k = 0; k < K; ++k) {
         const uint64_t id =
             f.ids16 ? ((pos[k] & 1u) ? id_word[k] >> 16 : id_word[k] & 0xFFFFu) : id_word[k];
-        // chunks_per_frag is the largest count of any alignment that occurs: a
-        // fragment that has fewer moves its last one twice.
-        const uint32_t start =
-            chunk_start(chunk[k], frag_bytes, static_cast<uint32_t>(far[k]) & 15u);
+        // chunks_per_frag is the largest count of any alignment that occurs.
+        const uint32_t mis = static_cast<uint32_t>(far[k]) & 15u;
+        ok[k] = ok[k] && chunk[k] < chunk_count(frag_bytes, mis);
+        const uint32_t start = chunk_start(chunk[k], frag_bytes, mis);
         const uint64_t near_addr = near_seg + id * f.block_stride + start;
         src[k] = TO_FAR ? near_addr : far[k] + start;
         dst[k] = TO_FAR ? far[k] + start : near_addr;
       }
 #pragma unroll
       for (int k = 0; k < K; ++k) v[k] = load16_any(src[k]);
-      wait_for_loads();
+      if (TO_FAR) wait_for_loads();
       if (TO_FAR && !f.paged) {
         // The far side of a segment is one range (below 4 GiB: the host checks),
         // so aligned chunks can take the store policy that the link wants.

@@ -746,17 +746,21 @@ FillPlan plan_staged_fills(const std::vector<FillLayer>& layers, uint64_t slot_b
 // it, for fragments below 8 KiB, whose tiles leave half a workgroup and more
 // without work.  From there on both forms reach the link's rate in a long call
 // and the tile form, whose ids are scalar loads, is ahead in a short one (25 MB
-// per call, save / load in GB/s, chunks against tiles: 4112 bytes 54.7 / 54.9
-// against 51.4 / 51.5, 4 KiB 55.8 / 55.5 against 55.8 / 55.9, 8 KiB 56.0 / 56.3
-// against 56.2 / 56.7).
+// per call, save / load in GB/s, chunks against tiles: 4112 bytes 56.1 / 55.9
+// against 51.4 / 51.5, 4 KiB 56.1 / 55.7 against 55.8 / 55.9, 8176 bytes 56.2 /
+// 56.1 against 56.2 / 56.7 for tiles of 8 KiB).
 uint32_t Xfer::chunks_per_fragment(const LayerPlan& p, const BlockUnit& u) const {
   const uint64_t frag = u.frag_bytes;
   if (frag < 16 || (p.vec_ok && frag >= 8192)) return 0;
-  // The chunks of a fragment are one more where its host side does not start
-  // on a 16-byte boundary.
-  const bool starts_aligned = p.vec_ok || (p.page_dev == nullptr && aligned16(u.far_stride) &&
-                                           aligned16(u.far_base[0]) && aligned16(u.far_base[1]));
-  const uint64_t chunks = (frag + (starts_aligned ? 0 : 15) + 15) / 16;
+  // A fragment whose host side starts off a 16-byte boundary may have one chunk
+  // more: the furthest off is what the alignment of all starts leaves open (1000
+  // bytes at multiples of 8: 63 chunks either way).
+  uint64_t starts = 16;
+  if (!p.vec_ok) {
+    starts |= p.page_dev != nullptr ? 1 : u.far_stride | u.far_base[0] | u.far_base[1];
+  }
+  const uint64_t alignment = starts & (~starts + 1);
+  const uint64_t chunks = (frag + (16 - alignment) + 15) / 16;
   // 32-bit chunk indices, and one buffer descriptor for a segment's host image.
   if (chunks * u.n_blocks >= (1ull << 31)) return 0;
   if (p.page_dev == nullptr && (u.n_blocks - 1) * u.far_stride + frag > 0xFFFFFFF0ull) return 0;
