@@ -132,21 +132,85 @@ class RawBlock {
   uint64_t total_size_ = 0;
 };
 
-// block.rs:255-330: immutable once every slot is filled.
+// The host side of one slot of a block, by value: what a transfer needs of it
+// (one or two segments; a slot with none is empty).
+struct SlotView {
+  uint32_t segments = 0;
+  MappedPinnedPtr ptr[2];
+  uint64_t allocation_id[2] = {0, 0};
+  uint64_t size = 0;  // of segment 0
+  bool segment(size_t i, MappedPinnedPtr* out) const {
+    if (i >= segments) return false;
+    *out = ptr[i];
+    return true;
+  }
+  static SlotView of(const RawBlock& raw) {
+    SlotView v;
+    v.segments = raw.num_segments() < 2 ? static_cast<uint32_t>(raw.num_segments()) : 2u;
+    for (uint32_t i = 0; i < v.segments; ++i) {
+      raw.segment_mapped_ptr(i, &v.ptr[i]);
+      v.allocation_id[i] = raw.segment_allocation_id(i);
+    }
+    v.size = raw.segment_size(0);
+    return v;
+  }
+};
+
+// The host images of one save, shared by all its blocks: position q of slot s
+// lies at base[i] + q * stride of that slot's one or two buffers.  A block of
+// such a save is this image and its position.  With a segment record per slot
+// instead, a save of 1024 blocks of 61 layers wrote 62 464 of them (1.45 ms,
+// longer than its 64 MB take on the link), a later save's eviction took them
+// apart again (0.69 ms) and a load read them back one by one (1.36 ms).
+class SaveImage {
+ public:
+  struct Slot {
+    std::shared_ptr<PinnedAllocation> allocation[2];
+    MappedPinnedPtr base[2];
+    uint32_t segments = 0;
+    uint64_t stride = 0;
+  };
+  explicit SaveImage(size_t total_slots) : slots_(total_slots) {}
+  Slot& slot(size_t id) { return slots_[id]; }
+  const Slot& slot(size_t id) const { return slots_[id]; }
+  size_t num_slots() const { return slots_.size(); }
+  SlotView view(size_t id, uint32_t position) const {
+    const Slot& s = slots_[id];
+    SlotView v;
+    v.segments = s.segments;
+    for (uint32_t i = 0; i < s.segments; ++i) {
+      v.ptr[i] = s.base[i].add(position * s.stride);
+      v.allocation_id[i] = s.allocation[i]->allocation_id();
+    }
+    v.size = s.stride;
+    return v;
+  }
+
+ private:
+  std::vector<Slot> slots_;
+};
+
+// block.rs:255-330: immutable once every slot is filled.  Either a list of
+// slots or a position of a save's image.
 class SealedBlock {
  public:
-  explicit SealedBlock(std::vector<RawBlock> slots) : slots_(std::move(slots)) {
-    for (const auto& b : slots_) footprint_ += b.memory_footprint();
+  explicit SealedBlock(std::vector<RawBlock> slots) : slots_(std::move(slots)) {}
+  SealedBlock(std::shared_ptr<const SaveImage> image, uint32_t position)
+      : image_(std::move(image)), position_(position) {}
+  // False when the block has no such slot.
+  bool slot(size_t slot_id, SlotView* out) const {
+    if (slot_id >= num_slots()) return false;
+    *out = image_ ? image_->view(slot_id, position_) : SlotView::of(slots_[slot_id]);
+    return true;
   }
-  const RawBlock* get_slot(size_t slot_id) const {
-    return slot_id < slots_.size() ? &slots_[slot_id] : nullptr;
-  }
-  size_t num_slots() const { return slots_.size(); }
-  uint64_t memory_footprint() const { return footprint_; }
+  size_t num_slots() const { return image_ ? image_->num_slots() : slots_.size(); }
+  const SaveImage* image() const { return image_.get(); }  // null: a list of slots
+  uint32_t position() const { return position_; }
 
  private:
   std::vector<RawBlock> slots_;
-  uint64_t footprint_ = 0;
+  std::shared_ptr<const SaveImage> image_;
+  uint32_t position_ = 0;
 };
 
 // block.rs:346-454: slots arrive one by one; seals when none remain.

@@ -55,7 +55,6 @@ struct SaveLayerCtx {
   uint64_t stride = 0;                         // host stride of one position
   // Batch image: one K (and V) allocation; blockwise: one per kept position.
   std::vector<std::shared_ptr<PinnedAllocation>> k_allocs, v_allocs;
-  std::vector<RawBlock> raw_blocks;            // blockwise only: handles the task points at
 
   // The host image of kept position q as a block of its own (offload.rs:454-509).
   bool make_raw(size_t q, bool blockwise, RawBlock* out) const {
@@ -73,6 +72,35 @@ struct SaveLayerCtx {
     return true;
   }
 };
+
+namespace {
+// The image of a save of `num` blocks whose layers are `members`, or null when
+// they do not fill every slot of a block (the rest comes with another save).
+std::shared_ptr<SaveImage> save_image(const std::vector<SaveLayerCtx*>& members, size_t total_slots,
+                                      size_t num) {
+  auto image = std::make_shared<SaveImage>(total_slots);
+  size_t filled = 0;
+  for (const SaveLayerCtx* ctx : members) {
+    if (ctx->slot_id >= total_slots) continue;
+    SaveImage::Slot& slot = image->slot(ctx->slot_id);
+    if (slot.segments != 0) continue;  // a slot named twice keeps its first block
+    const std::shared_ptr<PinnedAllocation>* buffers[2] = {
+        &ctx->k_allocs[0], ctx->v_allocs.empty() ? nullptr : &ctx->v_allocs[0]};
+    uint64_t bytes = 0;
+    if (__builtin_mul_overflow(ctx->stride, static_cast<uint64_t>(num), &bytes)) return nullptr;
+    for (const auto* buffer : buffers) {
+      if (buffer == nullptr) continue;
+      if (!(*buffer)->mapped_ptr_for_host_range((*buffer)->as_ptr(), bytes, &slot.base[slot.segments])) {
+        return nullptr;
+      }
+      slot.allocation[slot.segments++] = *buffer;
+    }
+    slot.stride = ctx->stride;
+    ++filled;
+  }
+  return filled == total_slots ? image : nullptr;
+}
+}  // namespace
 
 // ---------------------------------------------------------------------------
 // InstanceContext
@@ -469,7 +497,8 @@ int Engine::alloc_page_first_targets(const LayerTopology& topo, SaveLayerCtx* ct
                  "page-first save spans multiple shards (one writer must save one shard)");
     }
     // Same hashes (same list) and same block ids, position by position.
-    if (ctxs[i].list != first.list || *ctxs[i].ids != *first.ids) {
+    if (ctxs[i].list != first.list ||
+        (ctxs[i].ids != first.ids && *ctxs[i].ids != *first.ids)) {
       return bad(err, PF_ERR_INVALID_ARGUMENT,
                  "page-first save requires the same block set across all layers");
     }
@@ -639,12 +668,18 @@ int Engine::batch_save_kv_blocks(const std::string& instance_id, size_t tp_rank,
                             [&](const SaveLayerCtx& c) { return lists[c.list].kept.empty(); }),
              ctxs.end());
   if (ctxs.empty()) return PF_OK;
+  const SaveLayerCtx* before = nullptr;
   for (SaveLayerCtx& ctx : ctxs) {
     const SaveList& l = lists[ctx.list];
-    auto ids = std::make_shared<std::vector<uint32_t>>();
-    ids->reserve(l.kept.size());
-    for (uint32_t pos : l.kept) ids->push_back(static_cast<uint32_t>(ctx.block_ids[pos]));
-    ctx.ids = std::move(ids);
+    if (before != nullptr && before->block_ids == ctx.block_ids && before->list == ctx.list) {
+      ctx.ids = before->ids;  // the caller passed one array for all layers
+    } else {
+      auto ids = std::make_shared<std::vector<uint32_t>>();
+      ids->reserve(l.kept.size());
+      for (uint32_t pos : l.kept) ids->push_back(static_cast<uint32_t>(ctx.block_ids[pos]));
+      ctx.ids = std::move(ids);
+    }
+    before = &ctx;
   }
   prof.filter_ms = ms_since(t_phase);
 
@@ -706,19 +741,15 @@ int Engine::batch_save_kv_blocks(const std::string& instance_id, size_t tp_rank,
         if (split) ltd.image.seg_allocation_id[1] = ctx.v_allocs[0]->allocation_id();
       } else {
         // One allocation per block and segment: per-block handles.
-        ctx.raw_blocks.reserve(num);
+        ltd.blocks.reserve(num);
         for (size_t q = 0; q < num; ++q) {
           RawBlock raw;
           if (!ctx.make_raw(q, cfg_.blockwise_alloc, &raw)) {
             return bad(err, PF_ERR_STORAGE, "segment exceeds its pinned allocation");
           }
-          ctx.raw_blocks.push_back(std::move(raw));
-        }
-        ltd.blocks.reserve(num);
-        for (size_t q = 0; q < num; ++q) {
           TransferBlock tb;
           tb.block_idx = (*ctx.ids)[q];
-          tb.block.raw = &ctx.raw_blocks[q];
+          tb.block.slot = SlotView::of(raw);
           ltd.blocks.push_back(std::move(tb));
         }
       }
@@ -735,9 +766,27 @@ int Engine::batch_save_kv_blocks(const std::string& instance_id, size_t tp_rank,
 
   struct Assembled {
     BlockKey* key;  // in its SaveList; moved into the store when the block is published
-    InflightBlock block;
+    // A block whose slots this save carries all of, or the slots it carries.
+    std::shared_ptr<SealedBlock> sealed;
+    InflightBlock partial;
+    const std::vector<SaveLayerCtx*>* members;
+    uint32_t position;
   };
   std::vector<Assembled> assembled;
+  std::vector<std::vector<SaveLayerCtx*>> members_of(lists.size());
+  const bool blockwise = cfg_.blockwise_alloc;
+  // The slots of one block as records of their own (a slot named twice keeps
+  // its first block).
+  auto fill_slots = [blockwise](const std::vector<SaveLayerCtx*>& members, size_t q,
+                                InflightBlock* block) {
+    for (SaveLayerCtx* ctx : members) {
+      RawBlock* slot = block->empty_slot(ctx->slot_id);
+      if (slot == nullptr) continue;
+      if (!ctx->make_raw(q, blockwise, slot)) return false;
+      block->slot_filled();
+    }
+    return true;
+  };
   int prep_status = PF_OK;
   std::string prep_err;
   if (!page_first) {
@@ -752,24 +801,27 @@ int Engine::batch_save_kv_blocks(const std::string& instance_id, size_t tp_rank,
         prep_err = cause;
         break;
       }
-      std::vector<SaveLayerCtx*> members;
+      std::vector<SaveLayerCtx*>& members = members_of[li];
       for (auto& ctx : ctxs) {
         if (ctx.list == li) members.push_back(&ctx);
       }
       const auto created = Clock::now();
-      for (size_t q = 0; q < l.kept.size() && prep_status == PF_OK; ++q) {
-        assembled.push_back(Assembled{&l.keys[l.kept[q]], InflightBlock(total_slots, created)});
-        InflightBlock& block = assembled.back().block;
-        for (SaveLayerCtx* ctx : members) {
-          // Built in place; a slot named twice keeps its first block.
-          RawBlock* slot = block.empty_slot(ctx->slot_id);
-          if (slot == nullptr) continue;
-          if (!ctx->make_raw(q, cfg_.blockwise_alloc, slot)) {
-            prep_status = PF_ERR_STORAGE;
-            prep_err = "segment exceeds its pinned allocation";
-            break;
-          }
-          block.slot_filled();
+      std::shared_ptr<SaveImage> image;
+      if (!blockwise) image = save_image(members, total_slots, l.kept.size());
+      for (size_t q = 0; q < l.kept.size(); ++q) {
+        BlockKey* key = &l.keys[l.kept[q]];
+        const uint32_t position = static_cast<uint32_t>(q);
+        if (image) {
+          assembled.push_back(Assembled{key, std::make_shared<SealedBlock>(image, position),
+                                        InflightBlock(0, created), &members, position});
+          continue;
+        }
+        assembled.push_back(
+            Assembled{key, nullptr, InflightBlock(total_slots, created), &members, position});
+        if (!fill_slots(members, q, &assembled.back().partial)) {
+          prep_status = PF_ERR_STORAGE;
+          prep_err = "segment exceeds its pinned allocation";
+          break;
         }
       }
     }
@@ -817,20 +869,30 @@ int Engine::batch_save_kv_blocks(const std::string& instance_id, size_t tp_rank,
         // blocks: one table operation per block.
         auto it = inflight_.empty() ? inflight_.end() : inflight_.find(key);
         if (it == inflight_.end()) {
-          if (a.block.complete()) {
-            seal_insert(std::move(key), a.block.seal());  // no-op when sealed meanwhile
+          if (a.sealed) {
+            seal_insert(std::move(key), std::move(a.sealed));  // no-op when sealed meanwhile
+          } else if (a.partial.complete()) {
+            seal_insert(std::move(key), a.partial.seal());
           } else if (sealed_.find(key) == sealed_.end()) {
-            inflight_.emplace(std::move(key), std::move(a.block));
+            inflight_.emplace(std::move(key), std::move(a.partial));
           }
-        } else if (sealed_.find(key) != sealed_.end()) {
           continue;
-        } else if (it->second.total_slots() != a.block.total_slots()) {
+        }
+        if (sealed_.find(key) != sealed_.end()) continue;
+        const size_t slots = a.sealed ? a.sealed->num_slots() : a.partial.total_slots();
+        if (it->second.total_slots() != slots) {
           // The block in flight was begun by an instance with another slot
           // count (a namespace shared by incompatible layouts): this save's
           // part is dropped, the other one can still complete
           // (write_path.rs:147-165).
           continue;
-        } else if (it->second.absorb(std::move(a.block)) == InflightBlock::Insert::Completed) {
+        }
+        if (a.sealed) {
+          // Someone began this block slot by slot: give it this save's slots.
+          a.partial = InflightBlock(slots);
+          if (!fill_slots(*a.members, a.position, &a.partial)) continue;
+        }
+        if (it->second.absorb(std::move(a.partial)) == InflightBlock::Insert::Completed) {
           auto sealed_block = it->second.seal();
           inflight_.erase(it);
           seal_insert(std::move(key), std::move(sealed_block));
@@ -1010,6 +1072,82 @@ bool Engine::release_query_lease(uint64_t lease) {
   return leases_.erase(lease) > 0;
 }
 
+namespace {
+// Positions first, first + 1, ... of a save.
+struct SaveRun {
+  const SaveImage* save;
+  uint32_t first;
+  size_t count;
+};
+
+// The blocks of one load group as runs of positions of saves, when they are all
+// positions of saves and the runs are long enough to be worth it; otherwise
+// `runs` is empty and the group is loaded by per-block handles.
+struct GroupRuns {
+  std::vector<SaveRun> runs;
+  std::shared_ptr<const std::vector<uint32_t>> ids;
+  uint64_t max_id = 0;
+
+  GroupRuns(const std::vector<std::pair<uint64_t, size_t>>& targets,
+            const std::vector<std::shared_ptr<SealedBlock>>& blocks) {
+    auto list = std::make_shared<std::vector<uint32_t>>();
+    list->reserve(targets.size());
+    for (const auto& t : targets) {
+      const SealedBlock& block = *blocks[t.second];
+      if (block.image() == nullptr) {
+        runs.clear();
+        return;
+      }
+      if (!runs.empty() && runs.back().save == block.image() &&
+          runs.back().first + runs.back().count == block.position()) {
+        ++runs.back().count;
+      } else {
+        runs.push_back({block.image(), block.position(), 1});
+      }
+      max_id = std::max(max_id, t.first);
+      list->push_back(static_cast<uint32_t>(t.first));
+    }
+    if (runs.size() > 1 && runs.size() * 2 > targets.size()) runs.clear();
+    ids = std::move(list);
+  }
+
+  // The host side of a layer of the group.  False when per-block handles have
+  // to say what is wrong with it (an id out of range, a slot that is not there)
+  // or when blocks were saved smaller than the layer's.
+  bool layer(size_t slot_id, uint64_t host_offset, LayerTransferData* out) const {
+    if (runs.empty() || max_id >= out->layout.num_blocks()) return false;
+    const uint64_t frag = out->layout.fragment_bytes();
+    for (const SaveRun& run : runs) {
+      if (slot_id >= run.save->num_slots()) return false;
+      const SaveImage::Slot& slot = run.save->slot(slot_id);
+      if (slot.segments == 0 || slot.stride < frag) return false;
+    }
+    HostImage& image = out->image;
+    image.block_ids = ids;
+    if (runs.size() == 1) {
+      const SlotView at = runs[0].save->view(slot_id, runs[0].first);
+      image.kind = HostImage::Kind::Uniform;
+      image.stride = ids->size() > 1 ? at.size : frag;
+      for (uint32_t s = 0; s < at.segments; ++s) {
+        image.seg[s] = at.ptr[s].add(host_offset);
+        image.seg_allocation_id[s] = at.allocation_id[s];
+      }
+      return true;
+    }
+    image.kind = HostImage::Kind::Runs;
+    image.runs.resize(runs.size());
+    for (size_t r = 0; r < runs.size(); ++r) {
+      const SlotView at = runs[r].save->view(slot_id, runs[r].first);
+      HostImage::Run& run = image.runs[r];
+      for (uint32_t s = 0; s < at.segments; ++s) run.seg[s] = at.ptr[s].add(host_offset);
+      run.stride = at.size;
+      run.count = runs[r].count;
+    }
+    return true;
+  }
+};
+}  // namespace
+
 int Engine::batch_load_kv_blocks_multi_layer(
     const std::string& instance_id, size_t tp_rank, int device_id,
     const std::vector<std::vector<std::string>>& layer_groups,
@@ -1126,6 +1264,11 @@ int Engine::batch_load_kv_blocks_multi_layer(
   std::map<std::pair<size_t, size_t>, PageList> page_lists;
   const bool page_first = topo->is_page_first();
   std::vector<LayerTransferData> layers;
+  std::vector<GroupRuns> group_runs;
+  if (!page_first && !cfg_.use_descriptor_backends) {
+    group_runs.reserve(layer_groups.size());
+    for (const auto& t : targets) group_runs.emplace_back(t, block_cache);
+  }
   for (size_t gi = 0; gi < layer_groups.size(); ++gi) {
     for (const std::string& name : layer_groups[gi]) {
       size_t layer_id = 0;
@@ -1155,17 +1298,17 @@ int Engine::batch_load_kv_blocks_multi_layer(
           auto ids = std::make_shared<std::vector<uint32_t>>();
           uint64_t page_len = UINT64_MAX;
           for (auto& t : targets[gi]) {
-            const RawBlock* raw = block_cache[t.second]->get_slot(slot_id);
+            SlotView slot;
             MappedPinnedPtr p;
-            if (!raw || !raw->segment_mapped_ptr(0, &p)) {
+            if (!block_cache[t.second]->slot(slot_id, &slot) || !slot.segment(0, &p)) {
               return bad(err, PF_ERR_INVALID_ARGUMENT,
                          "stored block is missing slot " + std::to_string(slot_id) +
                              " for layer " + name);
             }
             pages->push_back(p);
-            alloc_ids->push_back(raw->segment_allocation_id(0));
+            alloc_ids->push_back(slot.allocation_id[0]);
             ids->push_back(static_cast<uint32_t>(t.first));
-            page_len = std::min(page_len, raw->segment_size(0));
+            page_len = std::min(page_len, slot.size);
           }
           pl.pages = std::move(pages);
           pl.alloc_ids = std::move(alloc_ids);
@@ -1181,18 +1324,22 @@ int Engine::batch_load_kv_blocks_multi_layer(
         layers.push_back(std::move(ltd));
         continue;
       }
+      if (!group_runs.empty() && group_runs[gi].layer(slot_id, host_offset, &ltd)) {
+        layers.push_back(std::move(ltd));
+        continue;
+      }
       ltd.blocks.reserve(targets[gi].size());
       for (auto& t : targets[gi]) {
         const auto& sealed = block_cache[t.second];
-        const RawBlock* raw = sealed->get_slot(slot_id);
-        if (!raw) {
+        SlotView slot;
+        if (!sealed->slot(slot_id, &slot)) {
           return bad(err, PF_ERR_INVALID_ARGUMENT,
                      "stored block is missing slot " + std::to_string(slot_id) + " for layer " +
                          name);
         }
         TransferBlock tb;
         tb.block_idx = t.first;
-        tb.block.raw = raw;
+        tb.block.slot = slot;
         tb.block.offset = host_offset;
         ltd.blocks.push_back(std::move(tb));
       }

@@ -86,8 +86,7 @@ bool BorrowedBlocks::build(const pf_layer_transfer* layers, uint64_t n_layers,
       keep->push_back(raw);
       pf::TransferBlock tb;
       tb.block_idx = in.block_idx[bi];
-      tb.block.raw = raw.get();
-      tb.block.keep = raw;
+      tb.block.slot = pf::SlotView::of(*raw);
       tb.block.offset = hb.host_offset;
       ltd.blocks.push_back(std::move(tb));
     }

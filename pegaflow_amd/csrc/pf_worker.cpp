@@ -38,6 +38,10 @@ bool build_copy_descs(const std::vector<LayerTransferData>& layers, std::vector<
       const HostImage& im = layer.image;
       const size_t n = im.size();
       const bool paged = im.kind == HostImage::Kind::Paged;
+      if (im.kind == HostImage::Kind::Runs) {
+        *err = "layer " + layer.layer_name + ": a host image in runs needs the block-ID engine";
+        return false;
+      }
       if (paged && (!im.pages || im.pages->size() != n || !im.page_allocation_ids ||
                     im.page_allocation_ids->size() != n)) {
         *err = "layer " + layer.layer_name + ": host image has a page list of the wrong length";
@@ -85,9 +89,9 @@ bool build_copy_descs(const std::vector<LayerTransferData>& layers, std::vector<
         *err = "layer " + layer.layer_name + ": " + cause;
         return false;
       }
-      const RawBlock* raw = tb.block.raw;
+      const SlotView& slot = tb.block.slot;
       MappedPinnedPtr k;
-      if (!raw || !raw->segment_mapped_ptr(0, &k)) {
+      if (!slot.segment(0, &k)) {
         *err = "layer " + layer.layer_name + ": host block has no segment 0";
         return false;
       }
@@ -95,21 +99,21 @@ bool build_copy_descs(const std::vector<LayerTransferData>& layers, std::vector<
       if (bc.n == 2) {
         MappedPinnedPtr v;
         uint64_t v_alloc;
-        if (raw->segment_mapped_ptr(1, &v)) {
+        if (slot.segment(1, &v)) {
           v = v.add(tb.block.offset);
-          v_alloc = raw->segment_allocation_id(1);
+          v_alloc = slot.allocation_id[1];
         } else {
           v = k.add(bc.k.bytes);  // single-segment host block: V follows K
-          v_alloc = raw->segment_allocation_id(0);
+          v_alloc = slot.allocation_id[0];
         }
         out->push_back({bc.k.addr, k.host, reinterpret_cast<uint64_t>(k.device), bc.k.bytes, li,
-                        raw->segment_allocation_id(0)});
+                        slot.allocation_id[0]});
         out->push_back({bc.v.addr, v.host, reinterpret_cast<uint64_t>(v.device), bc.v.bytes, li,
                         v_alloc});
         total += bc.k.bytes + bc.v.bytes;
       } else {
         out->push_back({bc.k.addr, k.host, reinterpret_cast<uint64_t>(k.device), bc.k.bytes, li,
-                        raw->segment_allocation_id(0)});
+                        slot.allocation_id[0]});
         total += bc.k.bytes;
       }
     }
@@ -223,7 +227,8 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
     lb.layout = layer.layout.c();
     const bool split = layer.layout.is_split();
     const uint64_t frag = layer.layout.fragment_bytes();
-    if (layer.image.kind != HostImage::Kind::None) {
+    const bool in_runs = layer.image.kind == HostImage::Kind::Runs;
+    if (layer.image.kind != HostImage::Kind::None && !in_runs) {
       const HostImage& im = layer.image;
       const size_t n_im = im.size();
       lb.n_blocks = n_im;
@@ -265,35 +270,49 @@ bool to_block_form(const std::vector<LayerTransferData>& all_layers, size_t begi
       out->layer_table[li] = static_cast<int>(ti);
       continue;
     }
-    const size_t n = layer.blocks.size();
+    const size_t n = in_runs ? layer.image.size() : layer.blocks.size();
     lb.n_blocks = n;
     if (n == 0) continue;
-    std::vector<uint32_t>& ids = out->ids[li];
-    ids.resize(n);
-    std::vector<MappedPinnedPtr> k(n), v(n);
-    for (size_t i = 0; i < n; ++i) {
-      const TransferBlock& tb = layer.blocks[i];
-      if (tb.block_idx >= layer.layout.num_blocks()) {
-        *err = "layer " + layer.layer_name + ": block " + std::to_string(tb.block_idx) +
-               " out of range (" + std::to_string(layer.layout.num_blocks()) + " blocks)";
-        return false;
-      }
-      ids[i] = static_cast<uint32_t>(tb.block_idx);
-      const RawBlock* raw = tb.block.raw;
-      if (!raw || !raw->segment_mapped_ptr(0, &k[i])) {
-        *err = "layer " + layer.layer_name + ": host block has no segment 0";
-        return false;
-      }
-      k[i] = k[i].add(tb.block.offset);
-      if (split) {
-        if (raw->segment_mapped_ptr(1, &v[i])) {
-          v[i] = v[i].add(tb.block.offset);
-        } else {
-          v[i] = k[i].add(frag);
+    std::vector<MappedPinnedPtr> k, v;
+    k.reserve(n);
+    v.reserve(split ? n : 0);
+    if (in_runs) {
+      // Block ids are range-checked by the transfer engine's own planning.
+      for (const HostImage::Run& run : layer.image.runs) {
+        for (size_t j = 0; j < run.count; ++j) {
+          k.push_back(run.seg[0].add(j * run.stride));
+          if (split) {
+            v.push_back(run.seg[1].host ? run.seg[1].add(j * run.stride) : k.back().add(frag));
+          }
         }
       }
+      if (k.size() != n) {
+        *err = "layer " + layer.layer_name + ": host image has runs of the wrong length";
+        return false;
+      }
+      lb.block_ids = layer.image.block_ids->data();
+    } else {
+      std::vector<uint32_t>& ids = out->ids[li];
+      ids.resize(n);
+      for (size_t i = 0; i < n; ++i) {
+        const TransferBlock& tb = layer.blocks[i];
+        if (tb.block_idx >= layer.layout.num_blocks()) {
+          *err = "layer " + layer.layer_name + ": block " + std::to_string(tb.block_idx) +
+                 " out of range (" + std::to_string(layer.layout.num_blocks()) + " blocks)";
+          return false;
+        }
+        ids[i] = static_cast<uint32_t>(tb.block_idx);
+        const SlotView& slot = tb.block.slot;
+        MappedPinnedPtr seg;
+        if (!slot.segment(0, &seg)) {
+          *err = "layer " + layer.layer_name + ": host block has no segment 0";
+          return false;
+        }
+        k.push_back(seg.add(tb.block.offset));
+        if (split) v.push_back(slot.segment(1, &seg) ? seg.add(tb.block.offset) : k[i].add(frag));
+      }
+      lb.block_ids = ids.data();
     }
-    lb.block_ids = ids.data();
     out->total_bytes += frag * (split ? 2 : 1) * n;
 
     // Uniform stride?

@@ -25,12 +25,11 @@
 
 namespace pf {
 
-// gpu_worker.rs:61-94: the host image of one block in a transfer.  `raw`
-// points at a block owned by the task (save) or at a slot of a cached sealed
-// block kept alive by `keep` (load); `offset` is the page-first byte offset.
+// gpu_worker.rs:61-94: the host image of one block in a transfer; `offset` is
+// the page-first byte offset.  Whoever submits the task keeps the memory alive
+// (LayerTransferData::keep).
 struct HostBlock {
-  const RawBlock* raw = nullptr;
-  std::shared_ptr<const void> keep;
+  SlotView slot;
   uint64_t offset = 0;
 };
 
@@ -46,9 +45,16 @@ struct TransferBlock {
 //   Uniform: list position i at seg[s] + i * stride (the batch image of a
 //            save: one K buffer and one V buffer, or one block buffer);
 //   Paged:   list position i at pages[i] + offset, V right behind K (one page
-//            or one allocation per block).
+//            or one allocation per block);
+//   Runs:    uniform images one after the other, `runs[r].count` positions each
+//            (a prefix that several saves have stored).  Block-ID engine only.
 struct HostImage {
-  enum class Kind { None, Uniform, Paged };
+  enum class Kind { None, Uniform, Paged, Runs };
+  struct Run {
+    MappedPinnedPtr seg[2];  // seg[1].host null: V right behind K
+    uint64_t stride = 0;
+    size_t count = 0;
+  };
   Kind kind = Kind::None;
   std::shared_ptr<const std::vector<uint32_t>> block_ids;  // device block of each position
   MappedPinnedPtr seg[2];
@@ -58,6 +64,7 @@ struct HostImage {
   std::shared_ptr<const std::vector<uint64_t>> page_allocation_ids;
   uint64_t offset = 0;
   uint64_t page_len = 0;
+  std::vector<Run> runs;
   std::vector<std::shared_ptr<const void>> keep;  // what owns the memory
   size_t size() const { return block_ids ? block_ids->size() : 0; }
 };

@@ -228,9 +228,24 @@ def _pack_hashes(hashes: Sequence[bytes]):
     return ptrs, lens, (blob, addrs, lens_keep)
 
 
+def _pack_destinations(ids: Sequence[int | None]):
+    """-> (int64 array for C, what owns it) of one destination list, None as -1."""
+    n = len(ids)
+    try:
+        packed = np.asarray(ids)
+    except ValueError:  # nested lists: int() says what is wrong with them
+        packed = np.empty(0)
+    if n and packed.ndim == 1 and packed.dtype.kind in "iu":
+        packed = np.ascontiguousarray(packed.astype(np.int64, copy=False))
+        return C.cast(packed.ctypes.data, C.POINTER(C.c_int64)), packed
+    d = (C.c_int64 * max(n, 1))(*[-1 if v is None else int(v) for v in ids])
+    return C.cast(d, C.POINTER(C.c_int64)), d
+
+
 class PackedSaves:
     """The C form of a list of LayerSave, reusable across calls.  Layers that
-    pass the very same hash list object share one packed copy."""
+    pass the very same hash list or id list object share one packed copy (the
+    objects are kept, so an identity cannot come back as another list)."""
 
     def __init__(self, saves: Sequence[LayerSave]):
         n = len(saves)
@@ -238,28 +253,34 @@ class PackedSaves:
         self.array = (_lib.PfLayerSave * max(n, 1))()
         self._keep = []
         packed_hashes = {}
+        packed_ids = {}
         for i, s in enumerate(saves):
-            if len(s.block_hashes) != len(s.block_ids):
+            block_ids, block_hashes = s.block_ids, s.block_hashes
+            if len(block_hashes) != len(block_ids):
                 # offload.rs:328-335
                 raise _lib.InvalidArgument(
                     _lib.PF_ERR_INVALID_ARGUMENT,
-                    f"block_ids length {len(s.block_ids)} does not match block_hashes "
-                    f"{len(s.block_hashes)} for layer {s.layer_name}")
-            ids = np.ascontiguousarray(s.block_ids, dtype=np.uint64)
-            if ids.size == 0:
-                ids = np.zeros(1, dtype=np.uint64)
+                    f"block_ids length {len(block_ids)} does not match block_hashes "
+                    f"{len(block_hashes)} for layer {s.layer_name}")
+            packed = packed_ids.get(id(block_ids))
+            if packed is None:
+                ids = np.ascontiguousarray(block_ids, dtype=np.uint64)
+                if ids.size == 0:
+                    ids = np.zeros(1, dtype=np.uint64)
+                packed = (ids, C.cast(ids.ctypes.data, C.POINTER(C.c_uint64)))
+                packed_ids[id(block_ids)] = packed
             name = s.layer_name.encode()
-            key = id(s.block_hashes)
+            key = id(block_hashes)
             if key not in packed_hashes:
-                packed_hashes[key] = _pack_hashes(s.block_hashes)
+                packed_hashes[key] = _pack_hashes(block_hashes)
             ptrs, lens, _ = packed_hashes[key]
             a = self.array[i]
             a.layer_name = name
-            a.block_ids = C.cast(ids.ctypes.data, C.POINTER(C.c_uint64))
-            a.n_blocks = len(s.block_ids)
+            a.block_ids = packed[1]
+            a.n_blocks = len(block_ids)
             a.block_hashes = ptrs
             a.block_hash_lens = lens
-            self._keep.append((ids, name, s.block_hashes))
+            self._keep.append((packed, name, block_ids, block_hashes))
         self._keep.append(packed_hashes)
 
 
@@ -369,9 +390,8 @@ class PegaEngine:
             if len(ids) != n_blocks:
                 raise _lib.InvalidArgument(_lib.PF_ERR_INVALID_ARGUMENT,
                                            "every load group needs one destination per leased block")
-            d = (C.c_int64 * max(n_blocks, 1))(*[-1 if v is None else int(v) for v in ids])
-            keep.append(d)
-            dests[i] = d
+            dests[i], owner = _pack_destinations(ids)
+            keep.append(owner)
         t = C.c_void_p()
         shm = load_state.shm_name.encode() if load_state is not None else None
         check(self._lib.pf_engine_batch_load(self.handle, instance_id.encode(), tp_rank, device_id,
@@ -438,9 +458,8 @@ class PegaEngine:
                     raise _lib.InvalidArgument(
                         _lib.PF_ERR_INVALID_ARGUMENT,
                         "every load group needs one destination per leased block")
-                d = (C.c_int64 * max(n_blocks, 1))(*[-1 if v is None else int(v) for v in ids])
-                keep.append(d)
-                ptrs[gi] = d
+                ptrs[gi], owner = _pack_destinations(ids)
+                keep.append(owner)
             keep.append(ptrs)
             reqs[li].lease = lease
             reqs[li].dest_block_ids = ptrs

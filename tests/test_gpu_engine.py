@@ -1111,3 +1111,57 @@ def test_load_of_blocks_from_several_saves(gpu, seg, turns, n_layers, paths):
     e.close()
     for d in devs:
         d.close()
+
+
+@pytest.mark.parametrize("order", ["prefix", "middle", "one", "reversed", "every_other", "two_saves",
+                                   "no_destination", "begun_by_another_save"])
+def test_loads_of_positions_of_saves(engine, order):
+    """Blocks of one save share its image: consecutive positions of it load as a
+    uniform image, anything else block by block, and a block that another save
+    has begun layer by layer keeps the slots it has."""
+    rng = np.random.default_rng(len(order))
+    num_blocks, n = 64, 12
+    shapes = [("kv0", 1000, 2), ("kv1", 4096, 2), ("latent", 1536, 1)]
+    caches = {name: random_bytes(rng, segs * num_blocks * seg) for name, seg, segs in shapes}
+    bufs = {name: DeviceBuffer(caches[name].nbytes) for name, _, _ in shapes}
+    for name, buf in bufs.items():
+        buf.copy_from_host(caches[name])
+    names = [name for name, _, _ in shapes]
+    engine.register_context_layer_batch(
+        "pos", "ns", 0, 0, 0, 1, 1, names, [bufs[k].ptr for k in names],
+        [caches[k].nbytes for k in names], [num_blocks] * 3, [seg for _, seg, _ in shapes],
+        [num_blocks * seg if segs == 2 else 0 for _, seg, segs in shapes], [s for _, _, s in shapes])
+    ids = rng.permutation(num_blocks)[:2 * n]
+    hashes = make_block_hashes(2 * n, 9)
+    begun = hashes[3] if order == "begun_by_another_save" else None
+    if begun is not None:  # block 3 has slot kv1 from other device blocks already
+        engine.batch_save_kv_blocks("pos", 0, 0, 0, [LayerSave("kv1", [int(ids[n])], [begun])])
+    for part in (slice(0, n), slice(n, 2 * n)):
+        engine.batch_save_kv_blocks("pos", 0, 0, 0, [
+            LayerSave(k, ids[part].tolist(), hashes[part]) for k in names])
+    want = {"prefix": list(range(5)), "middle": list(range(4, 9)), "one": [7],
+            "reversed": list(range(n))[::-1], "every_other": list(range(0, n, 2)),
+            "two_saves": list(range(n - 2, n + 2)), "no_destination": list(range(n)),
+            "begun_by_another_save": list(range(n))}[order]
+    dest = [int(d) for d in rng.permutation(num_blocks)[:len(want)]]
+    if order == "no_destination":
+        dest[2] = dest[-1] = None
+    for name, buf in bufs.items():
+        buf.fill(0)
+    hits, lease = engine.query_prefix("pos", [hashes[i] for i in want])
+    assert hits == len(want)
+    engine.batch_load_kv_blocks_multi_layer("pos", 0, 0, [names], lease, [dest]).wait()
+    for name, seg, segs in shapes:
+        src = caches[name].reshape(segs, num_blocks, seg)
+        expect = np.zeros_like(src)
+        for i, d in zip(want, dest):
+            if d is not None:
+                taken = ids[n] if name == "kv1" and hashes[i] == begun else ids[i]
+                expect[:, d] = src[:, taken]
+        assert np.array_equal(bufs[name].copy_to_host().reshape(expect.shape), expect), name
+    hits, lease = engine.query_prefix("pos", [hashes[i] for i in want])
+    with pytest.raises(_lib.StorageError, match="block 64 out of range"):
+        engine.batch_load_kv_blocks_multi_layer("pos", 0, 0, [names], lease,
+                                                [[64] + [None] * (len(want) - 1)]).wait()
+    for buf in bufs.values():
+        buf.close()
