@@ -163,6 +163,39 @@ int Xfer::ensure_side_stream(hipStream_t s) {
   return PF_OK;
 }
 
+// A fill's use of its slot: `writer` fills it, `reader` empties it.  On one
+// stream the order of the commands says all of that: a slot waits for an earlier
+// call only at its first fill, and is marked free once, behind the call's last
+// command.  (A marker between a copy and a kernel is a barrier of its own on the
+// queue.)
+int Xfer::slot_begin(Slot& sl, hipStream_t writer) {
+  if (sl.used && !sl.in_order) PF_HIP(hipStreamWaitEvent(writer, sl.freed, 0));
+  return PF_OK;
+}
+
+int Xfer::slot_ready(Slot& sl, hipStream_t writer, hipStream_t reader) {
+  if (writer == reader) return PF_OK;
+  PF_HIP(hipEventRecord(sl.ready, writer));
+  PF_HIP(hipStreamWaitEvent(reader, sl.ready, 0));
+  return PF_OK;
+}
+
+int Xfer::slot_end(Slot& sl, hipStream_t reader, bool in_order) {
+  sl.used = true;
+  sl.in_order = in_order;
+  if (!in_order) PF_HIP(hipEventRecord(sl.freed, reader));
+  return PF_OK;
+}
+
+int Xfer::slots_in_order_end(hipStream_t s) {
+  for (Slot& sl : slots_) {
+    if (!sl.in_order) continue;
+    sl.in_order = false;
+    PF_HIP(hipEventRecord(sl.freed, s));
+  }
+  return PF_OK;
+}
+
 int Xfer::timing_begin(hipStream_t s) {
   if (!timing_) return PF_OK;
   if (timing_used_ == timing_pool_.size()) {
@@ -610,25 +643,28 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
       return timing_end(s);
     };
     if (save) {
-      if (sl.used) PF_HIP(hipStreamWaitEvent(s, sl.freed, 0));
+      st = slot_begin(sl, s);
+      if (st != PF_OK) return st;
       st = launch(true);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.ready, s));
-      PF_HIP(hipStreamWaitEvent(side, sl.ready, 0));
+      st = slot_ready(sl, s, side);
+      if (st != PF_OK) return st;
       PF_HIP(hipMemcpyAsync(host_ptr, sl.buf, bytes, hipMemcpyDeviceToHost, side));
-      PF_HIP(hipEventRecord(sl.freed, side));
+      st = slot_end(sl, side, side == s);
+      if (st != PF_OK) return st;
       prof_mark_first(side);
     } else {
-      if (sl.used) PF_HIP(hipStreamWaitEvent(side, sl.freed, 0));
+      st = slot_begin(sl, side);
+      if (st != PF_OK) return st;
       PF_HIP(hipMemcpyAsync(sl.buf, host_ptr, bytes, hipMemcpyHostToDevice, side));
-      PF_HIP(hipEventRecord(sl.ready, side));
       prof_mark_first(side);
-      PF_HIP(hipStreamWaitEvent(s, sl.ready, 0));
+      st = slot_ready(sl, side, s);
+      if (st != PF_OK) return st;
       st = launch(false);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.freed, s));
+      st = slot_end(sl, s, side == s);
+      if (st != PF_OK) return st;
     }
-    sl.used = true;
     ++prof_.staged_groups;
     ++prof_.link_copies;
   }
@@ -636,6 +672,8 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     PF_HIP(hipEventRecord(join_, side));
     PF_HIP(hipStreamWaitEvent(s, join_, 0));
   }
+  st = slots_in_order_end(s);
+  if (st != PF_OK) return st;
   // Every layer of a page lands together: all per-layer events fire at the end.
   if (!layer_events_.empty()) {
     for (uint64_t li = 0; li < n_layers; ++li) PF_HIP(hipEventRecord(layer_events_[li], s));
@@ -674,6 +712,7 @@ int Xfer::run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool s
     if (side_ != nullptr) (void)hipStreamSynchronize(side_);
     (void)hipStreamSynchronize(s);
     (void)hipGetLastError();
+    for (Slot& sl : slots_) sl.in_order = false;  // nothing is using it any more
     last_error() = message;
   }
   return st;
@@ -1294,33 +1333,35 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         ue == unit_refs.size() || unit_refs[ue].plan != unit_refs[ue - 1].plan;
     const uint64_t fire_through = ends_a_layer ? last_layer : (last_layer == 0 ? UINT64_MAX : last_layer - 1);
     if (save) {
-      if (sl.used) PF_HIP(hipStreamWaitEvent(s, sl.freed, 0));
+      st = slot_begin(sl, s);
+      if (st != PF_OK) return st;
       st = launch_group(true);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.ready, s));
-      PF_HIP(hipStreamWaitEvent(side, sl.ready, 0));
+      st = slot_ready(sl, s, side);
+      if (st != PF_OK) return st;
       st = link_copies(true);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.freed, side));
+      st = slot_end(sl, side, side == s);
+      if (st != PF_OK) return st;
       prof_mark_first(side);
-      sl.used = true;
       if (fire_through != UINT64_MAX) {
         st = fire_events_through(fire_through, side);
         if (st != PF_OK) return st;
       }
     } else {
-      if (sl.used) PF_HIP(hipStreamWaitEvent(side, sl.freed, 0));
+      st = slot_begin(sl, side);
+      if (st != PF_OK) return st;
       st = link_copies(false);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.ready, side));
       prof_mark_first(side);
       st = upload_orders();
       if (st != PF_OK) return st;
-      PF_HIP(hipStreamWaitEvent(s, sl.ready, 0));
+      st = slot_ready(sl, side, s);
+      if (st != PF_OK) return st;
       st = launch_group(false);
       if (st != PF_OK) return st;
-      PF_HIP(hipEventRecord(sl.freed, s));
-      sl.used = true;
+      st = slot_end(sl, s, side == s);
+      if (st != PF_OK) return st;
       if (fire_through != UINT64_MAX) {
         st = fire_events_through(fire_through, s);
         if (st != PF_OK) return st;
@@ -1336,6 +1377,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     PF_HIP(hipEventRecord(join_, side));
     PF_HIP(hipStreamWaitEvent(s, join_, 0));
   }
+  st = slots_in_order_end(s);
+  if (st != PF_OK) return st;
   // Trailing empty layers.
   if (want_events && events_fired < n_layers) {
     st = fire_events_through(n_layers - 1, s);

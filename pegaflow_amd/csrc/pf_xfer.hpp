@@ -290,6 +290,7 @@ class Xfer {
     hipEvent_t ready = nullptr;  // contents complete (gather done / fill done)
     hipEvent_t freed = nullptr;  // contents consumed (drain done / scatter done)
     bool used = false;
+    bool in_order = false;  // used by the current call on one stream, not marked free yet
   };
 
   // Whole-page packing of page-first layers (see plan_page_pack).
@@ -304,6 +305,10 @@ class Xfer {
   int plan_layer(const pf_layer_blocks& in, const SecondSegmentTable& second, size_t index,
                  int path, LayerPlan* out, bool* skip);
   int ensure_slot(Slot& sl, uint64_t bytes);
+  int slot_begin(Slot& sl, hipStream_t writer);
+  int slot_ready(Slot& sl, hipStream_t writer, hipStream_t reader);
+  int slot_end(Slot& sl, hipStream_t reader, bool in_order);
+  int slots_in_order_end(hipStream_t s);
   uint32_t chunks_per_fragment(const LayerPlan& p, const BlockUnit& u) const;
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,

@@ -980,3 +980,43 @@ def test_call_size_rule_stages_small_layers_of_a_long_call(stream):
             c.close()
             h.close()
     xfer.close()
+
+
+@pytest.mark.parametrize("copy_stream", [1, 2], ids=["side_stream", "in_order"])
+def test_staging_slots_are_handed_on_between_calls_and_streams(gpu, copy_stream):
+    """Many fills per call through two small slots, calls on two streams in turn
+    with no synchronise between them: a call's first fills wait for the slots of
+    the call before, whichever stream that ran on."""
+    rng = np.random.default_rng(copy_stream)
+    xfer = BlockTransfer(staging_slot_bytes=256 << 10, copy_stream=copy_stream)
+    streams = [Stream(), Stream()]
+    cases = [Case(rng, num_blocks=96, seg=32768, segments=2) for _ in streams]
+    layouts = [c.product_layout() for c in cases]
+    hosts = [PinnedMemory(2 * len(c.ids) * 32768) for c in cases]
+    dests = [rng.choice(96, len(c.ids), replace=False).astype(np.uint32) for c in cases]
+    for c, h in zip(cases, hosts):
+        c.dev.copy_from_host(c.cache0)
+        h.as_numpy()[:] = SENT
+    for _ in range(4):
+        for c, layout, host, stream in zip(cases, layouts, hosts, streams):
+            xfer.save([_dense_layer(c, layout, host, c.ids)], stream, ST)
+    for s in streams:
+        s.synchronize()
+    for c in cases:
+        c.dev.fill(SENT)
+    for _ in range(4):
+        for c, layout, host, dest, stream in zip(cases, layouts, hosts, dests, streams):
+            xfer.load([_dense_layer(c, layout, host, dest)], stream, ST)
+    for s in streams:
+        s.synchronize()
+    for c, host, dest in zip(cases, hosts, dests):
+        src = c.cache0.reshape(2, 96, 32768)
+        assert np.array_equal(host.as_numpy().reshape(2, -1, 32768), src[:, c.ids])
+        expect = np.full_like(src, SENT)
+        expect[:, dest] = src[:, c.ids]
+        assert np.array_equal(c.dev.copy_to_host().reshape(src.shape), expect)
+        c.close()
+        host.close()
+    for s in streams:
+        s.close()
+    xfer.close()
