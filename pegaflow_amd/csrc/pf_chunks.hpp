@@ -1,0 +1,53 @@
+// The 16-byte chunks a fragment is cut into (kUnitChunks units and the tiles of
+// unaligned copies).  Arithmetic alone, for the kernels and the planner alike.
+#pragma once
+
+#include <cstdint>
+
+namespace pf {
+
+// Chunk boundaries lie on 16-byte boundaries of one side, whose address is `mis`
+// past one; the first and the last chunk overlap their neighbour and carry the
+// same bytes, so nothing is moved byte by byte: chunk i starts at
+// clamp(16 i - mis, 0, bytes - 16).  Needs 16 <= bytes <= kMaxChunkedBytes.
+constexpr uint64_t kMaxChunkedBytes = 0xFFFFFFFFull - 30;  // bytes + mis + 15 stays in 32 bits
+constexpr uint32_t chunk_count(uint32_t bytes, uint32_t mis) { return (bytes + mis + 15u) >> 4; }
+constexpr uint32_t chunk_start(uint32_t i, uint32_t bytes, uint32_t mis) {
+  const uint32_t raw = 16u * i;
+  const uint32_t in = raw > mis ? raw - mis : 0u;
+  const uint32_t last = bytes - 16u;
+  return in < last ? in : last;
+}
+
+// 16-byte chunks of a fragment of a zero-copy unit that is to be cut into chunks
+// (kUnitChunks), 0 when it keeps to tiles of one fragment.  `aligned`: every
+// fragment of the unit starts on a 16-byte boundary on both sides; `far_starts`:
+// the bitwise or of the numbers the host addresses of its fragments are sums of
+// multiples of (segment bases and stride), 1 when they come from a table;
+// `far_span`: bytes from the first to the end of the last fragment of a segment
+// in host memory, 0 for a table.
+//
+// Chunks are the faster form for every fragment off the 16-byte grid and, on
+// it, for fragments below 8 KiB, whose tiles leave half a workgroup and more
+// without work.  From there on both forms reach the link's rate in a long call
+// and the tile form, whose ids are scalar loads, is ahead in a short one (25 MB
+// per call, save / load in GB/s, chunks against tiles: 4112 bytes 56.1 / 55.9
+// against 51.4 / 51.5, 4 KiB 56.1 / 55.7 against 55.8 / 55.9, 8176 bytes 56.2 /
+// 56.1 against 56.2 / 56.7 for tiles of 8 KiB).
+constexpr uint32_t chunks_per_fragment(uint64_t frag, uint64_t n_blocks, bool aligned,
+                                       uint64_t far_starts, uint64_t far_span) {
+  // The kernel's chunk arithmetic is 32 bits wide and a segment's host image is
+  // one buffer descriptor; the tile form counts in 64 bits.
+  if (frag < 16 || frag > kMaxChunkedBytes || far_span > 0xFFFFFFF0ull) return 0;
+  if (aligned && frag >= 8192) return 0;
+  // A fragment whose host side starts off a 16-byte boundary may have one chunk
+  // more: the furthest off is what the alignment of all starts leaves open (1000
+  // bytes at multiples of 8: 63 chunks either way).
+  const uint64_t starts = aligned ? 16 : far_starts | 16;
+  const uint64_t alignment = starts & (~starts + 1);
+  const uint64_t chunks = (frag + (16 - alignment) + 15) / 16;
+  if (chunks * n_blocks >= (1ull << 31)) return 0;
+  return static_cast<uint32_t>(chunks);
+}
+
+}  // namespace pf

@@ -15,6 +15,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "pf_chunks.hpp"
 #include "pf_common.hpp"
 
 namespace pf {
@@ -157,24 +158,12 @@ __device__ __forceinline__ void copy_tile_vec(uint64_t dst, uint64_t src, uint32
 
 // Fragments that do not start on 16-byte boundaries are cut into 16-byte chunks
 // whose starts are aligned on ONE side (the link side where there is one: `mis`
-// is that side's address modulo 16) and unaligned on the other.  The first and
-// the last chunk are shifted inwards to lie inside the fragment, where they
-// overlap their neighbour and carry the same bytes, so nothing is moved byte by
-// byte: chunk i starts at clamp(16 i - mis, 0, bytes - 16).  Needs bytes >= 16.
+// is that side's address modulo 16) and unaligned on the other (chunk_start).
 // Measured on MI355X against words or, off the 4-byte grid, single bytes (one
 // load in flight per lane), descriptors over the link, 31 MB out and back:
 // 4097-byte fragments 3248 -> 1220 us, 12345 bytes 5932 -> 1190, 100001 bytes
 // 11717 -> 1230; packing 16 384 fragments of 4097 bytes in device memory 65 /
 // 101 us -> 38 / 31 (gather / scatter).
-__device__ __forceinline__ uint32_t chunk_count(uint32_t bytes, uint32_t mis) {
-  return (bytes + mis + 15u) >> 4;
-}
-__device__ __forceinline__ uint32_t chunk_start(uint32_t i, uint32_t bytes, uint32_t mis) {
-  const uint32_t raw = 16u * i;
-  const uint32_t in = raw > mis ? raw - mis : 0u;
-  const uint32_t last = bytes - 16u;
-  return in < last ? in : last;
-}
 __device__ __forceinline__ u32x4 load16_any(uint64_t addr) {
   return __builtin_nontemporal_load(reinterpret_cast<const g_u32x4_any*>(addr));
 }

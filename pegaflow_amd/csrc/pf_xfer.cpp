@@ -19,6 +19,7 @@
 #include <string>
 #include <vector>
 
+#include "pf_chunks.hpp"
 #include "pf_common.hpp"
 #include "pf_kernels.hpp"
 #include "pf_layout.hpp"
@@ -779,33 +780,6 @@ FillPlan plan_staged_fills(const std::vector<FillLayer>& layers, uint64_t slot_b
   return plan;
 }
 
-// 16-byte chunks of a fragment when the zero-copy unit `u` of layer `p` is to
-// be cut into chunks (kUnitChunks), 0 when it keeps to tiles of one fragment.
-// Chunks are the faster form for every fragment off the 16-byte grid and, on
-// it, for fragments below 8 KiB, whose tiles leave half a workgroup and more
-// without work.  From there on both forms reach the link's rate in a long call
-// and the tile form, whose ids are scalar loads, is ahead in a short one (25 MB
-// per call, save / load in GB/s, chunks against tiles: 4112 bytes 56.1 / 55.9
-// against 51.4 / 51.5, 4 KiB 56.1 / 55.7 against 55.8 / 55.9, 8176 bytes 56.2 /
-// 56.1 against 56.2 / 56.7 for tiles of 8 KiB).
-uint32_t Xfer::chunks_per_fragment(const LayerPlan& p, const BlockUnit& u) const {
-  const uint64_t frag = u.frag_bytes;
-  if (frag < 16 || (p.vec_ok && frag >= 8192)) return 0;
-  // A fragment whose host side starts off a 16-byte boundary may have one chunk
-  // more: the furthest off is what the alignment of all starts leaves open (1000
-  // bytes at multiples of 8: 63 chunks either way).
-  uint64_t starts = 16;
-  if (!p.vec_ok) {
-    starts |= p.page_dev != nullptr ? 1 : u.far_stride | u.far_base[0] | u.far_base[1];
-  }
-  const uint64_t alignment = starts & (~starts + 1);
-  const uint64_t chunks = (frag + (16 - alignment) + 15) / 16;
-  // 32-bit chunk indices, and one buffer descriptor for a segment's host image.
-  if (chunks * u.n_blocks >= (1ull << 31)) return 0;
-  if (p.page_dev == nullptr && (u.n_blocks - 1) * u.far_stride + frag > 0xFFFFFFF0ull) return 0;
-  return static_cast<uint32_t>(chunks);
-}
-
 int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save,
                    hipStream_t s, const SecondSegmentTable* second) {
   if (!timing_in_place_) timing_used_ = 0;
@@ -1090,7 +1064,10 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         u.far_stride = p.host_stride;
       }
       u.form = p.vec_ok ? kUnitVec : kUnitAny;
-      const uint32_t chunks = chunks_per_fragment(p, u);
+      const uint64_t span = p.page_dev ? 0 : (u.n_blocks - 1) * u.far_stride + u.frag_bytes;
+      const uint32_t chunks = chunks_per_fragment(
+          u.frag_bytes, u.n_blocks, p.vec_ok,
+          p.page_dev ? 1 : u.far_stride | u.far_base[0] | u.far_base[1], span);
       if (chunks != 0) {
         u.form = kUnitChunks;
         u.tiles_per_frag = chunks;

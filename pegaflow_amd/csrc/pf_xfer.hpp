@@ -309,7 +309,6 @@ class Xfer {
   int slot_ready(Slot& sl, hipStream_t writer, hipStream_t reader);
   int slot_end(Slot& sl, hipStream_t reader, bool in_order);
   int slots_in_order_end(hipStream_t s);
-  uint32_t chunks_per_fragment(const LayerPlan& p, const BlockUnit& u) const;
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
                      uint64_t min_frag_bytes, bool to_far, hipStream_t s);
