@@ -231,11 +231,13 @@ def _pack_hashes(hashes: Sequence[bytes]):
 def _pack_destinations(ids: Sequence[int | None]):
     """-> (int64 array for C, what owns it) of one destination list, None as -1."""
     n = len(ids)
-    try:
-        packed = np.asarray(ids)
-    except ValueError:  # nested lists: int() says what is wrong with them
-        packed = np.empty(0)
-    if n and packed.ndim == 1 and packed.dtype.kind in "iu":
+    packed = None
+    if type(ids) in (list, tuple, np.ndarray):
+        try:
+            packed = np.array(ids)
+        except Exception:  # an entry's own conversion refuses (a tensor in device memory): int() decides
+            packed = None
+    if n and packed is not None and packed.ndim == 1 and packed.dtype.kind in "iu":
         packed = np.ascontiguousarray(packed.astype(np.int64, copy=False))
         return C.cast(packed.ctypes.data, C.POINTER(C.c_int64)), packed
     d = (C.c_int64 * max(n, 1))(*[-1 if v is None else int(v) for v in ids])

@@ -194,3 +194,48 @@ def test_transfer_mode_names():
     assert TransferMode.from_name(" Kernel ") == TransferMode.KERNEL
     with pytest.raises(_lib.InvalidArgument, match="expected one of: direct, kernel"):
         TransferMode.from_name("nccl")
+
+
+class _Refuses:
+    """Integers that convert with int(), whose conversion to an array raises, as
+    that of a tensor in device memory does."""
+
+    def __init__(self, value, error):
+        self.value, self.error = value, error
+
+    def __int__(self):
+        return self.value
+
+    __index__ = __int__
+
+    def __len__(self):
+        return len(self.value)
+
+    def __iter__(self):
+        return (_Refuses(v, self.error) for v in self.value)
+
+    def __array__(self, *args, **kwargs):
+        raise self.error("convert it to host memory first")
+
+
+@pytest.mark.parametrize("ids", [
+    [], [3], [3, None, 5], [None, None], (7, 8), [True, 2], [1.0, 2.5], ["4", "5"], [2**63 - 1, 0], [2**64 - 1],
+    np.arange(6, dtype=np.int32)[::-2], np.arange(4, dtype=np.uint64), np.array([1, None], dtype=object),
+    np.arange(6).reshape(3, 2)[:, 1], np.array([1, 2], dtype=">i8"), range(3),
+    [_Refuses(4, TypeError), _Refuses(9, TypeError)], [_Refuses(4, RuntimeError), None],
+    _Refuses([5, 6, 7], TypeError), _Refuses([5, 6, 7], RuntimeError),
+], ids=lambda v: type(v).__name__ + str(len(v)))
+def test_destination_lists_of_any_kind(ids):
+    """Whatever int() takes entry by entry is a destination list."""
+    from pegaflow_amd.engine import _pack_destinations
+    want = [-1 if v is None else C.c_int64(int(v)).value for v in ids]
+    packed, owner = _pack_destinations(ids)
+    assert [packed[i] for i in range(len(want))] == want
+    assert owner is not ids
+
+
+@pytest.mark.parametrize("ids", [[[1], [2, 3]], [[1, 2], [3, 4]], ["x"], [object()], np.zeros((2, 2), dtype=np.int64)])
+def test_destination_lists_that_are_refused(ids):
+    from pegaflow_amd.engine import _pack_destinations
+    with pytest.raises((TypeError, ValueError)):
+        _pack_destinations(ids)
