@@ -162,8 +162,7 @@ __device__ __forceinline__ void copy_tile_vec(uint64_t dst, uint64_t src, uint32
 // Measured on MI355X against words or, off the 4-byte grid, single bytes (one
 // load in flight per lane), descriptors over the link, 31 MB out and back:
 // 4097-byte fragments 3248 -> 1220 us, 12345 bytes 5932 -> 1190, 100001 bytes
-// 11717 -> 1230; packing 16 384 fragments of 4097 bytes in device memory 65 /
-// 101 us -> 38 / 31 (gather / scatter).
+// 11717 -> 1230.
 __device__ __forceinline__ u32x4 load16_any(uint64_t addr) {
   return __builtin_nontemporal_load(reinterpret_cast<const g_u32x4_any*>(addr));
 }
@@ -206,6 +205,31 @@ __device__ __forceinline__ void copy_tile_any(uint64_t dst, uint64_t src, uint32
       }
     }
   });
+}
+
+// The same between two places in device memory, one chunk per lane and step, with
+// ordinary loads and stores: a fragment off the 16-byte grid starts and ends
+// inside a memory line that the next workgroup's fragment or tile shares, and the
+// caches put the two halves together.  Streaming accesses send each half to
+// memory by itself.  Measured on MI355X, 50 MB in two staged layers of K and V,
+// save / load in us with streaming accesses, with words and single bytes, and
+// with this: fragments of 516 bytes 1103 / 1045, 964 / 982, 961 / 966; 4100 bytes
+// 972 / 970, 939 / 951, 934 / 938; 20 004 bytes 965 / 967, 934 / 948, 931 / 935;
+// 1001 bytes 1023 / 1023, 970 / 999, 949 / 954; 20 bytes 2844 / 2753, 2466 / 2523,
+// 2440 / 2496.
+template <int LANES>
+__device__ __forceinline__ void copy_tile_in_hbm(uint64_t dst, uint64_t src, uint32_t bytes,
+                                                 uint32_t lane) {
+  if (bytes < 16) {
+    if (lane < bytes) reinterpret_cast<g_u8*>(dst)[lane] = reinterpret_cast<const g_u8*>(src)[lane];
+    return;
+  }
+  const uint32_t mis = static_cast<uint32_t>(dst) & 15u;
+  const uint32_t n = chunk_count(bytes, mis);
+  for (uint32_t i = lane; i < n; i += LANES) {
+    const uint32_t at = chunk_start(i, bytes, mis);
+    *reinterpret_cast<g_u32x4_any*>(dst + at) = *reinterpret_cast<const g_u32x4_any*>(src + at);
+  }
 }
 
 // Rows of a descriptor table, wave-uniform.  Rows3: [dst, src, size] as the
@@ -552,7 +576,7 @@ __device__ __forceinline__ void block_tiles_copy(UnitPtr up, uint32_t row, uint3
     const uint32_t j = (nvec << 4) + lane;
     if (j < bytes) reinterpret_cast<g_u8*>(dst)[j] = reinterpret_cast<const g_u8*>(src)[j];
   } else {
-    copy_tile_any<1, LT, false>(dst, src, bytes, lane);
+    copy_tile_in_hbm<LT>(dst, src, bytes, lane);
   }
 }
 
