@@ -351,6 +351,29 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
   return f;
 }
 
+// Where the tiles of a unit begin in its row of workgroups: take() gives a
+// workgroup's first tile of the next unit, the others follow grid_x apart.  A unit
+// with a few tiles more than whole rounds passes the turn on to the workgroup
+// behind its last tile; beginning every unit at workgroup 0 gives the same few
+// workgroups the odd tiles of all units (30 layers of 136 blocks of 6144 bytes, 51
+// tiles each for 48 workgroups, saved / loaded in 477 / 501 us, in turn in 450 /
+// 451; 30 layers of 203 blocks of 4 KiB loaded in 475, in turn in 452).  Where the
+// last round keeps more of the row busy the units stay at workgroup 0: 16 layers
+// of 777 blocks of 1000 bytes (96 tiles, 64 workgroups) loaded in 458 us, in turn
+// in 464.
+struct RowTurn {
+  uint32_t at = 0;  // workgroup whose turn it is
+  __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t grid_x) {
+    const uint32_t first = blockIdx.x >= at ? blockIdx.x - at : blockIdx.x + grid_x - at;
+    const uint32_t odd = n_tiles < grid_x ? n_tiles : n_tiles % grid_x;
+    if (odd * 4 < grid_x) {
+      at += odd;
+      if (at >= grid_x) at -= grid_x;
+    }
+    return first;
+  }
+};
+
 // A unit of the zero-copy form whose fragments are cut into 16-byte chunks (see
 // chunk_start) that fill the lanes one after the other, whatever fragment they
 // belong to: lane l of step k handles chunk 1024 t + 256 k + l of a segment.
@@ -364,14 +387,15 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
 // 39.1 -> 56.1 / 55.8, 4112 bytes 52.2 / 44.4 -> 56.1 / 55.9, 100 004 bytes
 // (tile form with the chunks of copy_tile_any) 44.6 / 52.1 -> 52.8 / 54.8.
 template <int U, bool TO_FAR>
-__device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t grid_x) {
+__device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t grid_x,
+                                                  RowTurn& turn) {
   const uint32_t frag_bytes = static_cast<uint32_t>(f.frag_bytes);
   const uint32_t chunks_per_frag = f.tiles_per_frag;
   // The host keeps a unit's chunk count below 2^31.
   const uint32_t n_chunks = f.n_blocks * chunks_per_frag;
   const uint32_t tiles_per_seg = (n_chunks + U * kLanes - 1) / (U * kLanes);
   const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-  for (uint32_t t = blockIdx.x; t < n_tiles; t += grid_x) {
+  for (uint32_t t = turn.take(n_tiles, grid_x); t < n_tiles; t += grid_x) {
     const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
     const uint32_t first = (seg ? t - tiles_per_seg : t) * (U * kLanes) + threadIdx.x;
     const uint64_t near_seg = f.near_base + (seg ? f.kv_stride : 0);
@@ -456,17 +480,18 @@ template <int U, bool TO_FAR, typename UnitPtr>
 __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units, uint32_t grid_x,
                                                  uint32_t grid_y, uint64_t bias) {
   constexpr uint64_t kTile = static_cast<uint64_t>(U) * kLanes * 16;
+  RowTurn turn;
   for (uint32_t unit = blockIdx.y; unit < n_units; unit += grid_y) {
     const UnitFields f = unit_fields(units + unit, bias);
     if (f.form == kUnitChunks) {
-      block_chunks_unit<U, TO_FAR>(f, grid_x);
+      block_chunks_unit<U, TO_FAR>(f, grid_x, turn);
       continue;
     }
     const bool vec_ok = f.form == kUnitVec;
     // The host keeps a unit's tile count below 2^32, so 32-bit scalar division.
     const uint32_t tiles_per_seg = f.n_blocks * f.tiles_per_frag;
     const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-    for (uint32_t t = blockIdx.x; t < n_tiles; t += grid_x) {
+    for (uint32_t t = turn.take(n_tiles, grid_x); t < n_tiles; t += grid_x) {
       const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
       const uint32_t r = seg ? t - tiles_per_seg : t;
       // The quotient is wave-uniform; pin it to a scalar register so the id and

@@ -1020,3 +1020,39 @@ def test_staging_slots_are_handed_on_between_calls_and_streams(gpu, copy_stream)
     for s in streams:
         s.close()
     xfer.close()
+
+
+@pytest.mark.parametrize("workgroups", [1, 3, 16, 0])
+def test_tiles_of_unlike_units_are_dealt_out_once(stream, workgroups):
+    """Zero-copy units of one launch take turns: unit after unit begins at the
+    workgroup behind the one that took the last tile.  Tile counts below, at and
+    above the number of workgroups and multiples of it, whole tiles and chunks,
+    one and two segments; every byte once, none beside them."""
+    rng = np.random.default_rng(workgroups)
+    shapes = [(n, seg, segments)
+              for n in (1, 2, 3, 4, 15, 16, 17, 33, 48, 50) for seg, segments in ((16384, 1), (1040, 2), (32784, 2))]
+    rng.shuffle(shapes)
+    xfer = BlockTransfer(zerocopy_max_workgroups=workgroups)
+    cases = [Case(rng, num_blocks=int(n) + 9, seg=int(seg), segments=int(segments), n_ids=int(n))
+             for n, seg, segments in shapes]
+    layouts = [c.product_layout() for c in cases]
+    hosts = [PinnedMemory(c.segments * len(c.ids) * c.seg) for c in cases]
+    for c, h in zip(cases, hosts):
+        c.dev.copy_from_host(c.cache0)
+        h.as_numpy()[:] = SENT
+    xfer.save([_dense_layer(c, L, h, c.ids) for c, L, h in zip(cases, layouts, hosts)], stream, ZC)
+    stream.synchronize()
+    dests = [rng.choice(c.num_blocks, len(c.ids), replace=False).astype(np.uint32) for c in cases]
+    for c in cases:
+        c.dev.fill(SENT)
+    xfer.load([_dense_layer(c, L, h, d) for c, L, h, d in zip(cases, layouts, hosts, dests)], stream, ZC)
+    stream.synchronize()
+    for c, host, dest in zip(cases, hosts, dests):
+        src = c.cache0.reshape(c.segments, c.num_blocks, c.seg)
+        assert np.array_equal(host.as_numpy().reshape(c.segments, -1, c.seg), src[:, c.ids]), c.args
+        expect = np.full_like(src, SENT)
+        expect[:, dest] = src[:, c.ids]
+        assert np.array_equal(c.dev.copy_to_host().reshape(src.shape), expect), c.args
+        c.close()
+        host.close()
+    xfer.close()
