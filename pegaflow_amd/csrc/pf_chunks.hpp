@@ -27,19 +27,28 @@ constexpr uint32_t chunk_start(uint32_t i, uint32_t bytes, uint32_t mis) {
 // `far_span`: bytes from the first to the end of the last fragment of a segment
 // in host memory, 0 for a table.
 //
-// Chunks are the faster form for every fragment off the 16-byte grid and, on
-// it, for fragments below 8 KiB, whose tiles leave half a workgroup and more
-// without work.  From there on both forms reach the link's rate in a long call
-// and the tile form, whose ids are scalar loads, is ahead in a short one (25 MB
-// per call, save / load in GB/s, chunks against tiles: 4112 bytes 56.1 / 55.9
-// against 51.4 / 51.5, 4 KiB 56.1 / 55.7 against 55.8 / 55.9, 8176 bytes 56.2 /
-// 56.1 against 56.2 / 56.7 for tiles of 8 KiB).
-constexpr uint32_t chunks_per_fragment(uint64_t frag, uint64_t n_blocks, bool aligned,
+// Chunks are the faster form for every fragment off the 16-byte grid and, on it,
+// for fragments below 8 KiB, whose tiles leave lanes without work, except where
+// one step of a tile takes the fragment whole and fills three quarters of its
+// wavefronts (fills_one_step): there both reach the link's rate in a long call
+// and the tile form, whose ids are scalar loads, is ahead in a short one.
+// Measured on MI355X, two layers of K and V, 1 / 4 / 20 MB per call, loads in us,
+// chunks against tiles: 2048 bytes 24.1 / 76.3 / 361 against 21.7 / 74.4 / 363,
+// 3072 bytes 24.1 / 76.4 / 365 against 21.9 / 74.0 / 353, 4096 bytes 24.1 / 76.4 /
+// 356 against 21.8 / 74.6 / 353, but 1040 bytes 24.4 / 77.9 / 375 against 28.0 /
+// 101 / 507, 4112 bytes 23.3 / 77.7 / 359 against 22.7 / 80.5 / 380, 7680 bytes
+// 22.2 / 75.8 / 354 against 21.9 / 76.2 / 366.  Saves gain from tiles later: 30
+// layers, 20 MB, 2048 bytes 363 against 375, 2560 bytes 362 / 365, 3072 bytes 364 /
+// 363.
+constexpr bool fills_one_step(uint64_t frag, bool save) {
+  return frag >= (save ? 3072 : 2048) && frag <= 4096 && frag * 4 >= 3 * ((frag + 1023) / 1024 * 1024);
+}
+constexpr uint32_t chunks_per_fragment(uint64_t frag, uint64_t n_blocks, bool aligned, bool save,
                                        uint64_t far_starts, uint64_t far_span) {
   // The kernel's chunk arithmetic is 32 bits wide and a segment's host image is
   // one buffer descriptor; the tile form counts in 64 bits.
   if (frag < 16 || frag > kMaxChunkedBytes || far_span > 0xFFFFFFF0ull) return 0;
-  if (aligned && frag >= 8192) return 0;
+  if (aligned && (frag >= 8192 || fills_one_step(frag, save))) return 0;
   // A fragment whose host side starts off a 16-byte boundary may have one chunk
   // more: the furthest off is what the alignment of all starts leaves open (1000
   // bytes at multiples of 8: 63 chunks either way).

@@ -352,21 +352,21 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
 }
 
 // Where the tiles of a unit begin in its row of workgroups: take() gives a
-// workgroup's first tile of the next unit, the others follow grid_x apart.  A unit
-// with a few tiles more than whole rounds passes the turn on to the workgroup
-// behind its last tile; beginning every unit at workgroup 0 gives the same few
-// workgroups the odd tiles of all units (30 layers of 136 blocks of 6144 bytes, 51
-// tiles each for 48 workgroups, saved / loaded in 477 / 501 us, in turn in 450 /
-// 451; 30 layers of 203 blocks of 4 KiB loaded in 475, in turn in 452).  Where the
-// last round keeps more of the row busy the units stay at workgroup 0: 16 layers
-// of 777 blocks of 1000 bytes (96 tiles, 64 workgroups) loaded in 458 us, in turn
-// in 464.
+// workgroup's first tile of the next unit, the others follow grid_x apart.  The
+// turn passes on to the workgroup behind the unit's last tile; beginning every
+// unit at workgroup 0 gives the same workgroups the odd tiles of all units (24
+// layers of 72 blocks of 3072 bytes, whole tiles, loaded in 126 us, in turn in 90;
+// 30 layers of 136 blocks of 6144 bytes, 51 tiles of chunks each for 48
+// workgroups, saved / loaded in 477 / 501, in turn in 450 / 451).  Units in chunks
+// of which more than `most_odd` tiles are left after whole rounds stay at workgroup
+// 0: 16 layers of 777 blocks of 1000 bytes (96 tiles, 64 workgroups) loaded in 458
+// us, in turn in 464.
 struct RowTurn {
   uint32_t at = 0;  // workgroup whose turn it is
-  __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t grid_x) {
+  __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t grid_x, uint32_t most_odd) {
     const uint32_t first = blockIdx.x >= at ? blockIdx.x - at : blockIdx.x + grid_x - at;
     const uint32_t odd = n_tiles < grid_x ? n_tiles : n_tiles % grid_x;
-    if (odd * 4 < grid_x) {
+    if (odd <= most_odd) {
       at += odd;
       if (at >= grid_x) at -= grid_x;
     }
@@ -395,7 +395,7 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
   const uint32_t n_chunks = f.n_blocks * chunks_per_frag;
   const uint32_t tiles_per_seg = (n_chunks + U * kLanes - 1) / (U * kLanes);
   const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-  for (uint32_t t = turn.take(n_tiles, grid_x); t < n_tiles; t += grid_x) {
+  for (uint32_t t = turn.take(n_tiles, grid_x, grid_x / 4); t < n_tiles; t += grid_x) {
     const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
     const uint32_t first = (seg ? t - tiles_per_seg : t) * (U * kLanes) + threadIdx.x;
     const uint64_t near_seg = f.near_base + (seg ? f.kv_stride : 0);
@@ -491,7 +491,7 @@ __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units
     // The host keeps a unit's tile count below 2^32, so 32-bit scalar division.
     const uint32_t tiles_per_seg = f.n_blocks * f.tiles_per_frag;
     const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-    for (uint32_t t = turn.take(n_tiles, grid_x); t < n_tiles; t += grid_x) {
+    for (uint32_t t = turn.take(n_tiles, grid_x, grid_x); t < n_tiles; t += grid_x) {
       const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
       const uint32_t r = seg ? t - tiles_per_seg : t;
       // The quotient is wave-uniform; pin it to a scalar register so the id and

@@ -1066,7 +1066,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       u.form = p.vec_ok ? kUnitVec : kUnitAny;
       const uint64_t span = p.page_dev ? 0 : (u.n_blocks - 1) * u.far_stride + u.frag_bytes;
       const uint32_t chunks = chunks_per_fragment(
-          u.frag_bytes, u.n_blocks, p.vec_ok,
+          u.frag_bytes, u.n_blocks, p.vec_ok, save,
           p.page_dev ? 1 : u.far_stride | u.far_base[0] | u.far_base[1], span);
       if (chunks != 0) {
         u.form = kUnitChunks;

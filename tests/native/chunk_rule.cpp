@@ -22,7 +22,7 @@ int main() {
         for (const uint64_t blocks : {1ull, 7ull, 4096ull, 1ull << 27}) {
           for (const bool table : {false, true}) {
             const uint64_t span = table ? 0 : (blocks - 1) * 512 + frag;
-            const uint32_t n = pf::chunks_per_fragment(frag, blocks, aligned, table ? 1 : far_starts, span);
+            const uint32_t n = pf::chunks_per_fragment(frag, blocks, aligned, blocks == 7, table ? 1 : far_starts, span);
             if (n == 0) continue;
             ++cut;
             bool ok = frag <= 0xFFFFFFFFull && static_cast<uint64_t>(n) * blocks < (1ull << 31) && span <= 0xFFFFFFF0ull;
@@ -57,9 +57,18 @@ int main() {
       }
     }
   }
-  // The form is used where it pays.
-  if (pf::chunks_per_fragment(1000, 777, false, 8, 777000) != 63 || pf::chunks_per_fragment(4096, 16, true, 16, 0) != 256 ||
-      pf::chunks_per_fragment(8192, 16, true, 16, 0) != 0 || cut < 1000) {
+  // The form is used where it pays: aligned fragments that fill three quarters of
+  // the wavefronts of one step (loads from 2 KiB, saves from 3 KiB, up to 4 KiB)
+  // and those from 8 KiB on keep to tiles.
+  auto aligned = [](uint64_t frag, bool save) { return pf::chunks_per_fragment(frag, 16, true, save, 16, 0) != 0; };
+  for (uint64_t f : {16ull, 1024ull, 1536ull, 2032ull, 2064ull, 2288ull, 4112ull, 5120ull, 6144ull, 8176ull}) {
+    if (!aligned(f, false) || !aligned(f, true)) return printf("%" PRIu64 " bytes in tiles\n", f), 1;
+  }
+  for (uint64_t f : {2048ull, 2304ull, 2560ull, 3072ull, 3088ull, 3584ull, 4080ull, 4096ull, 8192ull, 16384ull}) {
+    if (aligned(f, false) || aligned(f, true) != (f < 3072)) return printf("%" PRIu64 " bytes in chunks\n", f), 1;
+  }
+  if (pf::chunks_per_fragment(1000, 777, false, true, 8, 777000) != 63 ||
+      pf::chunks_per_fragment(4096, 16, false, false, 8, 1 << 20) != 257 || cut < 1000) {
     printf("rule\n");
     return 1;
   }

@@ -170,8 +170,8 @@ def test_save_load_matches_oracle(name, path, xfer, stream):
 
 
 # Zero-copy units cut into 16-byte chunks: the smallest fragment that has one,
-# fragments around the sizes where another form takes over (16 bytes, 8 KiB on
-# the 16-byte grid), segments of 1023, 1024 and 1025 chunks (a tile holds 1024)
+# fragments around the sizes where another form takes over (16 bytes, 2 to 4 KiB
+# and 8 KiB on the 16-byte grid), segments of 1023, 1024 and 1025 chunks (a tile holds 1024)
 # and a last tile with chunks for one wavefront only; aligned and not, dense and
 # padded.
 CHUNKS = {
@@ -184,6 +184,8 @@ CHUNKS = {
     "one_wave_in_the_last_tile": dict(num_blocks=80, seg=272, segments=2, n_ids=64),
     "padded_odd": dict(num_blocks=60, seg=1332, segments=2, pad_to=512),
     "off_grid_base": dict(num_blocks=60, seg=1040, segments=2, base_off=7),
+    "2304_in_tiles": dict(num_blocks=70, seg=2304, segments=2, n_ids=67),
+    "4080_in_tiles": dict(num_blocks=40, seg=4080, segments=1),
     "below_8k": dict(num_blocks=20, seg=8176, segments=2),
     "at_8k": dict(num_blocks=20, seg=8192, segments=2),
     "off_grid_40k": dict(num_blocks=12, seg=40003, segments=2, base_off=1),
