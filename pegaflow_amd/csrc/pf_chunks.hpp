@@ -59,4 +59,21 @@ constexpr uint32_t chunks_per_fragment(uint64_t frag, uint64_t n_blocks, bool al
   return static_cast<uint32_t>(chunks);
 }
 
+// Workgroups that a unit of a zero-copy launch needs to keep the link full: of
+// full tiles `full_tiles`, more of smaller ones, at most `most`.  Saves and units
+// in chunks take a whole multiple for every started share of a tile; a load of
+// whole fragments takes them in proportion, since reads beyond what the link holds
+// slow it down: fragments of 12 288 bytes had 32 workgroups and 393 KB in flight
+// and loaded (20 MB) in 367 us, with 22 in 352; 11 264 bytes 364 -> 352, 14 336
+// bytes 364 -> 352, 15 360 bytes 362 -> 353.  (In proportion, saves of 24 layers of
+// 13 312-byte fragments, 5 MB, took 86 us instead of 82, and loads in chunks, 30
+// layers of 7680 bytes, 382 instead of 360: chunks wait for their ids first.)
+constexpr uint32_t unit_workgroups(uint64_t frag, bool in_proportion, uint32_t tile, uint32_t full_tiles,
+                                   uint32_t most) {
+  if (frag == 0 || frag >= tile) return full_tiles;
+  const uint64_t n = in_proportion ? (static_cast<uint64_t>(full_tiles) * tile + frag - 1) / frag
+                                   : full_tiles * ((tile + frag - 1) / frag);
+  return n < most ? static_cast<uint32_t>(n) : most;
+}
+
 }  // namespace pf

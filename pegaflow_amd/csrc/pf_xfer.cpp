@@ -217,22 +217,22 @@ int Xfer::timing_end(hipStream_t s) {
 }
 
 int Xfer::launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
-                         uint64_t min_frag_bytes, bool to_far, hipStream_t s) {
+                         uint32_t workgroups, bool to_far, hipStream_t s) {
   int st = timing_begin(s);
   if (st != PF_OK) return st;
   st = launch_block_units(dev_units, n_units, max_tiles, to_far, unroll_,
-                          zero_copy_workgroups(min_frag_bytes), s);
+                          workgroups, s);
   if (st != PF_OK) return st;
   return timing_end(s);
 }
 
 int Xfer::launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
-                              uint64_t max_tiles, uint64_t min_frag_bytes, bool to_far,
+                              uint64_t max_tiles, uint32_t workgroups, bool to_far,
                               hipStream_t s) {
   int st = timing_begin(s);
   if (st != PF_OK) return st;
   st = launch_block_units_args(slab, first_unit, n_units, max_tiles, to_far, unroll_,
-                               zero_copy_workgroups(min_frag_bytes), s);
+                               workgroups, s);
   if (st != PF_OK) return st;
   return timing_end(s);
 }
@@ -1149,19 +1149,19 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       // wants a completion event per layer.
       size_t uj = ui + 1;
       uint64_t max_tiles = tiles_of(units_host[ui]);
-      uint64_t min_frag = units_host[ui].frag_bytes;
+      uint32_t workgroups = zero_copy_workgroups(units_host[ui], save);
       if (!want_events) {
         while (uj < unit_refs.size() && !plans[unit_refs[uj].plan].staged) {
           max_tiles = std::max(max_tiles, tiles_of(units_host[uj]));
-          min_frag = std::min(min_frag, units_host[uj].frag_bytes);
+          workgroups = std::max(workgroups, zero_copy_workgroups(units_host[uj], save));
           ++uj;
         }
       }
       if (in_args) {
         st = launch_strided_args(arg_slab, static_cast<uint32_t>(ui), static_cast<uint32_t>(uj - ui),
-                                 max_tiles, min_frag, save, s);
+                                 max_tiles, workgroups, save, s);
       } else {
-        st = launch_strided(units_dev + ui, static_cast<uint32_t>(uj - ui), max_tiles, min_frag,
+        st = launch_strided(units_dev + ui, static_cast<uint32_t>(uj - ui), max_tiles, workgroups,
                             save, s);
       }
       if (st != PF_OK) return st;

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/pegahip.h"
+#include "pf_chunks.hpp"
 #include "pf_common.hpp"
 #include "pf_kernels.hpp"
 #include "pf_layout.hpp"
@@ -120,7 +121,7 @@ constexpr int kDefaultUnroll = 4;
 // its 256 workgroups of 512 registers per lane need every compute unit.)
 // Sixteen workgroups of full 16 KiB tiles keep 256 KiB in flight, twice the
 // link's bandwidth-delay product; fragments smaller than a tile get
-// proportionally more workgroups, up to 64.
+// more workgroups, up to 64 (unit_workgroups).
 constexpr uint32_t kZeroCopyWorkgroupsFullTiles = 16;
 constexpr uint32_t kZeroCopyWorkgroupsMax = 64;
 
@@ -311,18 +312,16 @@ class Xfer {
   int slots_in_order_end(hipStream_t s);
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
-                     uint64_t min_frag_bytes, bool to_far, hipStream_t s);
-  // Workgroups of a zero-copy launch whose smallest fragment is `min_frag_bytes`.
-  uint32_t zero_copy_workgroups(uint64_t min_frag_bytes) const {
+                     uint32_t workgroups, bool to_far, hipStream_t s);
+  // Workgroups that a zero-copy unit asks its launch for.
+  uint32_t zero_copy_workgroups(const BlockUnit& u, bool save) const {
     if (zc_max_wg_ != 0) return zc_max_wg_;
-    const uint64_t tile = tile_bytes(unroll_);
-    if (min_frag_bytes == 0 || min_frag_bytes >= tile) return kZeroCopyWorkgroupsFullTiles;
-    const uint64_t scaled = kZeroCopyWorkgroupsFullTiles * ((tile + min_frag_bytes - 1) / min_frag_bytes);
-    return static_cast<uint32_t>(scaled < kZeroCopyWorkgroupsMax ? scaled : kZeroCopyWorkgroupsMax);
+    return unit_workgroups(u.frag_bytes, !save && u.form != kUnitChunks, tile_bytes(unroll_),
+                           kZeroCopyWorkgroupsFullTiles, kZeroCopyWorkgroupsMax);
   }
   // The same with the slab in the launch's arguments (short lists).
   int launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
-                          uint64_t max_tiles, uint64_t min_frag_bytes, bool to_far, hipStream_t s);
+                          uint64_t max_tiles, uint32_t workgroups, bool to_far, hipStream_t s);
   // Staged form: one tile per workgroup over one unit.
   int launch_tiles(const BlockUnit* dev_unit, const BlockUnit& host_unit, bool to_far,
                    hipStream_t s);

@@ -72,6 +72,16 @@ int main() {
     printf("rule\n");
     return 1;
   }
+  // In proportion, fragments keep 256 KiB in flight, no more than a fragment over; never fewer
+  // workgroups than full tiles need nor more than the cap.
+  for (uint64_t f = 1; f <= 40000; ++f) {
+    const uint64_t tiles = pf::unit_workgroups(f, true, 16384, 16, 64);
+    const bool ok = f >= 16384 ? tiles == 16 : tiles == 64 ? f <= 4161 : tiles * f >= 262144 && (tiles - 1) * f < 262144;
+    const uint64_t multiple = pf::unit_workgroups(f, false, 16384, 16, 64);
+    if (!ok || multiple < tiles || multiple > 64 || multiple % 16 != 0) {
+      return printf("%" PRIu64 " bytes: %" PRIu64 " / %" PRIu64 " workgroups\n", f, tiles, multiple), 1;
+    }
+  }
   printf("all ok\n");
   return 0;
 }
