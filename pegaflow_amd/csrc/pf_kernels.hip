@@ -182,6 +182,17 @@ __device__ __forceinline__ void copy_tile_any(uint64_t dst, uint64_t src, uint32
   }
   const uint32_t mis = static_cast<uint32_t>(ALIGN_SRC ? src : dst) & 15u;
   const uint32_t n = chunk_count(bytes, mis);
+  // A short row is one trip there and back, of which the choice of a body and of a
+  // store policy below are a measurable part (48 rows of 24 bytes out and back
+  // 25.8 us, this way 23.7; 1500 bytes 26.0 and 24.3).  From 188 chunks on the
+  // body below is the faster one again (7000 rows of 3000 bytes 884 against 908).
+  if (n <= LANES && n <= 2 * kWave) {
+    if (lane < n) {
+      const uint32_t at = chunk_start(lane, bytes, mis);
+      store16_any(dst + at, load16_any(src + at));
+    }
+    return;
+  }
   const __amdgpu_buffer_rsrc_t tile = tile_descriptor(dst, bytes);
   // A full tile that starts off a boundary has one chunk more than U steps hold.
   with_steps<U + 1>(wave_steps<LANES>(n, lane), [&](auto steps) {
@@ -1044,20 +1055,22 @@ int launch_plain_copy(void* dst, const void* src, uint64_t bytes, int unroll, hi
 
 namespace {
 // Launch of a descriptor copy: a row per wavefront while the largest row is
-// half a wavefront's tile, otherwise a row per workgroup, x over descriptors
-// and y over the tiles of the largest one.  From 4 KiB rows on both reach the
-// link's rate in a long batch and a row per workgroup is ahead in a short one
-// (437 rows of 4 KiB, there and back 78.6 against 79.5 us).  The kernels stride
-// over what the grid does not cover; `max_workgroups` (0 = no cap) bounds the
-// whole launch.
+// half a wavefront's tile and there are rows for more than kFewRows workgroups,
+// otherwise a row per workgroup, x over descriptors and y over the tiles of the
+// largest one.  From 4 KiB rows on both reach the link's rate in a long batch and
+// a row per workgroup is ahead in a short one (437 rows of 4 KiB, there and back
+// 78.6 against 79.5 us); few rows are a compute unit's work each (48 rows of 1500
+// bytes 25.3 against 25.9).  The kernels stride over what the grid does not cover;
+// `max_workgroups` (0 = no cap) bounds the whole launch.
 constexpr uint64_t kWaveRowBytes = 2048;
+constexpr uint64_t kFewRows = 64;
 
 template <bool HOST_IS_SRC, typename Rows>
 void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
                  uint32_t max_workgroups) {
   const dim3 block(kLanes, 1, 1);
   constexpr uint64_t kWaves = kLanes / kWave;
-  if (max_size <= kWaveRowBytes) {
+  if (max_size <= kWaveRowBytes && n > kFewRows) {
     uint64_t gx = (n + kWaves - 1) / kWaves;
     if (max_workgroups != 0 && gx > max_workgroups) gx = max_workgroups;
     if (gx > kMaxGridX) gx = kMaxGridX;
@@ -1069,6 +1082,7 @@ void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
   constexpr uint64_t kTile = tile_bytes(kDescUnroll);
   uint64_t gx = n < kMaxGridX ? n : kMaxGridX;
   uint64_t gy = (max_size + kTile - 1) / kTile;
+  if (gy < 1) gy = 1;
   if (gy > 64) gy = 64;
   if (max_workgroups != 0) {
     while (gx * gy > max_workgroups && gy > 1) gy >>= 1;

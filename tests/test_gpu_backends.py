@@ -116,9 +116,9 @@ def test_unaligned_and_odd_sizes_match_oracle(backends, stream, direction):
 
 
 @pytest.mark.parametrize("direction", ["h2d", "d2h"])
-@pytest.mark.parametrize("n, slot", [(70, 2080), (1300, 2080), (1300, 4128), (70, 16416), (9, 70000)])
+@pytest.mark.parametrize("n, slot", [(64, 2080), (65, 2080), (1300, 2080), (1300, 4128), (70, 16416), (9, 70000)])
 def test_rows_of_any_size_and_alignment(backends, stream, n, slot, direction):
-    """Row per wavefront (rows of at most 2 KiB) and row per workgroup, every alignment of both sides modulo 16,
+    """Row per wavefront (more than 64 rows of at most 2 KiB) and row per workgroup, every alignment of both sides modulo 16,
     sizes from one byte to a byte below, at and above a tile: only the fragments'
     bytes change."""
     rng = np.random.default_rng(n + slot)
