@@ -125,10 +125,11 @@ XferProfile Xfer::read_profile() {
   XferProfile out = prof_;
   float ms = 0.f;
   if (prof_begin_set_ && prof_end_set_ &&
-      hipEventElapsedTime(&ms, prof_begin_, prof_end_) == hipSuccess) {
+      hipEventElapsedTime(&ms, prof_begin_, end_marker()) == hipSuccess) {
     out.device_ms = ms;
+    if (prof_end_is_first_) out.device_first_ms = ms;
   }
-  if (prof_begin_set_ && prof_first_set_ &&
+  if (prof_begin_set_ && prof_first_set_ && !prof_end_is_first_ &&
       hipEventElapsedTime(&ms, prof_begin_, prof_first_) == hipSuccess) {
     out.device_first_ms = ms;
   }
@@ -679,9 +680,11 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   if (!layer_events_.empty()) {
     for (uint64_t li = 0; li < n_layers; ++li) PF_HIP(hipEventRecord(layer_events_[li], s));
   }
-  prof_mark_end(s);
+  st = slabs_.release_after(slab, s);
+  if (st != PF_OK) return st;
+  prof_mark_end(s, false);
   prof_.enqueue_ms += ms_since(t_enqueue);
-  return slabs_.release_after(slab, s);
+  return PF_OK;
 }
 
 int Xfer::run(const pf_layer_blocks* layers, uint64_t n_layers, int path, bool save,
@@ -1141,6 +1144,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     return PF_OK;
   };
 
+  bool one_launch = false;  // the call is a single zero-copy launch
   size_t ui = 0;
   while (ui < unit_refs.size()) {
     const LayerPlan& p = plans[unit_refs[ui].plan];
@@ -1166,7 +1170,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       }
       if (st != PF_OK) return st;
       ++prof_.zero_copy_launches;
-      prof_mark_first(s);
+      one_launch = ui == 0 && uj == unit_refs.size();
+      if (!one_launch) prof_mark_first(s);
       st = fire_events_through(plans[unit_refs[uj - 1].plan].src_index, s);
       if (st != PF_OK) return st;
       ui = uj;
@@ -1361,9 +1366,13 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     st = fire_events_through(n_layers - 1, s);
     if (st != PF_OK) return st;
   }
-  prof_mark_end(s);
+  if (!in_args) {
+    st = slabs_.release_after(slab, s);
+    if (st != PF_OK) return st;
+  }
+  prof_mark_end(s, one_launch);
   prof_.enqueue_ms += ms_since(t_enqueue);
-  return in_args ? PF_OK : slabs_.release_after(slab, s);
+  return PF_OK;
 }
 
 }  // namespace pf

@@ -275,11 +275,19 @@ class Xfer {
     return total;
   }
   // Three timing events bracket the device side of the calls of a profile
-  // window (begin, first slot ready, end); off unless enabled.
+  // window (begin, first slot ready, end); off unless enabled.  A marker behind a
+  // kernel is ~4.5 us on the queue, so a call of one launch gets one: its end is
+  // the first result as well, and whoever waits for the call waits for it.
   int enable_profile();
   void reset_profile() {
     prof_ = XferProfile();
     prof_begin_set_ = prof_first_set_ = prof_end_set_ = false;
+    prof_end_is_first_ = false;
+  }
+  // The event behind everything the window's calls enqueued; null when they
+  // enqueued nothing or without a profile.
+  hipEvent_t end_marker() const {
+    return !prof_end_set_ ? nullptr : prof_end_is_first_ ? prof_first_ : prof_end_;
   }
   // Call after the stream of the profiled calls has been synchronised.
   XferProfile read_profile();
@@ -376,14 +384,18 @@ class Xfer {
   bool profiling_ = false;
   hipEvent_t prof_begin_ = nullptr, prof_first_ = nullptr, prof_end_ = nullptr;
   bool prof_begin_set_ = false, prof_first_set_ = false, prof_end_set_ = false;
+  bool prof_end_is_first_ = false;  // the end was marked by prof_first_
   void prof_mark_begin(hipStream_t s) {
     if (profiling_ && !prof_begin_set_) prof_begin_set_ = hipEventRecord(prof_begin_, s) == hipSuccess;
   }
   void prof_mark_first(hipStream_t s) {
     if (profiling_ && !prof_first_set_) prof_first_set_ = hipEventRecord(prof_first_, s) == hipSuccess;
   }
-  void prof_mark_end(hipStream_t s) {
-    if (profiling_) prof_end_set_ = hipEventRecord(prof_end_, s) == hipSuccess;
+  void prof_mark_end(hipStream_t s, bool one_launch) {
+    if (!profiling_) return;
+    prof_end_is_first_ = one_launch && !prof_first_set_;
+    prof_end_set_ = hipEventRecord(prof_end_is_first_ ? prof_first_ : prof_end_, s) == hipSuccess;
+    if (prof_end_is_first_) prof_first_set_ = prof_end_set_;
   }
 };
 

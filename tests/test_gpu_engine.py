@@ -1066,6 +1066,29 @@ def test_engine_load_profile_and_staging_report(gpu):
     z.close()
 
 
+@pytest.mark.parametrize("blocks", [1, 100, 200])
+def test_device_times_of_a_task(gpu, blocks):
+    """A task of one launch has one marker behind it: its first result is its end.
+    From 8 MiB on the task is staged and the first filled slot comes before."""
+    e = PegaEngine(pool_size=64 << 20)
+    layers = [Layer(f"layer_{i}", 256, 16384, split_kv_stride=256 * 16384) for i in range(3)]
+    register(e, "markers", layers)
+    hashes = make_block_hashes(blocks, 6)
+    ids = list(range(20, 20 + blocks))
+    for _ in range(3):  # staged and unstaged tasks share the worker's events
+        for n in (blocks, 1):
+            e.batch_save_kv_blocks("markers", 0, 0, 0, [LayerSave(l.name, ids[:n], hashes[:n]) for l in layers])
+            _hits, lease = e.query_prefix("markers", hashes[:n])
+            res = e.batch_load_kv_blocks_multi_layer("markers", 0, 0, [[l.name for l in layers]], lease,
+                                                     [ids[:n]]).wait()
+            first, whole = res.phases_ms["device_first"], res.phases_ms["device"]
+            staged = n * 3 * 2 * 16384 >= 8 << 20
+            assert res.paths == (("staged",) if staged else ("zerocopy",))
+            assert 0 < first < whole if staged else 0 < first == whole
+            assert whole < res.elapsed_ms
+    e.close()
+
+
 @pytest.mark.parametrize("seg,turns,n_layers,paths", [
     (4096, (3, 1, 2), 2, ("zerocopy",)),                 # small: per-block bases of K and V
     (1000, (5, 1, 9), 3, ("zerocopy",)),                 # off 16-byte boundaries, pool padding
