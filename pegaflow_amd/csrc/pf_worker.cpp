@@ -15,12 +15,16 @@ namespace {
 // The workers move KV beside a running model: a task whose dense layers add up
 // to this much is staged whatever the size of its layers (see run()).
 constexpr uint64_t kWorkerStagedCallBytes = 8ull << 20;
-// Layers whose blocks come from several saves are staged piece by piece when
-// the pieces lie in host memory in runs of this length on average: every run
-// is a link copy of its own, which costs ~22 us beyond its bytes behind a
-// kernel on the same stream (8 MiB: 146 us at link rate, so 50 of 57 GB/s).
-// Shorter runs cross with the zero-copy kernel, which does not care.
-constexpr uint64_t kStagedPieceRunBytes = 8ull << 20;
+// K/V layers whose blocks come from several saves are staged piece by piece when
+// the pieces lie in host memory in runs of this length on average; every run is a
+// link copy of its own, which costs ~22 us beyond its bytes.  Shorter runs cross
+// with the zero-copy kernel, which does not depend on them but keeps its compute
+// units from the kernels beside it.  Measured on MI355X, us per load and, from a
+// stream of 2048^3 GEMMs beside a loop of them, GEMM time lost per load, staged
+// against zero-copy: 33 MB in runs of 4 MiB 860 and 43 against 727 and 502, 69 MB
+// in runs of 1.75 MiB 1779 and 83 against 1341 and 1007, of 1.09 MiB 2055 and 91
+// against 1353 and 1020.  The sum of both turns at runs of about 1 MiB.
+constexpr uint64_t kStagedPieceRunBytes = 1ull << 20;
 }  // namespace
 
 bool build_copy_descs(const std::vector<LayerTransferData>& layers, std::vector<CopyDesc>* out,
@@ -142,8 +146,9 @@ struct BlockForm {
   uint64_t total_bytes = 0;
 };
 
-// A maximal run of list positions whose segments follow one another in host
-// memory without a gap.
+// A maximal run of list positions of a K/V layer whose segments follow one another
+// in host memory without a gap.  (Blocks of one segment from several saves cross
+// with the zero-copy kernel.)
 struct Piece {
   size_t layer;  // index in the form
   size_t first, count;
@@ -159,9 +164,8 @@ void stage_in_pieces(BlockForm* form, std::vector<Piece>* pieces, uint64_t stage
   std::vector<std::pair<const uint8_t*, uint64_t>> spans;
   spans.reserve(pieces->size() * 2);
   for (const Piece& p : *pieces) {
-    const pf_kv_layout& layout = form->layers[p.layer].layout;
-    for (uint32_t s = 0; s < (layout.split ? 2u : 1u); ++s) {
-      const uint64_t len = p.count * layout.segment_bytes;
+    const uint64_t len = p.count * form->layers[p.layer].layout.segment_bytes;
+    for (uint32_t s = 0; s < 2; ++s) {
       spans.emplace_back(p.seg[s].host, len);
       bytes += len;
     }
@@ -185,7 +189,7 @@ void stage_in_pieces(BlockForm* form, std::vector<Piece>* pieces, uint64_t stage
     lb.block_ids += p.first;
     lb.n_blocks = p.count;
     lb.page_host = lb.page_host_device = nullptr;
-    for (uint32_t s = 0; s < (lb.layout.split ? 2u : 1u); ++s) {
+    for (uint32_t s = 0; s < 2; ++s) {
       lb.host[s] = p.seg[s].host;
       lb.host_device[s] = reinterpret_cast<uint64_t>(p.seg[s].device);
       lb.host_len[s] = p.count * frag;
