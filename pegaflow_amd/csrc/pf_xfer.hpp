@@ -367,11 +367,12 @@ class Xfer {
   // many short fills under way the runtime deals their copies to whichever
   // engine is idle when they are enqueued, some of which move 12 GB/s.  Measured
   // on MI355X, calls back to back / one call then a synchronise, GB/s, side
-  // stream against in order: 32 loads of 20 MB with layer events 44.4 / 53.3
-  // against 52.4 / 51.6; fills of 41 MB with zero-copy layers between them 35.5
-  // / 54.4 against 54.2 / 53.6; 8 saves of 21 MB 39.1 / 51.3 against 52.0 /
-  // 50.9; from 64 MB fills on it is the faster one both ways (55.2 / 54.9
-  // against 54.7 / 54.4; 131 MB 56.0 / 55.8 against 55.4 / 55.2).
+  // stream against in order: 32 loads of 20 MB with layer events 44.0 / 53.2
+  // against 53.4 / 52.9; fills of 41 MB with zero-copy layers between them 31.5
+  // / 54.5 against 54.5 / 53.9; 8 saves of 21 MB 33.7 / 51.7 against 52.4 /
+  // 51.8; 6 loads of 64 MB 55.4 / 55.2 against 55.2 / 54.9; 4 of 131 MB 56.0 /
+  // 55.9 against 55.6 / 55.5.  So calls of smaller fills go in order: alone they
+  // give up at most 1 % by it, back to back they gain a fifth and more.
   bool use_side_stream(size_t fills, uint64_t staged_bytes) const {
     if ((timing_ && !timing_in_place_) || copy_stream_ == 2) return false;
     if (copy_stream_ == 1) return true;
