@@ -333,9 +333,11 @@ def test_page_first_pages(xfer, stream):
     pool.close()
 
 
-def test_multi_layer_batch_with_layer_events_and_empty_layer(xfer, stream):
+@pytest.mark.parametrize("copy_stream", [0, 1], ids=["default", "side_stream"])
+def test_multi_layer_batch_with_layer_events_and_empty_layer(xfer, stream, copy_stream):
     """Several layers in one call, one of them empty; per-layer events all
-    fire; mixed paths in one call."""
+    fire, the link copies on the caller's stream or on one of their own; mixed
+    paths in one call."""
     rng = np.random.default_rng(13)
     cases = [Case(rng, num_blocks=64, seg=32768, segments=2, n_ids=40),
              Case(rng, num_blocks=64, seg=4096, segments=2, n_ids=1),
@@ -352,7 +354,8 @@ def test_multi_layer_batch_with_layer_events_and_empty_layer(xfer, stream):
         c.dev.copy_from_host(c.cache0)
         layers.append(_dense_layer(c, L, h, c.ids))
     events = [Event() for _ in cases]
-    big = BlockTransfer(staging_slot_bytes=1 << 20, staging_slots=2, auto_staged_min_bytes=1 << 20)
+    big = BlockTransfer(staging_slot_bytes=1 << 20, staging_slots=2, auto_staged_min_bytes=1 << 20,
+                        copy_stream=copy_stream)
     big.set_layer_events(events)
     big.save(layers, stream, TransferPath.AUTO)
     for e in events:
@@ -541,7 +544,7 @@ def test_page_packing_is_refused_when_it_would_touch_foreign_bytes(xfer, stream)
     pool.close()
 
 
-@pytest.mark.parametrize("copy_stream", [0, 2], ids=["side_stream", "in_order"])
+@pytest.mark.parametrize("copy_stream", [0, 1, 2], ids=["default", "side_stream", "in_order"])
 def test_small_staged_layers_share_slots_and_launches(stream, copy_stream):
     """Staged layers that are small share a staging slot and one gather /
     scatter launch per group.  Nine layers of unlike shapes in one call -
@@ -642,7 +645,7 @@ def test_small_staged_layers_share_slots_and_launches(stream, copy_stream):
 
 
 @pytest.mark.parametrize("kind", ["mixed", "contiguous"])
-@pytest.mark.parametrize("copy_stream", [0, 2], ids=["side_stream", "in_order"])
+@pytest.mark.parametrize("copy_stream", [0, 1, 2], ids=["default", "side_stream", "in_order"])
 def test_layers_split_across_staging_slot_fills(stream, copy_stream, kind):
     """Without per-layer events a staging slot is filled to the brim: whole
     layers while they fit, then the head of the next layer, whose tail opens
@@ -675,7 +678,7 @@ def test_layers_split_across_staging_slot_fills(stream, copy_stream, kind):
         layers.append(_dense_layer(c, L, h, c.ids))
     xfer = BlockTransfer(staging_slot_bytes=64 << 20, staging_slots=2, auto_staged_min_bytes=1,
                          copy_stream=copy_stream)
-    xfer.set_kernel_timing(1)
+    xfer.set_kernel_timing(2)  # in place: the link copies stay where copy_stream puts them
     xfer.save(layers, stream, TransferPath.STAGED)
     stream.synchronize()
     assert xfer.last_path == ST
