@@ -91,7 +91,6 @@ class RawBlock {
   explicit RawBlock(std::vector<Segment> segments) {
     n_ = segments.size();
     for (size_t i = 0; i < segments.size(); ++i) {
-      total_size_ += segments[i].size();
       if (i < 2) {
         inline_[i] = std::move(segments[i]);
       } else {
@@ -102,14 +101,12 @@ class RawBlock {
   static RawBlock single_segment(Segment s) {
     RawBlock b;
     b.n_ = 1;
-    b.total_size_ = s.size();
     b.inline_[0] = std::move(s);
     return b;
   }
   static RawBlock two_segments(Segment k, Segment v) {
     RawBlock b;
     b.n_ = 2;
-    b.total_size_ = k.size() + v.size();
     b.inline_[0] = std::move(k);
     b.inline_[1] = std::move(v);
     return b;
@@ -122,14 +119,12 @@ class RawBlock {
   }
   uint64_t segment_allocation_id(size_t i) const { return i < n_ ? at(i).allocation_id() : 0; }
   uint64_t segment_size(size_t i) const { return i < n_ ? at(i).size() : 0; }
-  uint64_t memory_footprint() const { return total_size_; }
 
  private:
   const Segment& at(size_t i) const { return i < 2 ? inline_[i] : extra_[i - 2]; }
   Segment inline_[2];
   std::vector<Segment> extra_;
   size_t n_ = 0;
-  uint64_t total_size_ = 0;
 };
 
 // The host side of one slot of a block, by value: what a transfer needs of it

@@ -27,7 +27,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // instead of flat accesses for addresses that arrive as integers.
 typedef __attribute__((address_space(1))) u32x4 g_u32x4;
 typedef __attribute__((address_space(1))) unsigned char g_u8;
-typedef __attribute__((address_space(1))) unsigned short g_u16;
 // 16 bytes at any address: the target allows unaligned global accesses, so
 // these are one global_load_dwordx4 / global_store_dwordx4 all the same.
 typedef u32x4 u32x4_any __attribute__((aligned(1)));

@@ -768,8 +768,9 @@ void GpuWorkerPool::run(Worker* w, bool is_load, NumaNode numa, std::promise<Tas
     init.message = "Failed to initialise GPU worker on device " + std::to_string(device_id_) +
                    ": " + last_error();
   } else {
-    backend = build_backend(mode_);
-    if (!options_.use_descriptor_backends) {
+    if (options_.use_descriptor_backends) {
+      backend = build_backend(mode_);
+    } else {
       // The pool always has a second engine (load next to save), so each
       // worker keeps to one stream: with a side stream per engine the link
       // copies of the two directions were seen on one hardware queue (a
