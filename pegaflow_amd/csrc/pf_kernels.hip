@@ -172,7 +172,7 @@ __device__ __forceinline__ void store16_any(uint64_t addr, u32x4 v) {
 // Copy `bytes` <= U*LANES*16 with no alignment assumption, by the LANES lanes
 // whose index is `lane`; chunks are aligned on the destination or, with
 // ALIGN_SRC, on the source.
-template <int U, int LANES, bool ALIGN_SRC>
+template <int U, int LANES, bool ALIGN_SRC, bool IN_HBM = false>
 __device__ __forceinline__ void copy_tile_any(uint64_t dst, uint64_t src, uint32_t bytes,
                                               uint32_t lane) {
   if (bytes < 16) {
@@ -188,7 +188,11 @@ __device__ __forceinline__ void copy_tile_any(uint64_t dst, uint64_t src, uint32
   if (n <= LANES && n <= 2 * kWave) {
     if (lane < n) {
       const uint32_t at = chunk_start(lane, bytes, mis);
-      store16_any(dst + at, load16_any(src + at));
+      if constexpr (IN_HBM) {
+        *reinterpret_cast<g_u32x4_any*>(dst + at) = *reinterpret_cast<const g_u32x4_any*>(src + at);
+      } else {
+        store16_any(dst + at, load16_any(src + at));
+      }
     }
     return;
   }
@@ -245,7 +249,9 @@ __device__ __forceinline__ void copy_tile_in_hbm(uint64_t dst, uint64_t src, uin
 // Rows of a descriptor table, wave-uniform.  Rows3: [dst, src, size] as the
 // backends write it; Rows48: the caller's pf_copy_desc array as it is, so the
 // host side repacks nothing.
+template <bool IN_HBM>
 struct Rows3 {
+  static constexpr bool kInHbm = IN_HBM;  // both sides in device memory (packing)
   const uint64_t* table;
   __device__ __forceinline__ void get(uint32_t i, uint64_t* dst, uint64_t* src,
                                       uint64_t* size) const {
@@ -257,6 +263,7 @@ struct Rows3 {
 };
 template <bool HOST_IS_SRC>
 struct Rows48 {
+  static constexpr bool kInHbm = false;
   const pf_copy_desc* table;
   __device__ __forceinline__ void get(uint32_t i, uint64_t* dst, uint64_t* src,
                                       uint64_t* size) const {
@@ -293,7 +300,7 @@ __device__ __forceinline__ void copy_rows(const Rows rows, uint32_t n, uint32_t 
       if (vec) {
         copy_tile_vec<U, LANES>(dst + off, src + off, bytes, lane);
       } else {
-        copy_tile_any<U, LANES, ALIGN_SRC>(dst + off, src + off, bytes, lane);
+        copy_tile_any<U, LANES, ALIGN_SRC, Rows::kInHbm>(dst + off, src + off, bytes, lane);
       }
     }
     if (!more) break;
@@ -1097,12 +1104,18 @@ void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
 }  // namespace
 
 int launch_desc_copy(const uint64_t* table, uint64_t n, uint64_t max_size, bool host_is_src,
-                     hipStream_t s, uint32_t max_workgroups) {
+                     bool packing, hipStream_t s, uint32_t max_workgroups) {
   if (n == 0) return PF_OK;
-  if (host_is_src) {
-    launch_rows<true>(Rows3{table}, n, max_size, s, max_workgroups);
+  if (packing) {
+    if (host_is_src) {
+      launch_rows<true>(Rows3<true>{table}, n, max_size, s, max_workgroups);
+    } else {
+      launch_rows<false>(Rows3<true>{table}, n, max_size, s, max_workgroups);
+    }
+  } else if (host_is_src) {
+    launch_rows<true>(Rows3<false>{table}, n, max_size, s, max_workgroups);
   } else {
-    launch_rows<false>(Rows3{table}, n, max_size, s, max_workgroups);
+    launch_rows<false>(Rows3<false>{table}, n, max_size, s, max_workgroups);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "desc_copy_kernel launch");

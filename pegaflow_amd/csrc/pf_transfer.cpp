@@ -432,7 +432,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
   }
   row = 0;
   if (isolated_by_kernel) {
-    st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, s,
+    st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, false, s,
                           host_link_workgroups(isolated_bytes, isolated.size()));
     if (st != PF_OK) return st;
     row = isolated.size();
@@ -453,7 +453,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     const uint64_t pieces = run.members.size();
     const uint32_t pack_workgroups =
         max_staged_piece <= 16384 && pieces >= 8192 ? static_cast<uint32_t>((pieces + 1) / 2) : 0;
-    st = launch_desc_copy(table_dev + 3 * row, pieces, max_staged_piece, host_is_src, s,
+    st = launch_desc_copy(table_dev + 3 * row, pieces, max_staged_piece, host_is_src, true, s,
                           pack_workgroups);
     if (st != PF_OK) return st;
     if (!host_is_src) {
@@ -517,7 +517,8 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
   } else {
     PF_HIP(hipMemcpyAsync(slab->dev, slab->host, bytes, hipMemcpyHostToDevice, s));
   }
-  st = launch_desc_copy(table_dev, n, max_size, host_is_src, s, host_link_workgroups(total_size, n));
+  st = launch_desc_copy(table_dev, n, max_size, host_is_src, false, s,
+                        host_link_workgroups(total_size, n));
   if (st != PF_OK) return st;
   return slabs_.release_after(slab, s);
 }
