@@ -7,7 +7,8 @@
 //     loads before the first store so U global_load_dwordx4 are in flight per
 //     lane, and consecutive lanes touch consecutive 16-byte words, so each
 //     wavefront's access is one 1 KiB contiguous burst;
-//   * loads are non-temporal and stores "sc1 nt": the data is touched once;
+//   * loads are non-temporal and stores "sc1 nt": the data is touched once (but see
+//     copy_tile_in_hbm);
 //   * all per-tile address arithmetic is wave-uniform (scalar registers), except
 //     for units cut into chunks (block_chunks_unit).
 #include "pf_kernels.hpp"
