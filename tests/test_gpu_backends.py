@@ -144,6 +144,33 @@ def test_rows_of_any_size_and_alignment(backends, stream, n, slot, direction):
     host.close()
 
 
+@pytest.mark.parametrize("size", [24, 600, 1500])
+def test_short_rows_packed_again_and_again(backends, stream, size):
+    """Host-dense rows off the 16-byte grid, packed through the same staging buffer
+    piece after piece and batch after batch, other bytes each time."""
+    rng = np.random.default_rng(size)
+    n = 40001
+    host, dev = PinnedMemory(n * size), DeviceBuffer(n * size)
+    for b in backends:
+        for _ in range(2):
+            data, order = random_bytes(rng, n * size), rng.permutation(n)
+            descs = [CopyDesc(dev.ptr + int(o) * size, host.host_ptr + i * size, host.device_ptr + i * size, size)
+                     for i, o in enumerate(order)]
+            dev.copy_from_host(data)
+            host.as_numpy()[:] = 0
+            b.d2h(descs, stream)
+            stream.synchronize()
+            assert np.array_equal(host.as_numpy().reshape(n, size), data.reshape(n, size)[order]), b.name
+            data = random_bytes(rng, n * size)
+            host.as_numpy()[:] = data
+            dev.fill(0)
+            b.h2d(descs, stream)
+            stream.synchronize()
+            assert np.array_equal(dev.copy_to_host().reshape(n, size)[order], data.reshape(n, size)), b.name
+    dev.close()
+    host.close()
+
+
 @pytest.mark.parametrize("n", [4096, 16385, 40001])
 def test_shuffled_4k_fragments(backends, stream, n):
     """Shape of the reference's transfer bench (benches/transfer_h2d.rs):

@@ -987,18 +987,21 @@ def test_call_size_rule_stages_small_layers_of_a_long_call(stream):
     xfer.close()
 
 
+@pytest.mark.parametrize("seg", [32768, 20004, 1001])
 @pytest.mark.parametrize("copy_stream", [1, 2], ids=["side_stream", "in_order"])
-def test_staging_slots_are_handed_on_between_calls_and_streams(gpu, copy_stream):
+def test_staging_slots_are_handed_on_between_calls_and_streams(gpu, copy_stream, seg):
     """Many fills per call through two small slots, calls on two streams in turn
     with no synchronise between them: a call's first fills wait for the slots of
-    the call before, whichever stream that ran on."""
-    rng = np.random.default_rng(copy_stream)
+    the call before, whichever stream that ran on.  Fragments off the 16-byte grid
+    are packed with cached accesses: no fill sees the bytes of the one before."""
+    rng = np.random.default_rng(copy_stream + seg)
     xfer = BlockTransfer(staging_slot_bytes=256 << 10, copy_stream=copy_stream)
     streams = [Stream(), Stream()]
-    cases = [Case(rng, num_blocks=96, seg=32768, segments=2) for _ in streams]
+    num_blocks = 96 * 32768 // seg
+    cases = [Case(rng, num_blocks=num_blocks, seg=seg, segments=2) for _ in streams]
     layouts = [c.product_layout() for c in cases]
-    hosts = [PinnedMemory(2 * len(c.ids) * 32768) for c in cases]
-    dests = [rng.choice(96, len(c.ids), replace=False).astype(np.uint32) for c in cases]
+    hosts = [PinnedMemory(2 * len(c.ids) * seg) for c in cases]
+    dests = [rng.choice(num_blocks, len(c.ids), replace=False).astype(np.uint32) for c in cases]
     for c, h in zip(cases, hosts):
         c.dev.copy_from_host(c.cache0)
         h.as_numpy()[:] = SENT
@@ -1015,8 +1018,8 @@ def test_staging_slots_are_handed_on_between_calls_and_streams(gpu, copy_stream)
     for s in streams:
         s.synchronize()
     for c, host, dest in zip(cases, hosts, dests):
-        src = c.cache0.reshape(2, 96, 32768)
-        assert np.array_equal(host.as_numpy().reshape(2, -1, 32768), src[:, c.ids])
+        src = c.cache0.reshape(2, num_blocks, seg)
+        assert np.array_equal(host.as_numpy().reshape(2, -1, seg), src[:, c.ids])
         expect = np.full_like(src, SENT)
         expect[:, dest] = src[:, c.ids]
         assert np.array_equal(c.dev.copy_to_host().reshape(src.shape), expect)
