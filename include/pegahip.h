@@ -318,9 +318,10 @@ typedef struct pf_layer_blocks {
 } pf_layer_blocks;
 
 /* How bytes cross the host link. */
-#define PF_PATH_AUTO 0     /* pick per shape */
+#define PF_PATH_AUTO 0     /* pick per shape; the launches of staged layers also move a share of
+                              ~2 % of the bytes over the link themselves (host_device) */
 #define PF_PATH_ZEROCOPY 1 /* kernel reads/writes mapped host memory */
-#define PF_PATH_STAGED 2   /* device gather/scatter + one DMA copy per unit */
+#define PF_PATH_STAGED 2   /* device gather/scatter + one DMA copy per unit, every byte */
 
 typedef struct pf_xfer_config {
   uint64_t staging_slot_bytes; /* 0 = default */

@@ -381,8 +381,9 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
 // us, in turn in 464.
 struct RowTurn {
   uint32_t at = 0;  // workgroup whose turn it is
-  __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t grid_x, uint32_t most_odd) {
-    const uint32_t first = blockIdx.x >= at ? blockIdx.x - at : blockIdx.x + grid_x - at;
+  __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t wg, uint32_t grid_x,
+                                           uint32_t most_odd) {
+    const uint32_t first = wg >= at ? wg - at : wg + grid_x - at;
     const uint32_t odd = n_tiles < grid_x ? n_tiles : n_tiles % grid_x;
     if (odd <= most_odd) {
       at += odd;
@@ -413,7 +414,7 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
   const uint32_t n_chunks = f.n_blocks * chunks_per_frag;
   const uint32_t tiles_per_seg = (n_chunks + U * kLanes - 1) / (U * kLanes);
   const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-  for (uint32_t t = turn.take(n_tiles, grid_x, grid_x / 4); t < n_tiles; t += grid_x) {
+  for (uint32_t t = turn.take(n_tiles, blockIdx.x, grid_x, grid_x / 4); t < n_tiles; t += grid_x) {
     const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
     const uint32_t first = (seg ? t - tiles_per_seg : t) * (U * kLanes) + threadIdx.x;
     const uint64_t near_seg = f.near_base + (seg ? f.kv_stride : 0);
@@ -481,6 +482,49 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
   }
 }
 
+// The tiles of a unit over mapped host memory, by workgroup `wg` of the `grid_x` of
+// its row.  VEC_ONLY: the unit is known to be of the form kUnitVec, with one range
+// of host memory per segment and 32-bit ids.
+template <int U, int LANES, bool TO_FAR, bool VEC_ONLY>
+__device__ __forceinline__ void unit_tiles(const UnitFields& f, RowTurn& turn, uint32_t wg,
+                                           uint32_t grid_x) {
+  constexpr uint64_t kTile = static_cast<uint64_t>(U) * LANES * 16;
+  const bool vec_ok = VEC_ONLY || f.form == kUnitVec;
+  const bool ids16 = !VEC_ONLY && f.ids16;
+  // The host keeps a unit's tile count below 2^32, so 32-bit scalar division.
+  const uint32_t tiles_per_seg = f.n_blocks * f.tiles_per_frag;
+  const uint32_t n_tiles = tiles_per_seg * f.n_seg;
+  for (uint32_t t = turn.take(n_tiles, wg, grid_x, grid_x); t < n_tiles; t += grid_x) {
+    const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
+    const uint32_t r = seg ? t - tiles_per_seg : t;
+    // The quotient is wave-uniform; pin it to a scalar register so the id and
+    // page-table reads below are scalar loads.
+    const uint32_t pos = __builtin_amdgcn_readfirstlane(r / f.tiles_per_frag);
+    const uint32_t c = r - pos * f.tiles_per_frag;
+    const uint64_t off = static_cast<uint64_t>(c) * kTile;
+    const uint64_t left = f.frag_bytes - off;
+    const uint32_t bytes = left < kTile ? static_cast<uint32_t>(left) : static_cast<uint32_t>(kTile);
+    // 16-bit ids sit two to a word (there is no scalar load of half a word).
+    const uint32_t id_word = f.ids[ids16 ? pos >> 1 : pos];
+    const uint64_t id = ids16 ? ((pos & 1u) ? id_word >> 16 : id_word & 0xFFFFu) : id_word;
+    const uint64_t near_addr = f.near_base + id * f.block_stride + (seg ? f.kv_stride : 0) + off;
+    uint64_t far_addr;
+    if (!VEC_ONLY && f.paged) {
+      far_addr = f.far_table[pos + (seg ? f.seg1_entries : 0)] + f.far_table_off +
+                 (seg ? f.seg1_bytes : 0) + off;
+    } else {
+      far_addr = (seg ? f.far_base1 : f.far_base0) + static_cast<uint64_t>(pos) * f.far_stride + off;
+    }
+    const uint64_t dst = TO_FAR ? far_addr : near_addr;
+    const uint64_t src = TO_FAR ? near_addr : far_addr;
+    if (vec_ok) {
+      copy_tile_vec<U, LANES>(dst, src, bytes, threadIdx.x);
+    } else {
+      copy_tile_any<U, LANES, !TO_FAR>(dst, src, bytes, threadIdx.x);
+    }
+  }
+}
+
 // Block-ID gather / scatter over mapped host memory (the zero-copy form).  The
 // grid is a few rows of workgroups, as many workgroups in all as the launch
 // may keep on the device.  Row y walks the units y, y + rows, ... one after the
@@ -497,7 +541,6 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
 template <int U, bool TO_FAR, typename UnitPtr>
 __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units, uint32_t grid_x,
                                                  uint32_t grid_y, uint64_t bias) {
-  constexpr uint64_t kTile = static_cast<uint64_t>(U) * kLanes * 16;
   RowTurn turn;
   for (uint32_t unit = blockIdx.y; unit < n_units; unit += grid_y) {
     const UnitFields f = unit_fields(units + unit, bias);
@@ -505,39 +548,7 @@ __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units
       block_chunks_unit<U, TO_FAR>(f, grid_x, turn);
       continue;
     }
-    const bool vec_ok = f.form == kUnitVec;
-    // The host keeps a unit's tile count below 2^32, so 32-bit scalar division.
-    const uint32_t tiles_per_seg = f.n_blocks * f.tiles_per_frag;
-    const uint32_t n_tiles = tiles_per_seg * f.n_seg;
-    for (uint32_t t = turn.take(n_tiles, grid_x, grid_x); t < n_tiles; t += grid_x) {
-      const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
-      const uint32_t r = seg ? t - tiles_per_seg : t;
-      // The quotient is wave-uniform; pin it to a scalar register so the id and
-      // page-table reads below are scalar loads.
-      const uint32_t pos = __builtin_amdgcn_readfirstlane(r / f.tiles_per_frag);
-      const uint32_t c = r - pos * f.tiles_per_frag;
-      const uint64_t off = static_cast<uint64_t>(c) * kTile;
-      const uint64_t left = f.frag_bytes - off;
-      const uint32_t bytes = left < kTile ? static_cast<uint32_t>(left) : static_cast<uint32_t>(kTile);
-      // 16-bit ids sit two to a word (there is no scalar load of half a word).
-      const uint32_t id_word = f.ids[f.ids16 ? pos >> 1 : pos];
-      const uint64_t id = f.ids16 ? ((pos & 1u) ? id_word >> 16 : id_word & 0xFFFFu) : id_word;
-      const uint64_t near_addr = f.near_base + id * f.block_stride + (seg ? f.kv_stride : 0) + off;
-      uint64_t far_addr;
-      if (f.paged) {
-        far_addr = f.far_table[pos + (seg ? f.seg1_entries : 0)] + f.far_table_off +
-                   (seg ? f.seg1_bytes : 0) + off;
-      } else {
-        far_addr = (seg ? f.far_base1 : f.far_base0) + static_cast<uint64_t>(pos) * f.far_stride + off;
-      }
-      const uint64_t dst = TO_FAR ? far_addr : near_addr;
-      const uint64_t src = TO_FAR ? near_addr : far_addr;
-      if (vec_ok) {
-        copy_tile_vec<U, kLanes>(dst, src, bytes, threadIdx.x);
-      } else {
-        copy_tile_any<U, kLanes, !TO_FAR>(dst, src, bytes, threadIdx.x);
-      }
-    }
+    unit_tiles<U, kLanes, TO_FAR, false>(f, turn, blockIdx.x, grid_x);
   }
 }
 
@@ -593,7 +604,8 @@ __device__ __forceinline__ void block_tiles_copy(UnitPtr up, uint32_t row, uint3
   }
   const uint64_t frag_bytes = up->frag_bytes;
   const uint64_t off = static_cast<uint64_t>(blockIdx.x) * kTile;
-  if (seg >= up->n_seg || pos >= up->n_blocks || off >= frag_bytes) return;
+  // (Fragments of a segment that the unit does not have lie behind all it has.)
+  if (pos >= up->n_blocks || seg * up->n_blocks + pos >= up->staged_frags || off >= frag_bytes) return;
   c_u32* ids = reinterpret_cast<c_u32*>(reinterpret_cast<uint64_t>(up->ids));
   const uint64_t id = ids[pos];
   const uint64_t near_addr =
@@ -623,18 +635,37 @@ __device__ __forceinline__ void block_tiles_copy(UnitPtr up, uint32_t row, uint3
   }
 }
 
+// The launch's share of the link: the workgroups of the first `planes` planes of the
+// grid (the first to be dispatched) move it while all others go through HBM.
+// True for a workgroup of these planes.
+template <int LT, bool TO_FAR>
+__device__ __forceinline__ bool link_share(const LinkShare& share, uint32_t planes, bool planes_are_z) {
+  if ((planes_are_z ? blockIdx.z : blockIdx.y) >= planes) return false;
+  const uint32_t wg = blockIdx.x + gridDim.x * (planes_are_z ? blockIdx.y + gridDim.y * blockIdx.z
+                                                             : blockIdx.y);
+  if (wg >= share.workgroups || (!planes_are_z && blockIdx.z != 0)) return true;
+  constexpr int kUnroll = kShareTileBytes / (LT * 16);
+  RowTurn turn;
+  for (uint32_t k = 0; k < share.n_units; ++k) {
+    unit_tiles<kUnroll, LT, TO_FAR, true>(unit_fields(share.units + k, 0), turn, wg, share.workgroups);
+  }
+  return true;
+}
+
 template <int LT, bool TO_FAR, int SEGS, bool UNITS_INNER, typename UnitPtr>
-__device__ __forceinline__ void block_tiles_body(UnitPtr units) {
+__device__ __forceinline__ void block_tiles_body(UnitPtr units, const LinkShare& share, uint32_t planes) {
+  if (link_share<LT, TO_FAR>(share, planes, UNITS_INNER)) return;
   const uint32_t unit_seg = UNITS_INNER ? blockIdx.y : blockIdx.z;
-  const uint32_t row = UNITS_INNER ? blockIdx.z : blockIdx.y;
+  const uint32_t row = (UNITS_INNER ? blockIdx.z : blockIdx.y) - planes;
   UnitPtr up = units + (SEGS == 2 ? unit_seg >> 1 : unit_seg);
   const uint32_t seg = SEGS == 2 ? (unit_seg & 1u) : 0u;
   block_tiles_copy<LT, TO_FAR, UnitPtr>(up, row, seg);
 }
 
 template <int LT, bool TO_FAR, int SEGS, bool UNITS_INNER>
-__global__ __launch_bounds__(LT) void block_tiles_kernel(const BlockUnit* __restrict__ units) {
-  block_tiles_body<LT, TO_FAR, SEGS, UNITS_INNER, const BlockUnit*>(units);
+__global__ __launch_bounds__(LT) void block_tiles_kernel(const BlockUnit* __restrict__ units,
+                                                         LinkShare share, uint32_t planes) {
+  block_tiles_body<LT, TO_FAR, SEGS, UNITS_INNER, const BlockUnit*>(units, share, planes);
 }
 
 // A few units of different lengths in one launch (the fills of a staging slot:
@@ -650,11 +681,13 @@ struct RowEnds {
 
 template <int LT, bool TO_FAR, int SEGS>
 __global__ __launch_bounds__(LT) void block_tiles_rows_kernel(const BlockUnit* __restrict__ units,
-                                                              RowEnds ends) {
+                                                              RowEnds ends, LinkShare share,
+                                                              uint32_t planes) {
+  if (link_share<LT, TO_FAR>(share, planes, false)) return;
   // More rows than one grid extent are folded over grid.z: z = chunk * SEGS + segment.
   const uint32_t chunk = SEGS == 2 ? blockIdx.z >> 1 : blockIdx.z;
   const uint32_t seg = SEGS == 2 ? blockIdx.z & 1u : 0u;
-  const uint32_t row = chunk * gridDim.y + blockIdx.y;
+  const uint32_t row = chunk * (gridDim.y - planes) + blockIdx.y - planes;
   uint32_t unit = 0, first = 0;
 #pragma unroll
   for (uint32_t k = 0; k + 1 < kMaxRowUnits; ++k) {
@@ -673,10 +706,12 @@ __global__ __launch_bounds__(LT) void block_tiles_rows_kernel(const BlockUnit* _
 // every level of that chain is a measurable part of its life).  The unit is the
 // first argument: offset 0 of the argument segment.
 template <int LT, bool TO_FAR, int SEGS>
-__global__ __launch_bounds__(LT) void block_tiles_one_kernel(BlockUnit unit) {
+__global__ __launch_bounds__(LT) void block_tiles_one_kernel(BlockUnit unit, LinkShare share,
+                                                             uint32_t planes) {
   (void)unit;
   block_tiles_body<LT, TO_FAR, SEGS, false, c_unit*>(
-      reinterpret_cast<c_unit*>(reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr())));
+      reinterpret_cast<c_unit*>(reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr())),
+      share, planes);
 }
 
 // The two halves of streams_run_concurrently().  The wait is bounded by the
@@ -817,29 +852,41 @@ int launch_block_units_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n
   return PF_OK;
 }
 
-int launch_block_tiles_one(const BlockUnit& unit, bool to_far, hipStream_t s) {
+namespace {
+// Planes of a grid, `per_plane` workgroups each, that hold a share's workgroups.
+uint32_t share_planes(const LinkShare& share, uint64_t per_plane) {
+  return static_cast<uint32_t>((share.workgroups + per_plane - 1) / per_plane);
+}
+}  // namespace
+
+int launch_block_tiles_one(const BlockUnit& unit, bool to_far, hipStream_t s, const LinkShare& share) {
   if (unit.n_blocks == 0 || unit.frag_bytes == 0) return PF_OK;
   if (unit.n_seg != 1 && unit.n_seg != 2) {
     return fail(PF_ERR_INVALID_ARGUMENT, "tile launch: %u segments per block", unit.n_seg);
   }
   constexpr uint64_t kTile = kTileLanes * 16;
   const uint64_t gx = (unit.frag_bytes + kTile - 1) / kTile;
-  if (unit.n_blocks > kMaxTileBlocks || gx > 0x7FFFFFFFull) {
+  const uint32_t planes = share_planes(share, gx);
+  if (unit.n_blocks > kMaxTileBlocks - planes || gx > 0x7FFFFFFFull) {
     return fail(PF_ERR_INVALID_ARGUMENT, "tile launch out of range: %u blocks, %llu-byte fragments",
                 unit.n_blocks, static_cast<unsigned long long>(unit.frag_bytes));
   }
-  dim3 grid(static_cast<uint32_t>(gx), unit.n_blocks, unit.n_seg);
+  dim3 grid(static_cast<uint32_t>(gx), unit.n_blocks + planes, unit.n_seg);
   dim3 block(kTileLanes, 1, 1);
   if (unit.n_seg == 2) {
     if (to_far) {
-      hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, true, 2>), grid, block, 0, s, unit);
+      hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, true, 2>), grid, block, 0, s, unit, share,
+                         planes);
     } else {
-      hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, false, 2>), grid, block, 0, s, unit);
+      hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, false, 2>), grid, block, 0, s, unit, share,
+                         planes);
     }
   } else if (to_far) {
-    hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, true, 1>), grid, block, 0, s, unit);
+    hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, true, 1>), grid, block, 0, s, unit, share,
+                         planes);
   } else {
-    hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, false, 1>), grid, block, 0, s, unit);
+    hipLaunchKernelGGL((block_tiles_one_kernel<kTileLanes, false, 1>), grid, block, 0, s, unit, share,
+                         planes);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "block_tiles_one_kernel launch");
@@ -847,7 +894,7 @@ int launch_block_tiles_one(const BlockUnit& unit, bool to_far, hipStream_t s) {
 }
 
 int launch_block_tiles_rows(const BlockUnit* units, const BlockUnit* host_units, uint32_t n_units,
-                            bool to_far, hipStream_t s, bool* launched) {
+                            bool to_far, hipStream_t s, bool* launched, const LinkShare& share) {
   *launched = false;
   if (n_units == 0 || n_units > kMaxRowUnits) return PF_OK;
   RowEnds ends;
@@ -872,8 +919,10 @@ int launch_block_tiles_rows(const BlockUnit* units, const BlockUnit* host_units,
     return PF_OK;
   }
   // Rows beyond one grid extent go into further chunks of equal length along grid.z.
-  const uint64_t chunks = (rows + kMaxTileBlocks - 1) / kMaxTileBlocks;
-  const uint64_t gy = (rows + chunks - 1) / chunks;
+  const uint32_t planes = share_planes(share, gx);
+  const uint64_t chunk_rows = kMaxTileBlocks - planes;
+  const uint64_t chunks = (rows + chunk_rows - 1) / chunk_rows;
+  const uint64_t gy = (rows + chunks - 1) / chunks + planes;
   if (chunks * max_seg > kMaxTileBlocks || rows >= 0xFFFFFFFFull || gx > 0x7FFFFFFFull) {
     return PF_OK;  // the caller takes another form
   }
@@ -882,14 +931,18 @@ int launch_block_tiles_rows(const BlockUnit* units, const BlockUnit* host_units,
   dim3 block(kTileLanes, 1, 1);
   if (max_seg == 2) {
     if (to_far) {
-      hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, true, 2>), grid, block, 0, s, units, ends);
+      hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, true, 2>), grid, block, 0, s, units, ends,
+                         share, planes);
     } else {
-      hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, false, 2>), grid, block, 0, s, units, ends);
+      hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, false, 2>), grid, block, 0, s, units, ends,
+                         share, planes);
     }
   } else if (to_far) {
-    hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, true, 1>), grid, block, 0, s, units, ends);
+    hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, true, 1>), grid, block, 0, s, units, ends,
+                         share, planes);
   } else {
-    hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, false, 1>), grid, block, 0, s, units, ends);
+    hipLaunchKernelGGL((block_tiles_rows_kernel<kTileLanes, false, 1>), grid, block, 0, s, units, ends,
+                         share, planes);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "block_tiles_rows_kernel launch");
@@ -898,7 +951,8 @@ int launch_block_tiles_rows(const BlockUnit* units, const BlockUnit* host_units,
 }
 
 int launch_block_tiles(const BlockUnit* units, uint32_t n_units, uint32_t max_blocks,
-                       uint64_t max_frag_bytes, uint32_t max_seg, bool to_far, hipStream_t s) {
+                       uint64_t max_frag_bytes, uint32_t max_seg, bool to_far, hipStream_t s,
+                       const LinkShare& share) {
   if (n_units == 0 || max_blocks == 0 || max_frag_bytes == 0) return PF_OK;
   if (max_seg != 1 && max_seg != 2) {
     return fail(PF_ERR_INVALID_ARGUMENT, "tile launch: %u segments per block", max_seg);
@@ -924,12 +978,17 @@ int launch_block_tiles(const BlockUnit* units, uint32_t n_units, uint32_t max_bl
   constexpr uint32_t kUnitsInnerFrom = 9;
   const bool units_inner = n_units >= kUnitsInnerFrom;
   const uint32_t unit_segs = max_seg * n_units;
-  dim3 grid(static_cast<uint32_t>(gx), units_inner ? unit_segs : max_blocks,
-            units_inner ? max_blocks : unit_segs);
+  const uint32_t planes = share_planes(share, units_inner ? gx * unit_segs : gx);
+  if (max_blocks > kMaxTileBlocks - planes) {
+    return fail(PF_ERR_INVALID_ARGUMENT, "tile launch out of range: %u blocks and a share of the link",
+                max_blocks);
+  }
+  dim3 grid(static_cast<uint32_t>(gx), units_inner ? unit_segs : max_blocks + planes,
+            units_inner ? max_blocks + planes : unit_segs);
   dim3 block(kTileLanes, 1, 1);
 #define PF_LAUNCH_TILES(TO_FAR_, SEGS_, INNER_)                                                \
   hipLaunchKernelGGL((block_tiles_kernel<kTileLanes, TO_FAR_, SEGS_, INNER_>), grid, block, 0, s, \
-                     units)
+                     units, share, planes)
   if (units_inner) {
     if (max_seg == 2) {
       if (to_far) {

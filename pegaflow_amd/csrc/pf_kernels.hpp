@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "pf_share.hpp"
+
 namespace pf {
 
 // One unit of block-ID work, read by the kernel from device memory.
@@ -31,7 +33,11 @@ struct BlockUnit {
   uint64_t far_table_off;
   uint32_t n_blocks;
   uint32_t n_seg;             // fragments per block: 1 or 2
-  uint32_t tiles_per_frag;    // ceil(frag_bytes / tile_bytes); kUnitChunks: 16-byte chunks of one
+  union {
+    uint32_t tiles_per_frag;  // zero-copy: ceil(frag_bytes / tile_bytes); kUnitChunks: 16-byte chunks of one
+    uint32_t staged_frags;    // staged: the first so many fragments, in (segment, position) order, are
+                              // in the slot; the others are the launch's share of the link (LinkShare)
+  };
   uint32_t form;              // UnitForm
   uint32_t ids16;             // the id list holds 16-bit ids (zero-copy form only)
   uint32_t far_table_step;    // entries between a position's bases of segment 0 and 1; 0 = one base
@@ -78,6 +84,18 @@ constexpr uint32_t kRowsLaunchUnits = 8;  // units one launch_block_tiles_rows c
 constexpr uint64_t kStagedTileBytes = 2048;  // bytes one workgroup of the staged kernels moves
 constexpr uint32_t kMaxTileUnits = 32767;
 
+// What a staged launch moves over the link beside its units (pf_share.hpp):
+// `units` (device) describe the fragments, every one of the form kUnitVec with its
+// far side in mapped host memory, tiles of kShareTileBytes and 32-bit ids.
+struct LinkShare {
+  const BlockUnit* units = nullptr;
+  uint32_t n_units = 0;
+  uint32_t workgroups = 0;  // 0 = nothing to move
+};
+// Positions a unit of a launch with a share may have: the share's workgroups are
+// rows or planes of the same grid.
+constexpr uint32_t kMaxSharedTileBlocks = kMaxTileBlocks - kShareWorkgroupsMax;
+
 // Launch the one-tile-per-workgroup form over `n_units` units: the HBM-bound
 // kernel of the staged path.  Every unit needs n_blocks <= kMaxTileBlocks;
 // max_seg (1 or 2) is the largest n_seg among the units.  A unit's `order`
@@ -88,7 +106,8 @@ constexpr uint32_t kMaxTileUnits = 32767;
 // reads tolerate the shuffle (the same trick on the gather, sequential reads
 // and shuffled writes, is slower: 5.8 against 6.4).
 int launch_block_tiles(const BlockUnit* units, uint32_t n_units, uint32_t max_blocks,
-                       uint64_t max_frag_bytes, uint32_t max_seg, bool to_far, hipStream_t s);
+                       uint64_t max_frag_bytes, uint32_t max_seg, bool to_far, hipStream_t s,
+                       const LinkShare& share = {});
 
 // Up to eight units of any lengths in one launch with no idle workgroups: the
 // rows of all units laid end to end along grid.y (`host_units` is the host
@@ -96,11 +115,13 @@ int launch_block_tiles(const BlockUnit* units, uint32_t n_units, uint32_t max_bl
 // does not fit this form (more than eight units):
 // nothing was enqueued and the caller uses launch_block_tiles.
 int launch_block_tiles_rows(const BlockUnit* units, const BlockUnit* host_units, uint32_t n_units,
-                            bool to_far, hipStream_t s, bool* launched);
+                            bool to_far, hipStream_t s, bool* launched,
+                            const LinkShare& share = {});
 
 // The same for a single unit, handed over by value (its `ids` / `order` are
 // device addresses as usual).
-int launch_block_tiles_one(const BlockUnit& unit, bool to_far, hipStream_t s);
+int launch_block_tiles_one(const BlockUnit& unit, bool to_far, hipStream_t s,
+                           const LinkShare& share = {});
 
 // Plain device copy kernel of the same tile shape, for calibrating counters
 // and measuring the HBM copy ceiling: copies `bytes` (multiple of 16).

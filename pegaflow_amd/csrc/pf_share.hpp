@@ -1,0 +1,83 @@
+// Which part of a staging fill crosses the link with the gather / scatter launch
+// itself.  Arithmetic alone, for the planner and its test.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace pf {
+
+// A fill's link copy and its gather or scatter take turns on one stream, so the
+// link has nothing to do while the launch moves the fill through HBM.  The launch
+// therefore also moves a share of the fill straight between the cache and host
+// memory, with a few workgroups of its own, and the link copy is shorter by it.  A
+// launch of b bytes takes 4-6 us and b / 3.05 TB/s, in which the link moves b / 53
+// and 250-350 KB; with a little more than the first and less than the second the
+// share ends with the launch at every size.  (A longer share gains nothing: the
+// launch then waits for it instead of the link copy for the launch.)  Measured on
+// MI355X, calls back to back, save / load in us without a share, with b / 58 and
+// with this: one layer of 20 MB 393.7 / 398.7, 390.4 / 393.2, 390.2 / 392.5; 105 MB
+// in two 1904 / 1899, 1881 / 1868, 1876 / 1868; 524 MB in twelve 9432 / 9406, 9313 /
+// 9248, 9240 / 9230.
+constexpr uint64_t kShareBase = 64 << 10;
+constexpr uint64_t kSharePart = 44;
+constexpr uint64_t link_share_bytes(uint64_t launch_bytes) {
+  return kShareBase + launch_bytes / kSharePart;
+}
+
+// A unit of a fill: n_blocks list positions of n_seg fragments, in the order
+// (segment, position) both in the slot and in the host image.
+struct ShareUnit {
+  uint64_t n_blocks;
+  uint32_t n_seg;
+  uint64_t frag_bytes;
+  bool eligible;  // its fragments can be moved over mapped host memory in 16-byte words
+};
+
+// The share is the tail of the fill, so that link copies which cross layers stay
+// one copy: units [0, unit) and the first `staged_frags` fragments of unit `unit`
+// go through the slot, everything behind them over the link.  bytes = 0: no share
+// (unit = number of units).
+struct ShareCut {
+  size_t unit = 0;
+  uint64_t staged_frags = 0;
+  uint64_t bytes = 0;
+};
+// As many whole fragments as `want` holds, from the end of the fill up to the first
+// unit that is not eligible; never the whole fill.
+template <typename UnitAt>
+ShareCut plan_link_share(size_t n_units, uint64_t want, UnitAt unit_at) {
+  ShareCut cut;
+  cut.unit = n_units;
+  for (size_t k = n_units; k-- > 0;) {
+    const ShareUnit u = unit_at(k);
+    const uint64_t frags = u.n_blocks * u.n_seg;
+    if (!u.eligible || u.frag_bytes == 0) break;
+    uint64_t take = (want - cut.bytes) / u.frag_bytes;
+    if (take > frags) take = frags;
+    if (k == 0 && take == frags && take != 0) --take;
+    if (take == 0) break;
+    cut.unit = k;
+    cut.staged_frags = frags - take;
+    cut.bytes += take * u.frag_bytes;
+    if (take != frags) break;
+  }
+  return cut;
+}
+
+// A workgroup of a share moves a tile of one fragment at a time.  Full tiles keep
+// the link busy with 16 workgroups on the way out, whose stores nobody waits for,
+// and with 32 on the way in; more of them slow the rest of the launch (524 MB saved
+// with 16 / 32 / 64 in 9267 / 9338 / 9342 us).  Smaller fragments take
+// proportionally more (20 MB of 1 KiB fragments loaded with 16 / 64 / 256 in 444 /
+// 409 / 411, without a share in 415).
+constexpr uint64_t kShareTileBytes = 8192;
+constexpr uint32_t kShareWorkgroupsMax = 256;
+constexpr uint32_t share_workgroups(uint64_t min_frag, bool save) {
+  const uint32_t full = save ? 16 : 32;
+  if (min_frag == 0 || min_frag >= kShareTileBytes) return full;
+  const uint64_t n = full * ((kShareTileBytes + min_frag - 1) / min_frag);
+  return n < kShareWorkgroupsMax ? static_cast<uint32_t>(n) : kShareWorkgroupsMax;
+}
+
+}  // namespace pf

@@ -238,12 +238,10 @@ int Xfer::launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t
   return timing_end(s);
 }
 
-int Xfer::launch_tiles(const BlockUnit* dev_unit, const BlockUnit& host_unit, bool to_far,
-                       hipStream_t s) {
+int Xfer::launch_tiles(const BlockUnit& host_unit, bool to_far, hipStream_t s, const LinkShare& share) {
   int st = timing_begin(s);
   if (st != PF_OK) return st;
-  (void)dev_unit;
-  st = launch_block_tiles_one(host_unit, to_far, s);
+  st = launch_block_tiles_one(host_unit, to_far, s, share);
   if (st != PF_OK) return st;
   return timing_end(s);
 }
@@ -513,7 +511,7 @@ void fill_row_order(const uint32_t* ids, uint64_t n, uint64_t per_unit, uint32_t
 }  // namespace
 
 int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uint64_t n_layers,
-                        bool save, hipStream_t s) {
+                        bool save, hipStream_t s, bool may_share) {
   const LayerPlan& first = plans.front();
   const uint64_t n = first.n_blocks;
   const size_t n_plans = plans.size();
@@ -537,8 +535,22 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     int st = ensure_slot(sl, max_chunk_bytes);
     if (st != PF_OK) return st;
   }
-  // Slab: one BlockUnit per (chunk, layer), then the shared id list.
-  const uint64_t units_bytes = (chunks.size() * n_plans * sizeof(BlockUnit) + 255) & ~255ull;
+  // The last pages of a chunk are its share of the link (pf_share.hpp).
+  std::vector<uint64_t> shared_pages(chunks.size(), 0);
+  uint64_t min_frag = UINT64_MAX;
+  for (const LayerPlan& p : plans) {
+    may_share = may_share && p.vec_ok;
+    min_frag = std::min(min_frag, p.frag_bytes);
+  }
+  for (size_t ci = 0; may_share && ci < chunks.size(); ++ci) {
+    const uint64_t count = chunks[ci].count;
+    const uint64_t pages = link_share_bytes(count * pack.page_bytes) / pack.page_bytes;
+    if (pages < count && count <= kMaxSharedTileBlocks) shared_pages[ci] = pages;
+  }
+  // Slab: one BlockUnit per (chunk, layer), again for the shares, then the id list
+  // that all of them read.
+  const size_t n_units = chunks.size() * n_plans;
+  const uint64_t units_bytes = ((may_share ? 2 : 1) * n_units * sizeof(BlockUnit) + 255) & ~255ull;
   const uint64_t ids_bytes = (n * sizeof(uint32_t) + 255) & ~255ull;
   // Loads visit the pages of a chunk in ascending destination id (launch_block_tiles).
   const uint64_t slab_bytes = units_bytes + ids_bytes + (save ? 0 : ids_bytes);
@@ -606,10 +618,20 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
       }
       u.n_blocks = static_cast<uint32_t>(chunks[ci].count);
       u.n_seg = 1;
-      u.tiles_per_frag = 1;
+      u.staged_frags = static_cast<uint32_t>(chunks[ci].count - shared_pages[ci]);
       u.form = aligned16(p.layout.data_ptr()) && aligned16(p.layout.block_stride_bytes()) &&
                        aligned16(p.page_offset - pack.lo) && aligned16(pack.page_bytes)
                    ? kUnitVec : kUnitAny;
+      if (shared_pages[ci] == 0) continue;
+      const uint64_t first_shared = chunks[ci].first + u.staged_frags;
+      BlockUnit& su = units_host[n_units + ci * n_plans + k];
+      su = u;
+      su.far_base[0] = first.page_dev[first_shared] + p.page_offset;
+      su.ids = u.ids + u.staged_frags;
+      su.order = nullptr;
+      su.n_blocks = static_cast<uint32_t>(shared_pages[ci]);
+      su.tiles_per_frag = static_cast<uint32_t>((p.frag_bytes + kShareTileBytes - 1) / kShareTileBytes);
+      su.form = kUnitVec;
     }
   }
 
@@ -632,14 +654,19 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     const Chunk& c = chunks[ci];
     Slot& sl = slots_[chunk_slot[ci]];
     uint8_t* host_ptr = reinterpret_cast<uint8_t*>(first.page_host[c.first] + pack.lo);
-    const uint64_t bytes = c.count * pack.page_bytes;
+    const uint64_t bytes = (c.count - shared_pages[ci]) * pack.page_bytes;
+    // With the first launch of a chunk, that of the largest slices.
+    LinkShare share;
+    if (shared_pages[ci] != 0) {
+      share = {units_dev + n_units + ci * n_plans, static_cast<uint32_t>(n_plans), share_workgroups(min_frag, save)};
+    }
     auto launch = [&](bool to_far) -> int {
       int rc = timing_begin(s);
       if (rc != PF_OK) return rc;
       for (const UnitRun& run : unit_runs) {
         rc = launch_block_tiles(units_dev + ci * n_plans + run.begin,
                                 static_cast<uint32_t>(run.count), static_cast<uint32_t>(c.count),
-                                run.max_frag, 1, to_far, s);
+                                run.max_frag, 1, to_far, s, &run == &unit_runs.front() ? share : LinkShare());
         if (rc != PF_OK) return rc;
       }
       return timing_end(s);
@@ -834,7 +861,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (path == PF_PATH_STAGED || total >= auto_min_) {
         last_path_ = PF_PATH_STAGED;
         prof_.plan_ms += ms_since(t_call);
-        return run_page_pack(plans, pack, n_layers, save, s);
+        return run_page_pack(plans, pack, n_layers, save, s, path == PF_PATH_AUTO);
       }
     } else if (path == PF_PATH_STAGED) {
       return fail(PF_ERR_INVALID_ARGUMENT,
@@ -887,6 +914,53 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (plans[u.layer].staged) plans[u.layer].units.emplace_back(u.first, u.count);
     }
   }
+  // The share of every fill that crosses the link with its launch (pf_share.hpp),
+  // by the fill's first unit.  Calls that asked for the staged path keep every byte
+  // on it.
+  struct FillShare {
+    size_t staged_end = 0;      // one past the last unit of which a part takes the slot
+    uint64_t staged_frags = 0;  // fragments of that last unit in the slot
+    uint32_t first = 0, count = 0, workgroups = 0;  // units of the share
+  };
+  std::vector<FillShare> shares(unit_refs.size());
+  uint32_t n_share_units = 0;
+  for (size_t ui = 0; ui < unit_refs.size(); ++ui) {
+    if (group_end[ui] == 0) continue;
+    FillShare& sh = shares[ui];
+    sh.staged_end = group_end[ui];
+    uint64_t fill_bytes = 0, max_blocks = 0;
+    for (size_t k = ui; k < sh.staged_end; ++k) {
+      const LayerPlan& p = plans[unit_refs[k].plan];
+      fill_bytes += unit_refs[k].count * p.frag_bytes * p.n_seg;
+      max_blocks = std::max(max_blocks, unit_refs[k].count);
+    }
+    sh.staged_frags = unit_refs[sh.staged_end - 1].count * plans[unit_refs[sh.staged_end - 1].plan].n_seg;
+    if (path != PF_PATH_AUTO || max_blocks > kMaxSharedTileBlocks) continue;
+    const ShareCut cut = plan_link_share(sh.staged_end - ui, link_share_bytes(fill_bytes), [&](size_t k) {
+      const LayerPlan& p = plans[unit_refs[ui + k].plan];
+      return ShareUnit{unit_refs[ui + k].count, p.n_seg, p.frag_bytes, p.vec_ok};
+    });
+    if (cut.bytes == 0) continue;
+    sh.first = n_share_units;
+    uint64_t min_frag = UINT64_MAX;
+    for (size_t k = ui + cut.unit; k < sh.staged_end; ++k) {
+      const LayerPlan& p = plans[unit_refs[k].plan];
+      const uint64_t skipped = k == ui + cut.unit ? cut.staged_frags : 0;
+      // A cut inside segment 0 of two leaves its tail and segment 1 as two units.
+      sh.count += p.n_seg == 2 && skipped != 0 && skipped < unit_refs[k].count ? 2 : 1;
+      min_frag = std::min(min_frag, p.frag_bytes);
+    }
+    n_share_units += sh.count;
+    sh.workgroups = share_workgroups(min_frag, save);
+    if (cut.staged_frags != 0) {
+      sh.staged_end = ui + cut.unit + 1;
+      sh.staged_frags = cut.staged_frags;
+    } else {
+      sh.staged_end = ui + cut.unit;
+      const UnitRef& last = unit_refs[sh.staged_end - 1];
+      sh.staged_frags = last.count * plans[last.plan].n_seg;
+    }
+  }
   // The visiting orders of staged loads sit behind everything else in the slab
   // and are uploaded on their own, after the first link copy is under way:
   // `order_slab_off` is relative to that tail until the head's size is known.
@@ -900,7 +974,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     }
   }
   auto lay_out = [&](uint64_t id_bytes) {
-    slab_bytes = unit_refs.size() * sizeof(BlockUnit);
+    slab_bytes = (unit_refs.size() + n_share_units) * sizeof(BlockUnit);
     slab_bytes = (slab_bytes + 255) & ~255ull;
     order_bytes = 0;
     // Plans whose id list is in the slab: a call of many layers (times the
@@ -1051,6 +1125,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       u.far_base[0] = base;
       u.far_base[1] = base + r.count * p.frag_bytes;
       u.far_stride = p.frag_bytes;
+      u.staged_frags = u.n_blocks * u.n_seg;
       // Staging is 256-byte aligned device memory; only the near side and the
       // fragment size decide whether 16-byte vectors are safe.
       u.form = aligned16(p.layout.data_ptr()) && aligned16(p.layout.block_stride_bytes()) &&
@@ -1078,6 +1153,38 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     }
   }
   next_slot_ = slot_cursor;
+  for (size_t ui = 0; ui < unit_refs.size(); ++ui) {
+    const FillShare& sh = shares[ui];
+    if (sh.count == 0) continue;
+    BlockUnit* su = units_host + unit_refs.size() + sh.first;
+    const size_t cut = sh.staged_end - 1;
+    const bool inside = sh.staged_frags != static_cast<uint64_t>(units_host[cut].n_blocks) * units_host[cut].n_seg;
+    units_host[cut].staged_frags = static_cast<uint32_t>(sh.staged_frags);
+    // Positions [first, n) of segment `seg` (2: of both) of unit k over host memory.
+    auto add = [&](size_t k, uint64_t first, uint32_t seg) {
+      const UnitRef& r = unit_refs[k];
+      const LayerPlan& p = plans[r.plan];
+      const uint64_t far = (r.first + first) * p.host_stride;
+      BlockUnit& u = *su++;
+      u = units_host[k];
+      u.ids += first;
+      u.order = nullptr;
+      u.n_blocks = static_cast<uint32_t>(r.count - first);
+      u.n_seg = seg == 2 ? p.n_seg : 1;
+      u.far_base[0] = p.host_dev[seg == 1 ? 1 : 0] + far;
+      u.far_base[1] = p.host_dev[1] + far;
+      u.far_stride = p.host_stride;
+      if (seg == 1) u.near_base += u.kv_stride;
+      u.tiles_per_frag = static_cast<uint32_t>((p.frag_bytes + kShareTileBytes - 1) / kShareTileBytes);
+      u.form = kUnitVec;
+    };
+    if (inside) {
+      const uint64_t n = unit_refs[cut].count;
+      if (sh.staged_frags < n) add(cut, sh.staged_frags, 0);
+      if (plans[unit_refs[cut].plan].n_seg == 2) add(cut, sh.staged_frags < n ? 0 : sh.staged_frags - n, 1);
+    }
+    for (size_t k = sh.staged_end; k < group_end[ui]; ++k) add(k, 0, 2);
+  }
 
   // ---- 4. enqueue ---------------------------------------------------------
   // A second stream pays off when the link copies of one fill can overlap the
@@ -1182,6 +1289,9 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     st = fork_side();
     if (st != PF_OK) return st;
     const size_t ue = group_end[ui];
+    const FillShare& fill_share = shares[ui];
+    const size_t us = fill_share.staged_end;
+    const LinkShare share{units_dev + unit_refs.size() + fill_share.first, fill_share.count, fill_share.workgroups};
     Slot& sl = slots_[unit_slot[ui]];
     // The link copies of the group, coalesced: pieces that follow one another
     // both in staging and in the host image cross as one copy (a copy costs
@@ -1195,12 +1305,15 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       uint64_t bytes;
     };
     std::vector<LinkCopy> group_copies;
-    for (size_t k = ui; k < ue; ++k) {
+    for (size_t k = ui; k < us; ++k) {
       const UnitRef& r = unit_refs[k];
       const LayerPlan& q = plans[r.plan];
       const BlockUnit& u = units_host[k];
       for (uint32_t sgm = 0; sgm < q.n_seg; ++sgm) {
-        LinkCopy c{q.host[sgm] + r.first * q.host_stride, u.far_base[sgm], r.count * q.frag_bytes};
+        const uint64_t before = sgm * r.count;
+        const uint64_t frags = u.staged_frags > before ? std::min<uint64_t>(u.staged_frags - before, r.count) : 0;
+        if (frags == 0) break;
+        LinkCopy c{q.host[sgm] + r.first * q.host_stride, u.far_base[sgm], frags * q.frag_bytes};
         if (!group_copies.empty() &&
             group_copies.back().host + group_copies.back().bytes == c.host &&
             group_copies.back().staged + group_copies.back().bytes == c.staged) {
@@ -1222,7 +1335,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       return PF_OK;
     };
     auto launch_group = [&](bool to_far) -> int {
-      if (ue - ui == 1) return launch_tiles(units_dev + ui, units_host[ui], to_far, s);
+      if (us - ui == 1) return launch_tiles(units_host[ui], to_far, s, share);
       // Workgroups the one-launch form would start: the rows form (up to
       // kRowsLaunchUnits units) starts every row with the tiles of the largest
       // fragment and the segments of the widest unit; the units-inner form also
@@ -1232,7 +1345,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       };
       uint32_t max_blocks = 0, max_seg = 0;
       uint64_t max_frag = 0, max_tiles = 0, total_rows = 0;
-      for (size_t k = ui; k < ue; ++k) {
+      for (size_t k = ui; k < us; ++k) {
         const BlockUnit& u = units_host[k];
         max_blocks = std::max(max_blocks, u.n_blocks);
         max_seg = std::max(max_seg, u.n_seg);
@@ -1240,7 +1353,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         max_tiles = std::max(max_tiles, tiles_of(u));
         total_rows += u.n_blocks;
       }
-      const size_t n_group = ue - ui;
+      const size_t n_group = us - ui;
       const bool rows_form = n_group <= kRowsLaunchUnits;
       const uint64_t started =
           (rows_form ? total_rows : static_cast<uint64_t>(max_blocks) * n_group) * max_tiles * max_seg;
@@ -1259,11 +1372,12 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         size_t begin, end;
       };
       std::vector<Run> runs;
-      uint64_t runs_started = 0;
-      for (size_t k = ui; k < ue;) {
+      uint64_t runs_started = 0, most_tiles = 0;
+      size_t largest_run = 0;  // carries the share
+      for (size_t k = ui; k < us;) {
         size_t e = k;
         uint64_t run_useful = 0, run_rows = 0, run_tiles = 0, run_seg = 0;
-        while (e < ue && e - k < kRowsLaunchUnits) {
+        while (e < us && e - k < kRowsLaunchUnits) {
           const BlockUnit& u = units_host[e];
           const uint64_t nu = run_useful + static_cast<uint64_t>(u.n_blocks) * tiles_of(u) * u.n_seg;
           const uint64_t nr = run_rows + u.n_blocks;
@@ -1275,6 +1389,10 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
           run_tiles = nt;
           run_seg = ns;
           ++e;
+        }
+        if (run_useful > most_tiles) {
+          most_tiles = run_useful;
+          largest_run = runs.size();
         }
         runs.push_back({k, e});
         runs_started += run_rows * run_tiles * run_seg;
@@ -1288,10 +1406,11 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (rc != PF_OK) return rc;
       bool launched = false;
       if (in_runs) {
-        for (const Run& run : runs) {
+        for (size_t ri = 0; ri < runs.size(); ++ri) {
+          const Run& run = runs[ri];
           rc = launch_block_tiles_rows(units_dev + run.begin, units_host + run.begin,
                                        static_cast<uint32_t>(run.end - run.begin), to_far, s,
-                                       &launched);
+                                       &launched, ri == largest_run ? share : LinkShare());
           if (rc != PF_OK) return rc;
           // (Only a launch beyond the grid limits is refused; what went out
           // before it is then simply done again by the form below.)
@@ -1299,12 +1418,12 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         }
       } else if (rows_form) {
         rc = launch_block_tiles_rows(units_dev + ui, units_host + ui, static_cast<uint32_t>(n_group),
-                                     to_far, s, &launched);
+                                     to_far, s, &launched, share);
         if (rc != PF_OK) return rc;
       }
       if (!launched) {
         rc = launch_block_tiles(units_dev + ui, static_cast<uint32_t>(n_group), max_blocks, max_frag,
-                                max_seg, to_far, s);
+                                max_seg, to_far, s, share);
         if (rc != PF_OK) return rc;
       }
       return timing_end(s);

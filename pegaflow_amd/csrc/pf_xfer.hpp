@@ -310,7 +310,7 @@ class Xfer {
   };
   bool plan_page_pack(const std::vector<LayerPlan>& plans, bool save, PagePack* out);
   int run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uint64_t n_layers,
-                    bool save, hipStream_t s);
+                    bool save, hipStream_t s, bool may_share);
   int plan_layer(const pf_layer_blocks& in, const SecondSegmentTable& second, size_t index,
                  int path, LayerPlan* out, bool* skip);
   int ensure_slot(Slot& sl, uint64_t bytes);
@@ -331,8 +331,7 @@ class Xfer {
   int launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
                           uint64_t max_tiles, uint32_t workgroups, bool to_far, hipStream_t s);
   // Staged form: one tile per workgroup over one unit.
-  int launch_tiles(const BlockUnit* dev_unit, const BlockUnit& host_unit, bool to_far,
-                   hipStream_t s);
+  int launch_tiles(const BlockUnit& host_unit, bool to_far, hipStream_t s, const LinkShare& share);
   int timing_begin(hipStream_t s);
   int timing_end(hipStream_t s);
 

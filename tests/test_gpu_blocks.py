@@ -1064,3 +1064,81 @@ def test_tiles_of_unlike_units_are_dealt_out_once(stream, workgroups):
         c.close()
         host.close()
     xfer.close()
+
+
+# Staged calls of AUTO move a share of every fill over the link with the gather /
+# scatter launch (pf_share.hpp).  Layers (blocks, fragment, segments) by where the
+# fill is cut and by the launch that carries the share.
+SHARES = {
+    "tail_of_v": [(80, 32768, 2)],                                   # 5 MiB: ordered rows on the load
+    "tail_of_k_and_v": [(60, 32768, 2), (5, 16384, 2)],
+    "one_segment": [(40, 73728, 1)],
+    "whole_layers": [(60, 32768, 2), (1, 32768, 2), (1, 16384, 1), (2, 4096, 2)],
+    "whole_layer_to_the_fragment": [(61, 16384, 1), (1, 65536, 1)],  # 64 KiB and a little are wanted
+    "short_tiles": [(300, 1040, 2), (100, 12304, 2)],
+    "fragments_of_1k": [(1500, 1024, 1)],
+    "fragment_larger_than_the_share": [(3, 262144, 2)],
+    "last_layer_off_the_grid": [(60, 32768, 2), (50, 1000, 2)],
+    "off_the_grid_before": [(50, 1000, 2), (60, 32768, 2)],
+    "units_inner": [(7 + i, 16384, 1 + i % 2) for i in range(12)],
+    "unlike_lengths_in_runs": [(600, 16384, 2)] + [(2, 16384, 2)] * 11,
+    "rows_folded": [(40000, 64, 1), (40000, 64, 1)],
+    "most_rows_of_one_unit": [(65279, 64, 1)],
+    "too_many_rows": [(65500, 64, 1)],
+}
+
+
+@pytest.mark.parametrize("copy_stream", [1, 2], ids=["side_stream", "in_order"])
+@pytest.mark.parametrize("name", sorted(SHARES))
+def test_share_of_the_link_matches_oracle(name, copy_stream, stream):
+    rng = np.random.default_rng(zlib.crc32(name.encode()))
+    cases = [Case(rng, num_blocks=n + 9, seg=seg, segments=segments, n_ids=n) for n, seg, segments in SHARES[name]]
+    sizes = [len(c.ids) * c.seg * c.segments for c in cases]
+    pool = PinnedMemory(sum(sizes) + 4096)
+    x = BlockTransfer(auto_staged_min_bytes=1, copy_stream=copy_stream)
+
+    def layers(lists):
+        out, at = [], 0
+        for c, ids, size in zip(cases, lists, sizes):
+            offs = [at + s * (size // c.segments) for s in range(c.segments)]
+            out.append(LayerBlocks(layout=c.product_layout(), block_ids=ids,
+                                   host=tuple(pool.host_ptr + o for o in offs),
+                                   host_device=tuple(pool.device_ptr + o for o in offs),
+                                   host_len=(size // c.segments,) * c.segments, host_stride=c.seg))
+            at += size
+        return out
+
+    try:
+        for c in cases:
+            c.dev.copy_from_host(c.cache0)
+        pool.as_numpy()[:] = SENT
+        x.save(layers([c.ids for c in cases]), stream, TransferPath.AUTO)
+        stream.synchronize()
+        assert x.last_path == ST
+        want = np.full(pool.as_numpy().size, SENT, dtype=np.uint8)
+        at = 0
+        for c, size in zip(cases, sizes):
+            segs = [want[at + s * (size // c.segments): at + (s + 1) * (size // c.segments)] for s in range(2)]
+            cache = c.cache0.copy()  # alive across the call: the layout holds its address
+            O.transfer_layer(c.oracle_layout(cache), c.ids, segs[0], segs[1] if c.segments == 2 else None,
+                             host_is_src=False)
+            at += size
+        assert np.array_equal(pool.as_numpy(), want)
+        dests = [rng.choice(c.num_blocks, len(c.ids), replace=False).astype(np.uint32) for c in cases]
+        for c in cases:
+            c.dev.fill(SENT)
+        x.load(layers(dests), stream, TransferPath.AUTO)
+        stream.synchronize()
+        at = 0
+        for c, ids, size in zip(cases, dests, sizes):
+            cache = np.full_like(c.cache0, SENT)
+            segs = [want[at + s * (size // c.segments): at + (s + 1) * (size // c.segments)] for s in range(2)]
+            O.transfer_layer(c.oracle_layout(cache), ids, segs[0], segs[1] if c.segments == 2 else None,
+                             host_is_src=True)
+            assert np.array_equal(c.dev.copy_to_host(), cache), (c.args, len(ids))
+            at += size
+    finally:
+        x.close()
+        pool.close()
+        for c in cases:
+            c.close()
