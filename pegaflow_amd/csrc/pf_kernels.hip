@@ -333,6 +333,25 @@ __global__ __launch_bounds__(kLanes) void desc_copy_waves_kernel(Rows rows, uint
                                    threadIdx.x % kWave);
 }
 
+// A packing launch: rows between the cache and staging, one per LANES lanes, and
+// beside them, by the first `link_groups` workgroups, the rows of the run's share of
+// the link (pf_share.hpp).
+template <int U, bool HOST_IS_SRC, int LANES>
+__global__ __launch_bounds__(kLanes) void desc_pack_kernel(Rows3<true> rows, uint32_t n,
+                                                           Rows3<false> link, uint32_t n_link,
+                                                           uint32_t link_groups) {
+  constexpr uint32_t kRows = kLanes / LANES;  // of a workgroup at a time
+  const uint32_t sub = __builtin_amdgcn_readfirstlane(threadIdx.x / LANES);
+  const uint32_t lane = threadIdx.x % LANES;
+  if (blockIdx.x < link_groups) {
+    copy_rows<U, LANES, HOST_IS_SRC>(link, n_link, blockIdx.x * kRows + sub, link_groups * kRows,
+                                     blockIdx.y, gridDim.y, lane);
+  } else {
+    copy_rows<U, LANES, HOST_IS_SRC>(rows, n, (blockIdx.x - link_groups) * kRows + sub,
+                                     (gridDim.x - link_groups) * kRows, blockIdx.y, gridDim.y, lane);
+  }
+}
+
 // The fields of a unit, wave-uniform: read once into scalar registers, all
 // before the first branch on them, so that they cost one trip to memory.
 struct UnitFields {
@@ -1131,19 +1150,17 @@ namespace {
 constexpr uint64_t kWaveRowBytes = 2048;
 constexpr uint64_t kFewRows = 64;
 
-template <bool HOST_IS_SRC, typename Rows>
-void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
-                 uint32_t max_workgroups) {
-  const dim3 block(kLanes, 1, 1);
+struct RowsGrid {
+  uint32_t x, y;
+  bool waves;  // a row per wavefront
+};
+RowsGrid rows_grid(uint64_t n, uint64_t max_size, uint32_t max_workgroups) {
   constexpr uint64_t kWaves = kLanes / kWave;
   if (max_size <= kWaveRowBytes && n > kFewRows) {
     uint64_t gx = (n + kWaves - 1) / kWaves;
     if (max_workgroups != 0 && gx > max_workgroups) gx = max_workgroups;
     if (gx > kMaxGridX) gx = kMaxGridX;
-    hipLaunchKernelGGL((desc_copy_waves_kernel<kDescUnroll, HOST_IS_SRC, Rows>),
-                       dim3(static_cast<uint32_t>(gx), 1, 1), block, 0, s, rows,
-                       static_cast<uint32_t>(n));
-    return;
+    return {static_cast<uint32_t>(gx), 1, true};
   }
   constexpr uint64_t kTile = tile_bytes(kDescUnroll);
   uint64_t gx = n < kMaxGridX ? n : kMaxGridX;
@@ -1157,28 +1174,65 @@ void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
   // Keep the launch to a few million workgroups; a smaller grid only means
   // more iterations per workgroup.
   while (gx * gy > (1ull << 22) && gy > 1) gy >>= 1;
-  hipLaunchKernelGGL((desc_copy_kernel<kDescUnroll, HOST_IS_SRC, Rows>),
-                     dim3(static_cast<uint32_t>(gx), static_cast<uint32_t>(gy), 1), block, 0, s,
-                     rows, static_cast<uint32_t>(n));
+  return {static_cast<uint32_t>(gx), static_cast<uint32_t>(gy), false};
+}
+
+template <bool HOST_IS_SRC, typename Rows>
+void launch_rows(const Rows rows, uint64_t n, uint64_t max_size, hipStream_t s,
+                 uint32_t max_workgroups) {
+  const RowsGrid g = rows_grid(n, max_size, max_workgroups);
+  const dim3 grid(g.x, g.y, 1), block(kLanes, 1, 1);
+  if (g.waves) {
+    hipLaunchKernelGGL((desc_copy_waves_kernel<kDescUnroll, HOST_IS_SRC, Rows>), grid, block, 0, s,
+                       rows, static_cast<uint32_t>(n));
+  } else {
+    hipLaunchKernelGGL((desc_copy_kernel<kDescUnroll, HOST_IS_SRC, Rows>), grid, block, 0, s, rows,
+                       static_cast<uint32_t>(n));
+  }
+}
+
+template <bool HOST_IS_SRC>
+void launch_packing(const uint64_t* table, uint64_t n, uint64_t n_link, uint64_t max_size,
+                    uint32_t link_workgroups, hipStream_t s, uint32_t max_workgroups) {
+  const RowsGrid g = rows_grid(n, max_size, max_workgroups);
+  const uint32_t link_groups = n_link == 0 ? 0 : (link_workgroups + g.y - 1) / g.y;
+  const dim3 grid(g.x + link_groups, g.y, 1), block(kLanes, 1, 1);
+  const Rows3<true> rows{table};
+  const Rows3<false> link{table + 3 * n};
+  if (g.waves) {
+    hipLaunchKernelGGL((desc_pack_kernel<kDescUnroll, HOST_IS_SRC, kWave>), grid, block, 0, s, rows,
+                       static_cast<uint32_t>(n), link, static_cast<uint32_t>(n_link), link_groups);
+  } else {
+    hipLaunchKernelGGL((desc_pack_kernel<kDescUnroll, HOST_IS_SRC, kLanes>), grid, block, 0, s, rows,
+                       static_cast<uint32_t>(n), link, static_cast<uint32_t>(n_link), link_groups);
+  }
 }
 }  // namespace
 
 int launch_desc_copy(const uint64_t* table, uint64_t n, uint64_t max_size, bool host_is_src,
-                     bool packing, hipStream_t s, uint32_t max_workgroups) {
+                     hipStream_t s, uint32_t max_workgroups) {
   if (n == 0) return PF_OK;
-  if (packing) {
-    if (host_is_src) {
-      launch_rows<true>(Rows3<true>{table}, n, max_size, s, max_workgroups);
-    } else {
-      launch_rows<false>(Rows3<true>{table}, n, max_size, s, max_workgroups);
-    }
-  } else if (host_is_src) {
+  if (host_is_src) {
     launch_rows<true>(Rows3<false>{table}, n, max_size, s, max_workgroups);
   } else {
     launch_rows<false>(Rows3<false>{table}, n, max_size, s, max_workgroups);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "desc_copy_kernel launch");
+  return PF_OK;
+}
+
+int launch_desc_pack(const uint64_t* table, uint64_t n, uint64_t n_link, uint64_t max_size,
+                     bool host_is_src, hipStream_t s, uint32_t max_workgroups,
+                     uint32_t link_workgroups) {
+  if (n == 0) return PF_OK;
+  if (host_is_src) {
+    launch_packing<true>(table, n, n_link, max_size, link_workgroups, s, max_workgroups);
+  } else {
+    launch_packing<false>(table, n, n_link, max_size, link_workgroups, s, max_workgroups);
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail_hip(e, "desc_pack_kernel launch");
   return PF_OK;
 }
 

@@ -4,6 +4,7 @@
 #include <cstring>
 
 #include "pf_common.hpp"
+#include "pf_share.hpp"
 
 namespace pf {
 
@@ -280,6 +281,8 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     uint8_t* host_begin;
     uint64_t bytes;
     std::vector<uint32_t> members;  // indices into `ranges`
+    size_t packed = 0;              // members that go through staging; the others are
+    uint64_t link_bytes = 0;        // the packing launch's share of the link (pf_share.hpp)
   };
   std::vector<Run> runs;
   std::vector<std::pair<uint64_t, size_t>> open;  // host allocation -> index of its open run
@@ -316,7 +319,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       if (open.size() >= 64) open.erase(open.begin());  // bound the linear search
       open.emplace_back(r.host_allocation, runs.size());
     }
-    runs.push_back(Run{r.host, r.size, {static_cast<uint32_t>(i)}});
+    runs.push_back(Run{r.host, r.size, {static_cast<uint32_t>(i)}, 0, 0});
   }
   std::vector<uint32_t> isolated;
   bool isolated_mapped = true;
@@ -327,7 +330,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       if (ranges[i].size < kLargeRange && ranges[i].size != 0) isolated.push_back(static_cast<uint32_t>(i));
     }
   }
-  for (const Run& run : runs) {
+  for (Run& run : runs) {
     if (run.members.size() == 1) {
       isolated.push_back(run.members[0]);
       isolated_mapped = isolated_mapped && ranges[run.members[0]].host_device != 0;
@@ -335,6 +338,12 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       staged_pieces += run.members.size();
       max_run_bytes = std::max(max_run_bytes, run.bytes + 16);
       for (uint32_t m : run.members) max_staged_piece = std::max(max_staged_piece, ranges[m].size);
+      const ShareCut cut = plan_link_share(run.members.size(), link_share_bytes(run.bytes), [&](size_t k) {
+        const Range& r = ranges[run.members[k]];
+        return ShareUnit{1, 1, r.size, r.host_device != 0};
+      });
+      run.packed = cut.unit;
+      run.link_bytes = cut.bytes;
     }
   }
   const bool isolated_by_kernel = isolated_mapped && isolated.size() > kFewRanges;
@@ -410,11 +419,12 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     // Keep the host side's alignment modulo 16 so aligned pieces stay on the
     // 16-byte path of the kernel.
     const uint64_t pad = reinterpret_cast<uint64_t>(run.host_begin) & 15ull;
-    for (uint32_t m : run.members) {
-      const Range& r = ranges[m];
-      const uint64_t in_staging = staging_base + pad + static_cast<uint64_t>(r.host - run.host_begin);
-      table[3 * row + 0] = host_is_src ? r.device : in_staging;
-      table[3 * row + 1] = host_is_src ? in_staging : r.device;
+    for (size_t k = 0; k < run.members.size(); ++k) {
+      const Range& r = ranges[run.members[k]];
+      const uint64_t far = k < run.packed ? staging_base + pad + static_cast<uint64_t>(r.host - run.host_begin)
+                                          : r.host_device;
+      table[3 * row + 0] = host_is_src ? r.device : far;
+      table[3 * row + 1] = host_is_src ? far : r.device;
       table[3 * row + 2] = r.size;
       ++row;
     }
@@ -432,7 +442,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
   }
   row = 0;
   if (isolated_by_kernel) {
-    st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, false, s,
+    st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, s,
                           host_link_workgroups(isolated_bytes, isolated.size()));
     if (st != PF_OK) return st;
     row = isolated.size();
@@ -445,20 +455,20 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     uint8_t* in_staging = static_cast<uint8_t*>(staging_) + pad;
     if (host_is_src) {
       PF_HIP(hipMemcpyHtoDAsync(reinterpret_cast<hipDeviceptr_t>(in_staging), run.host_begin,
-                                run.bytes, s));
+                                run.bytes - run.link_bytes, s));
     }
     // Many pieces of at most one tile: two rows per workgroup, so that the second
     // row's descriptor is on its way while the first is copied (65 536 pieces of
     // 4 KiB: 92 us instead of 98).
-    const uint64_t pieces = run.members.size();
+    const uint64_t pieces = run.packed, shared = run.members.size() - run.packed;
     const uint32_t pack_workgroups =
         max_staged_piece <= 16384 && pieces >= 8192 ? static_cast<uint32_t>((pieces + 1) / 2) : 0;
-    st = launch_desc_copy(table_dev + 3 * row, pieces, max_staged_piece, host_is_src, true, s,
-                          pack_workgroups);
+    st = launch_desc_pack(table_dev + 3 * row, pieces, shared, max_staged_piece, host_is_src, s,
+                          pack_workgroups, shared ? host_link_workgroups(run.link_bytes, shared) : 0);
     if (st != PF_OK) return st;
     if (!host_is_src) {
       PF_HIP(hipMemcpyDtoHAsync(run.host_begin, reinterpret_cast<hipDeviceptr_t>(in_staging),
-                                run.bytes, s));
+                                run.bytes - run.link_bytes, s));
     }
     row += run.members.size();
   }
@@ -517,7 +527,7 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
   } else {
     PF_HIP(hipMemcpyAsync(slab->dev, slab->host, bytes, hipMemcpyHostToDevice, s));
   }
-  st = launch_desc_copy(table_dev, n, max_size, host_is_src, false, s,
+  st = launch_desc_copy(table_dev, n, max_size, host_is_src, s,
                         host_link_workgroups(total_size, n));
   if (st != PF_OK) return st;
   return slabs_.release_after(slab, s);

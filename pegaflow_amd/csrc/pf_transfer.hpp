@@ -128,10 +128,15 @@ class KernelBackend : public TransferBackend {
 std::unique_ptr<TransferBackend> build_backend(TransferMode mode);
 
 // Launch the descriptor-table copy kernel: `table` is a device array of
-// 3*n u64 words [dst, src, size].  `max_size` is the largest size in it.
-// `packing`: both sides lie in device memory.  `max_workgroups` caps the grid (0 =
-// as many as the batch has tiles).
+// 3*n u64 words [dst, src, size].  `max_size` is the largest size in it;
+// `max_workgroups` caps the grid (0 = as many as the batch has tiles).
 int launch_desc_copy(const uint64_t* table, uint64_t n, uint64_t max_size, bool host_is_src,
-                     bool packing, hipStream_t s, uint32_t max_workgroups = 0);
+                     hipStream_t s, uint32_t max_workgroups = 0);
+// The same between two places in device memory (packing), and beside it by about
+// `link_workgroups` workgroups of their own the `n_link` rows that follow, whose far
+// side is mapped host memory.
+int launch_desc_pack(const uint64_t* table, uint64_t n, uint64_t n_link, uint64_t max_size,
+                     bool host_is_src, hipStream_t s, uint32_t max_workgroups,
+                     uint32_t link_workgroups);
 
 }  // namespace pf

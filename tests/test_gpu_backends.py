@@ -351,6 +351,36 @@ def test_direct_backend_packs_host_dense_runs(stream, gpu, n):
         b.close()
 
 
+@pytest.mark.parametrize("size, n, unmapped", [
+    (600, 30000, 0),      # a row per wavefront, packed and over the link
+    (4097, 4200, 0),      # a row per workgroup, off the 16-byte grid
+    (20016, 900, 0),      # two tiles a row
+    (300000, 60, 0),      # one row over the link, 19 tiles
+    (600000, 30, 0),      # no row as short as the share
+    (4096, 4200, 1),      # the last piece has no device-visible address: no share
+    (4096, 4200, 4200),
+])
+def test_direct_backend_moves_the_tail_of_a_run_over_the_link(stream, gpu, size, n, unmapped):
+    """Runs of more than 16 MiB are packed; their tail crosses the link with the
+    packing launch (pf_share.hpp)."""
+    from pegaflow_amd.transfer import desc_array
+    pos = np.arange(n, dtype=np.uint64)
+    dev_off = np.array(xorshift_shuffle(n), dtype=np.uint64) * np.uint64(size + 48) + np.uint64(16)
+    host_off = pos * np.uint64(size) + np.uint64(32)
+    mapped = (pos < n - unmapped).astype(np.uint64)
+    rows = [(int(d), int(h), size) for d, h in zip(dev_off, host_off)]
+
+    def descs(dev, host):
+        return desc_array(dev.ptr + dev_off, host.host_ptr + host_off, (host.device_ptr + host_off) * mapped,
+                          size, 0, 1)
+
+    b = MemcpyBackend()
+    try:
+        _run_both_directions(b, stream, descs, n * (size + 48) + 64, n * size + 64, rows, seed=size)
+    finally:
+        b.close()
+
+
 def test_direct_backend_mixed_batch(stream, gpu):
     """One batch holding a large range, a host-dense run of odd-sized unaligned
     pieces, isolated small ranges without a device-visible host address (so
