@@ -247,6 +247,14 @@ __device__ __forceinline__ void copy_tile_in_hbm(uint64_t dst, uint64_t src, uin
   }
 }
 
+// A call's tables from mapped host memory to their place in device memory, 16 bytes
+// per lane.  The launches behind it read them through the scalar cache of every XCD.
+__global__ __launch_bounds__(kLanes) void table_upload_kernel(uint64_t dst, uint64_t src, uint32_t n) {
+  for (uint32_t i = blockIdx.x * kLanes + threadIdx.x; i < n; i += gridDim.x * kLanes) {
+    reinterpret_cast<g_u32x4*>(dst)[i] = reinterpret_cast<const g_u32x4*>(src)[i];
+  }
+}
+
 // Rows of a descriptor table, wave-uniform.  Rows3: [dst, src, size] as the
 // backends write it; Rows48: the caller's pf_copy_desc array as it is, so the
 // host side repacks nothing.
@@ -781,6 +789,7 @@ constexpr int kTileLanes = 128;  // lanes of a block_tiles_kernel workgroup
 static_assert(kTileLanes * 16 == kStagedTileBytes, "tile size the planner of launches assumes");
 constexpr uint32_t kMaxGridX = 1u << 22;  // the kernels grid-stride past this
 constexpr int kDescUnroll = 4;
+constexpr uint32_t kMaxUploadWorkgroups = 64;
 
 }  // namespace
 
@@ -1135,6 +1144,20 @@ int launch_plain_copy(void* dst, const void* src, uint64_t bytes, int unroll, hi
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "plain_copy_kernel launch");
+  return PF_OK;
+}
+
+int launch_table_upload(uint64_t dst, uint64_t src, uint64_t bytes, hipStream_t s) {
+  const uint64_t n = bytes / 16;
+  if (n == 0) return PF_OK;
+  if ((bytes & 15ull) != 0 || ((dst | src) & 15ull) != 0 || n > 0xFFFFFFFFull - (kMaxUploadWorkgroups * kLanes)) {
+    return fail(PF_ERR_INVALID_ARGUMENT, "table upload of %llu bytes", static_cast<unsigned long long>(bytes));
+  }
+  const uint64_t groups = (n + kLanes - 1) / kLanes;
+  const dim3 grid(static_cast<uint32_t>(groups < kMaxUploadWorkgroups ? groups : kMaxUploadWorkgroups), 1, 1);
+  hipLaunchKernelGGL(table_upload_kernel, grid, dim3(kLanes, 1, 1), 0, s, dst, src, static_cast<uint32_t>(n));
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail_hip(e, "table_upload_kernel launch");
   return PF_OK;
 }
 

@@ -142,7 +142,10 @@ int SlabPool::acquire(uint64_t bytes, Slab** out) {
   while (cap < bytes) cap <<= 1;
   std::unique_ptr<Slab> s(new Slab());
   PF_HIP(hipHostMalloc(&s->host, cap, hipHostMallocMapped | hipHostMallocPortable));
-  hipError_t e = hipMalloc(&s->dev, cap);
+  void* alias = nullptr;
+  hipError_t e = hipHostGetDevicePointer(&alias, s->host, 0);
+  s->host_alias = reinterpret_cast<uint64_t>(alias);
+  if (e == hipSuccess) e = hipMalloc(&s->dev, cap);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->done, hipEventDisableTiming);
   if (e != hipSuccess) {
     (void)hipHostFree(s->host);
@@ -152,6 +155,25 @@ int SlabPool::acquire(uint64_t bytes, Slab** out) {
   s->cap = cap;
   *out = s.get();
   slabs_.push_back(std::move(s));
+  return PF_OK;
+}
+
+// A kernel reads the slab where it was written: as a command it is cheaper than a
+// copy, which the runtime carries out with a kernel or an engine of its own, and the
+// launch behind it follows without a hand-over.  Measured on MI355X: 16 384 descriptors
+// (393 KB) out and back 2442 -> 2426 us, a staged save of 33 MB in 32 layers (4 KB)
+// 677 -> 654 us from submission to completion.  Longer tables belong to calls of
+// milliseconds and leave the compute units alone.
+constexpr uint64_t kUploadByKernel = 1ull << 20;
+
+int SlabPool::upload(const Slab* slab, uint64_t first, uint64_t end, hipStream_t s) {
+  if (end <= first) return PF_OK;
+  const uint64_t bytes = (end - first + 15) & ~15ull;
+  if (bytes <= kUploadByKernel) {
+    return launch_table_upload(reinterpret_cast<uint64_t>(slab->dev) + first, slab->host_alias + first, bytes, s);
+  }
+  PF_HIP(hipMemcpyAsync(static_cast<uint8_t*>(slab->dev) + first, static_cast<uint8_t*>(slab->host) + first,
+                        end - first, hipMemcpyHostToDevice, s));
   return PF_OK;
 }
 
@@ -432,16 +454,20 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
   // A short table of ranges that all go through the mapped-memory kernel is
   // read where it was written (see KernelBackend::submit_impl); tables of
   // packing launches stay in device memory, where the HBM-rate kernels read them.
+  bool uploaded = false;
+  auto upload_table = [&]() -> int {
+    if (uploaded) return PF_OK;
+    uploaded = true;
+    return SlabPool::upload(slab, 0, table_rows * 3 * sizeof(uint64_t), s);
+  };
   if (staged_pieces == 0 && table_rows * 3 * sizeof(uint64_t) <= kHostTableBytes) {
-    void* alias = nullptr;
-    PF_HIP(hipHostGetDevicePointer(&alias, slab->host, 0));
-    table_dev = static_cast<const uint64_t*>(alias);
-  } else {
-    PF_HIP(hipMemcpyAsync(slab->dev, slab->host, table_rows * 3 * sizeof(uint64_t),
-                          hipMemcpyHostToDevice, s));
+    table_dev = reinterpret_cast<const uint64_t*>(slab->host_alias);
+    uploaded = true;
   }
   row = 0;
   if (isolated_by_kernel) {
+    st = upload_table();
+    if (st != PF_OK) return st;
     st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, s,
                           host_link_workgroups(isolated_bytes, isolated.size()));
     if (st != PF_OK) return st;
@@ -457,6 +483,9 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       PF_HIP(hipMemcpyHtoDAsync(reinterpret_cast<hipDeviceptr_t>(in_staging), run.host_begin,
                                 run.bytes - run.link_bytes, s));
     }
+    // (Behind the first run's copy on the way in: the link starts with the payload.)
+    st = upload_table();
+    if (st != PF_OK) return st;
     // Many pieces of at most one tile: two rows per workgroup, so that the second
     // row's descriptor is on its way while the first is copied (65 536 pieces of
     // 4 KiB: 92 us instead of 98).
@@ -521,11 +550,10 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
   // hides behind the copy of the row before.
   const uint64_t* table_dev = static_cast<const uint64_t*>(slab->dev);
   if (bytes <= kHostTableBytes) {
-    void* alias = nullptr;
-    PF_HIP(hipHostGetDevicePointer(&alias, slab->host, 0));
-    table_dev = static_cast<const uint64_t*>(alias);
+    table_dev = reinterpret_cast<const uint64_t*>(slab->host_alias);
   } else {
-    PF_HIP(hipMemcpyAsync(slab->dev, slab->host, bytes, hipMemcpyHostToDevice, s));
+    st = SlabPool::upload(slab, 0, bytes, s);
+    if (st != PF_OK) return st;
   }
   st = launch_desc_copy(table_dev, n, max_size, host_is_src, s,
                         host_link_workgroups(total_size, n));

@@ -41,6 +41,7 @@ class SlabPool {
   struct Slab {
     void* host = nullptr;
     void* dev = nullptr;
+    uint64_t host_alias = 0;  // device-visible address of `host`
     uint64_t cap = 0;
     hipEvent_t done = nullptr;
     bool in_flight = false;
@@ -48,6 +49,9 @@ class SlabPool {
   ~SlabPool();
   // A slab of at least `bytes` whose previous use (if any) has completed.
   int acquire(uint64_t bytes, Slab** out);
+  // Bring bytes [first, end) of the slab to the device, in order on `s`; `first` is a
+  // multiple of 16, and up to 15 bytes behind `end` may go along.
+  static int upload(const Slab* slab, uint64_t first, uint64_t end, hipStream_t s);
   // Mark the slab busy until everything enqueued on `s` so far has run.
   int release_after(Slab* slab, hipStream_t s);
 
@@ -126,6 +130,9 @@ class KernelBackend : public TransferBackend {
 
 // gpu_worker.rs:264-276.
 std::unique_ptr<TransferBackend> build_backend(TransferMode mode);
+
+// Copy `bytes` (a multiple of 16) of a table from mapped host memory to device memory.
+int launch_table_upload(uint64_t dst, uint64_t src, uint64_t bytes, hipStream_t s);
 
 // Launch the descriptor-table copy kernel: `table` is a device array of
 // 3*n u64 words [dst, src, size].  `max_size` is the largest size in it;

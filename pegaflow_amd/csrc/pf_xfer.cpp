@@ -644,11 +644,15 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   began_ = true;
   const Clock::time_point t_enqueue = Clock::now();
   prof_mark_begin(s);
-  PF_HIP(hipMemcpyAsync(slab->dev, slab->host, slab_bytes, hipMemcpyHostToDevice, s));
   hipStream_t side = on_side ? side_ : s;
   if (side != s) {
     PF_HIP(hipEventRecord(fork_, s));
     PF_HIP(hipStreamWaitEvent(side, fork_, 0));
+  }
+  // Loads begin with the first link copy: the tables are needed behind it.
+  if (save) {
+    st = SlabPool::upload(slab, 0, slab_bytes, s);
+    if (st != PF_OK) return st;
   }
   for (size_t ci = 0; ci < chunks.size(); ++ci) {
     const Chunk& c = chunks[ci];
@@ -687,6 +691,10 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
       if (st != PF_OK) return st;
       PF_HIP(hipMemcpyAsync(sl.buf, host_ptr, bytes, hipMemcpyHostToDevice, side));
       prof_mark_first(side);
+      if (ci == 0) {
+        st = SlabPool::upload(slab, 0, slab_bytes, s);
+        if (st != PF_OK) return st;
+      }
       st = slot_ready(sl, side, s);
       if (st != PF_OK) return st;
       st = launch(false);
@@ -701,15 +709,15 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     PF_HIP(hipEventRecord(join_, side));
     PF_HIP(hipStreamWaitEvent(s, join_, 0));
   }
-  st = slots_in_order_end(s);
-  if (st != PF_OK) return st;
   // Every layer of a page lands together: all per-layer events fire at the end.
   if (!layer_events_.empty()) {
     for (uint64_t li = 0; li < n_layers; ++li) PF_HIP(hipEventRecord(layer_events_[li], s));
   }
+  prof_mark_end(s, false);
+  st = slots_in_order_end(s);
+  if (st != PF_OK) return st;
   st = slabs_.release_after(slab, s);
   if (st != PF_OK) return st;
-  prof_mark_end(s, false);
   prof_.enqueue_ms += ms_since(t_enqueue);
   return PF_OK;
 }
@@ -962,7 +970,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     }
   }
   // The visiting orders of staged loads sit behind everything else in the slab
-  // and are uploaded on their own, after the first link copy is under way:
+  // and are uploaded after the first link copy is under way:
   // `order_slab_off` is relative to that tail until the head's size is known.
   uint64_t slab_bytes = 0, order_bytes = 0;
   bool all_zero_copy = true;
@@ -1203,15 +1211,22 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   prof_.plan_ms += ms_since(t_call) - (prof_.staging_alloc_ms - alloc_before);
   const Clock::time_point t_enqueue = Clock::now();
   prof_mark_begin(s);
-  if (!in_args) {
-    PF_HIP(hipMemcpyAsync(slab->dev, slab->host, head_bytes, hipMemcpyHostToDevice, s));
+  // The tables go ahead of a save's gather and of zero-copy launches.  A load that
+  // begins with a link copy needs them behind it, with the visiting orders.
+  uint64_t uploaded = 0;
+  auto upload_through = [&](uint64_t end) -> int {
+    const uint64_t first = uploaded;
+    uploaded = std::max(uploaded, end);
+    return SlabPool::upload(slab, first, end, s);
+  };
+  if (!in_args && (save || !plans[unit_refs[0].plan].staged)) {
+    st = upload_through(head_bytes);
+    if (st != PF_OK) return st;
   }
   // Sorting the ids of a long list takes the submitting thread about a
   // millisecond per 64 Ki ids: do it while the first unit's link copy runs.
-  bool orders_pending = order_bytes != 0;
-  auto upload_orders = [&]() -> int {
-    if (!orders_pending) return PF_OK;
-    orders_pending = false;
+  auto upload_rest = [&]() -> int {
+    if (uploaded == slab_bytes) return PF_OK;
     for (const LayerPlan& p : plans) {
       if (p.order_owner) {
         uint32_t* order = reinterpret_cast<uint32_t*>(slab_host + p.order_slab_off);
@@ -1220,9 +1235,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         }
       }
     }
-    PF_HIP(hipMemcpyAsync(reinterpret_cast<void*>(slab_dev + head_bytes), slab_host + head_bytes,
-                          order_bytes, hipMemcpyHostToDevice, s));
-    return PF_OK;
+    return upload_through(slab_bytes);
   };
   // With kernel timing on, the DMA copies run on the caller's stream too, so
   // that every timed kernel executes alone (a measurement mode: no overlap).
@@ -1251,7 +1264,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     return PF_OK;
   };
 
-  bool one_launch = false;  // the call is a single zero-copy launch
+  bool one_result = false;  // the call is a single zero-copy launch, or a save of one fill
   size_t ui = 0;
   while (ui < unit_refs.size()) {
     const LayerPlan& p = plans[unit_refs[ui].plan];
@@ -1277,8 +1290,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       }
       if (st != PF_OK) return st;
       ++prof_.zero_copy_launches;
-      one_launch = ui == 0 && uj == unit_refs.size();
-      if (!one_launch) prof_mark_first(s);
+      one_result = ui == 0 && uj == unit_refs.size();
+      if (!one_result) prof_mark_first(s);
       st = fire_events_through(plans[unit_refs[uj - 1].plan].src_index, s);
       if (st != PF_OK) return st;
       ui = uj;
@@ -1444,7 +1457,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (st != PF_OK) return st;
       st = slot_end(sl, side, side == s);
       if (st != PF_OK) return st;
-      prof_mark_first(side);
+      one_result = ui == 0 && ue == unit_refs.size();
+      if (!one_result) prof_mark_first(side);
       if (fire_through != UINT64_MAX) {
         st = fire_events_through(fire_through, side);
         if (st != PF_OK) return st;
@@ -1455,7 +1469,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       st = link_copies(false);
       if (st != PF_OK) return st;
       prof_mark_first(side);
-      st = upload_orders();
+      st = upload_rest();
       if (st != PF_OK) return st;
       st = slot_ready(sl, side, s);
       if (st != PF_OK) return st;
@@ -1478,18 +1492,20 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     PF_HIP(hipEventRecord(join_, side));
     PF_HIP(hipStreamWaitEvent(s, join_, 0));
   }
-  st = slots_in_order_end(s);
-  if (st != PF_OK) return st;
   // Trailing empty layers.
   if (want_events && events_fired < n_layers) {
     st = fire_events_through(n_layers - 1, s);
     if (st != PF_OK) return st;
   }
+  // Whoever waits for the call waits for this marker, not for those of the slots and
+  // of the slab behind it.
+  prof_mark_end(s, one_result);
+  st = slots_in_order_end(s);
+  if (st != PF_OK) return st;
   if (!in_args) {
     st = slabs_.release_after(slab, s);
     if (st != PF_OK) return st;
   }
-  prof_mark_end(s, one_launch);
   prof_.enqueue_ms += ms_since(t_enqueue);
   return PF_OK;
 }

@@ -276,8 +276,9 @@ class Xfer {
   }
   // Three timing events bracket the device side of the calls of a profile
   // window (begin, first slot ready, end); off unless enabled.  A marker behind a
-  // kernel is ~4.5 us on the queue, so a call of one launch gets one: its end is
-  // the first result as well, and whoever waits for the call waits for it.
+  // kernel is ~4.5 us on the queue, so a call of one launch, or a save of one fill,
+  // gets one: its end is the first result as well, and whoever waits for the call
+  // waits for it.
   int enable_profile();
   void reset_profile() {
     prof_ = XferProfile();
@@ -391,9 +392,9 @@ class Xfer {
   void prof_mark_first(hipStream_t s) {
     if (profiling_ && !prof_first_set_) prof_first_set_ = hipEventRecord(prof_first_, s) == hipSuccess;
   }
-  void prof_mark_end(hipStream_t s, bool one_launch) {
+  void prof_mark_end(hipStream_t s, bool one_result) {
     if (!profiling_) return;
-    prof_end_is_first_ = one_launch && !prof_first_set_;
+    prof_end_is_first_ = one_result && !prof_first_set_;
     prof_end_set_ = hipEventRecord(prof_end_is_first_ ? prof_first_ : prof_end_, s) == hipSuccess;
     if (prof_end_is_first_) prof_first_set_ = prof_end_set_;
   }

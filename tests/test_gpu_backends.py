@@ -207,6 +207,33 @@ def test_shuffled_4k_fragments(backends, stream, n):
     host.close()
 
 
+@pytest.mark.parametrize("n", [4096, 4097, 10923, 43690, 43691])
+def test_descriptor_tables_of_every_way_to_the_device(backends, stream, n):
+    """Tables of 24-byte rows: read in host memory up to 96 KiB, uploaded by one step
+    of the upload kernel, by several, to its last MiB and by a copy beyond."""
+    from pegaflow_amd.transfer import desc_array
+    rng = np.random.default_rng(n)
+    order = rng.permutation(n).astype(np.uint64)
+    host, dev = PinnedMemory(32 * n), DeviceBuffer(16 * n)
+    data = random_bytes(rng, 16 * n)
+    at = np.arange(n, dtype=np.uint64)
+    for b in backends:  # every other 16 bytes of the host side: nothing merges, no run is packed
+        descs = desc_array(dev.ptr + order * 16, host.host_ptr + at * 32, host.device_ptr + at * 32, 16)
+        dev.copy_from_host(data)
+        host.as_numpy()[:] = 0
+        b.d2h(descs, stream)
+        stream.synchronize()
+        want = np.zeros((n, 2, 16), dtype=np.uint8)
+        want[:, 0] = data.reshape(n, 16)[order.astype(np.int64)]
+        assert np.array_equal(host.as_numpy().reshape(n, 2, 16), want), b.name
+        dev.fill(0)
+        b.h2d(descs, stream)
+        stream.synchronize()
+        assert np.array_equal(dev.copy_to_host(), data), b.name
+    dev.close()
+    host.close()
+
+
 def test_few_large_descriptors_spread_over_tiles(backends, stream):
     """A batch of two large copies (one with a 48-byte tail): the kernel
     backend splits each descriptor over many workgroups."""
