@@ -13,6 +13,8 @@
 //     for units cut into chunks (block_chunks_unit).
 #include "pf_kernels.hpp"
 
+#include <hip/hip_ext.h>
+
 #include <mutex>
 #include <type_traits>
 
@@ -813,24 +815,32 @@ dim3 block_units_grid(uint32_t n_units, uint64_t max_tiles, uint32_t max_workgro
 }
 }  // namespace
 
+namespace {
+// A zero-copy launch; its dispatch completes `stop`, with no barrier behind it.
+template <typename... Params>
+hipError_t launch_units(void (*kernel)(Params...), dim3 grid, hipStream_t s, hipEvent_t stop,
+                        Params... params) {
+  const void* address = reinterpret_cast<const void*>(kernel);
+  void* args[] = {&params...};
+  const dim3 block(kLanes, 1, 1);
+  return stop != nullptr ? hipExtLaunchKernel(address, grid, block, args, 0, s, nullptr, stop, 0)
+                         : hipLaunchKernel(address, grid, block, args, 0, s);
+}
+}  // namespace
+
 int launch_block_units(const BlockUnit* units, uint32_t n_units, uint64_t max_tiles, bool to_far,
-                       int unroll, uint32_t max_workgroups_x, hipStream_t s) {
+                       int unroll, uint32_t max_workgroups_x, hipStream_t s, hipEvent_t stop) {
   if (n_units == 0 || max_tiles == 0) return PF_OK;
   if (max_tiles > 0x7FFFFFFFull) {
     return fail(PF_ERR_INVALID_ARGUMENT, "unit of %llu tiles exceeds the kernel limit",
                 static_cast<unsigned long long>(max_tiles));
   }
   const dim3 grid = block_units_grid(n_units, max_tiles, max_workgroups_x);
-  dim3 block(kLanes, 1, 1);
-#define PF_LAUNCH_UNITS(U_)                                                                   \
-  case U_:                                                                                    \
-    if (to_far) {                                                                             \
-      hipLaunchKernelGGL((block_units_kernel<U_, true>), grid, block, 0, s, units, n_units,   \
-                         grid.x, grid.y);                                                     \
-    } else {                                                                                  \
-      hipLaunchKernelGGL((block_units_kernel<U_, false>), grid, block, 0, s, units, n_units,  \
-                         grid.x, grid.y);                                                     \
-    }                                                                                         \
+  hipError_t e = hipSuccess;
+#define PF_LAUNCH_UNITS(U_)                                                                    \
+  case U_:                                                                                     \
+    e = launch_units(to_far ? block_units_kernel<U_, true> : block_units_kernel<U_, false>,    \
+                     grid, s, stop, units, n_units, grid.x, grid.y);                          \
     break;
   switch (unroll) {
     PF_LAUNCH_UNITS(1)
@@ -841,30 +851,24 @@ int launch_block_units(const BlockUnit* units, uint32_t n_units, uint64_t max_ti
       return fail(PF_ERR_INVALID_ARGUMENT, "unsupported tile unroll %d", unroll);
   }
 #undef PF_LAUNCH_UNITS
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "block_units_kernel launch");
   return PF_OK;
 }
 
 int launch_block_units_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
                             uint64_t max_tiles, bool to_far, int unroll, uint32_t max_workgroups_x,
-                            hipStream_t s) {
+                            hipStream_t s, hipEvent_t stop) {
   if (n_units == 0 || max_tiles == 0) return PF_OK;
   if (max_tiles > 0x7FFFFFFFull) {
     return fail(PF_ERR_INVALID_ARGUMENT, "unit of %llu tiles exceeds the kernel limit",
                 static_cast<unsigned long long>(max_tiles));
   }
   const dim3 grid = block_units_grid(n_units, max_tiles, max_workgroups_x);
-  dim3 block(kLanes, 1, 1);
-#define PF_LAUNCH_ARGS(U_)                                                                       \
-  case U_:                                                                                       \
-    if (to_far) {                                                                                \
-      hipLaunchKernelGGL((block_units_args_kernel<U_, true>), grid, block, 0, s, slab,           \
-                         first_unit, n_units, grid.x, grid.y);                                   \
-    } else {                                                                                     \
-      hipLaunchKernelGGL((block_units_args_kernel<U_, false>), grid, block, 0, s, slab,          \
-                         first_unit, n_units, grid.x, grid.y);                                   \
-    }                                                                                            \
+  hipError_t e = hipSuccess;
+#define PF_LAUNCH_ARGS(U_)                                                                             \
+  case U_:                                                                                             \
+    e = launch_units(to_far ? block_units_args_kernel<U_, true> : block_units_args_kernel<U_, false>,  \
+                     grid, s, stop, slab, first_unit, n_units, grid.x, grid.y);                       \
     break;
   switch (unroll) {
     PF_LAUNCH_ARGS(1)
@@ -875,7 +879,6 @@ int launch_block_units_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n
       return fail(PF_ERR_INVALID_ARGUMENT, "unsupported tile unroll %d", unroll);
   }
 #undef PF_LAUNCH_ARGS
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail_hip(e, "block_units_args_kernel launch");
   return PF_OK;
 }

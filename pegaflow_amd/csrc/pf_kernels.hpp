@@ -61,10 +61,12 @@ bool unroll_supported(int unroll);
 // `max_workgroups_x` (0 = no cap) is the number of workgroups of the launch.
 // With units of at least that many tiles there is one row of workgroups: all of
 // them walk the units in order and stride over each unit's tiles.  Smaller
-// units get several rows, each walking every rows-th unit.
+// units get several rows, each walking every rows-th unit.  `stop`: null, or the event
+// that the launch itself completes (a marker recorded behind it is a command of its own).
 // to_far: true = gather near -> far (save), false = scatter far -> near (load).
 int launch_block_units(const BlockUnit* units, uint32_t n_units, uint64_t max_tiles, bool to_far,
-                       int unroll, uint32_t max_workgroups_x, hipStream_t s);
+                       int unroll, uint32_t max_workgroups_x, hipStream_t s,
+                       hipEvent_t stop = nullptr);
 
 // A slab small enough to travel in the arguments of a launch (the limit for all
 // arguments of a kernel is 4 KiB): units first, then id lists and page tables,
@@ -76,7 +78,7 @@ struct ArgSlab {
 // Units [first_unit, first_unit + n_units) of the slab.
 int launch_block_units_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
                             uint64_t max_tiles, bool to_far, int unroll, uint32_t max_workgroups_x,
-                            hipStream_t s);
+                            hipStream_t s, hipEvent_t stop = nullptr);
 
 // Limits of one block_tiles launch (grid.y and grid.z are 16-bit).
 constexpr uint32_t kMaxTileBlocks = 65535;

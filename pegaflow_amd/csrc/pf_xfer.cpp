@@ -114,9 +114,10 @@ int Xfer::reserve_staging() {
 
 int Xfer::enable_profile() {
   if (profiling_) return PF_OK;
-  PF_HIP(hipEventCreate(&prof_begin_));
-  PF_HIP(hipEventCreate(&prof_first_));
-  PF_HIP(hipEventCreate(&prof_end_));
+  // Whoever waits for one of these reads host memory that kernels have written.
+  for (hipEvent_t* e : {&prof_begin_, &prof_first_, &prof_end_}) {
+    PF_HIP(hipEventCreateWithFlags(e, hipEventReleaseToSystem));
+  }
   profiling_ = true;
   return PF_OK;
 }
@@ -218,22 +219,22 @@ int Xfer::timing_end(hipStream_t s) {
 }
 
 int Xfer::launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
-                         uint32_t workgroups, bool to_far, hipStream_t s) {
+                         uint32_t workgroups, bool to_far, hipStream_t s, hipEvent_t stop) {
   int st = timing_begin(s);
   if (st != PF_OK) return st;
   st = launch_block_units(dev_units, n_units, max_tiles, to_far, unroll_,
-                          workgroups, s);
+                          workgroups, s, stop);
   if (st != PF_OK) return st;
   return timing_end(s);
 }
 
 int Xfer::launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
                               uint64_t max_tiles, uint32_t workgroups, bool to_far,
-                              hipStream_t s) {
+                              hipStream_t s, hipEvent_t stop) {
   int st = timing_begin(s);
   if (st != PF_OK) return st;
   st = launch_block_units_args(slab, first_unit, n_units, max_tiles, to_far, unroll_,
-                               workgroups, s);
+                               workgroups, s, stop);
   if (st != PF_OK) return st;
   return timing_end(s);
 }
@@ -1211,6 +1212,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   prof_.plan_ms += ms_since(t_call) - (prof_.staging_alloc_ms - alloc_before);
   const Clock::time_point t_enqueue = Clock::now();
   prof_mark_begin(s);
+  // A call of one zero-copy launch takes its end from the launch.
+  const bool single_launch = all_zero_copy && !want_events;
   // The tables go ahead of a save's gather and of zero-copy launches.  A load that
   // begins with a link copy needs them behind it, with the visiting orders.
   uint64_t uploaded = 0;
@@ -1264,7 +1267,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     return PF_OK;
   };
 
-  bool one_result = false;  // the call is a single zero-copy launch, or a save of one fill
+  bool one_result = false;  // the call is a save of one fill
   size_t ui = 0;
   while (ui < unit_refs.size()) {
     const LayerPlan& p = plans[unit_refs[ui].plan];
@@ -1281,17 +1284,21 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
           ++uj;
         }
       }
+      hipEvent_t stop = single_launch ? prof_launch_end() : nullptr;
       if (in_args) {
         st = launch_strided_args(arg_slab, static_cast<uint32_t>(ui), static_cast<uint32_t>(uj - ui),
-                                 max_tiles, workgroups, save, s);
+                                 max_tiles, workgroups, save, s, stop);
       } else {
         st = launch_strided(units_dev + ui, static_cast<uint32_t>(uj - ui), max_tiles, workgroups,
-                            save, s);
+                            save, s, stop);
       }
       if (st != PF_OK) return st;
       ++prof_.zero_copy_launches;
-      one_result = ui == 0 && uj == unit_refs.size();
-      if (!one_result) prof_mark_first(s);
+      if (single_launch) {
+        prof_launch_marked();
+      } else {
+        prof_mark_first(s);
+      }
       st = fire_events_through(plans[unit_refs[uj - 1].plan].src_index, s);
       if (st != PF_OK) return st;
       ui = uj;
@@ -1499,7 +1506,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   }
   // Whoever waits for the call waits for this marker, not for those of the slots and
   // of the slab behind it.
-  prof_mark_end(s, one_result);
+  if (!single_launch) prof_mark_end(s, one_result);
   st = slots_in_order_end(s);
   if (st != PF_OK) return st;
   if (!in_args) {

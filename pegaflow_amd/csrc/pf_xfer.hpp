@@ -275,10 +275,10 @@ class Xfer {
     return total;
   }
   // Three timing events bracket the device side of the calls of a profile
-  // window (begin, first slot ready, end); off unless enabled.  A marker behind a
-  // kernel is ~4.5 us on the queue, so a call of one launch, or a save of one fill,
-  // gets one: its end is the first result as well, and whoever waits for the call
-  // waits for it.
+  // window (begin, first slot ready, end); off unless enabled.  A marker is a command
+  // of its own, ~4.5 us behind a kernel: a save of one fill gets one, whose end is the
+  // first result as well, and the end of a call of one launch is
+  // that of the launch.  Whoever waits for the call waits for its end.
   int enable_profile();
   void reset_profile() {
     prof_ = XferProfile();
@@ -321,7 +321,7 @@ class Xfer {
   int slots_in_order_end(hipStream_t s);
   // Zero-copy form: grid-stride kernel over `n_units` units, capped grid.
   int launch_strided(const BlockUnit* dev_units, uint32_t n_units, uint64_t max_tiles,
-                     uint32_t workgroups, bool to_far, hipStream_t s);
+                     uint32_t workgroups, bool to_far, hipStream_t s, hipEvent_t stop);
   // Workgroups that a zero-copy unit asks its launch for.
   uint32_t zero_copy_workgroups(const BlockUnit& u, bool save) const {
     if (zc_max_wg_ != 0) return zc_max_wg_;
@@ -330,7 +330,8 @@ class Xfer {
   }
   // The same with the slab in the launch's arguments (short lists).
   int launch_strided_args(const ArgSlab& slab, uint32_t first_unit, uint32_t n_units,
-                          uint64_t max_tiles, uint32_t workgroups, bool to_far, hipStream_t s);
+                          uint64_t max_tiles, uint32_t workgroups, bool to_far, hipStream_t s,
+                          hipEvent_t stop);
   // Staged form: one tile per workgroup over one unit.
   int launch_tiles(const BlockUnit& host_unit, bool to_far, hipStream_t s, const LinkShare& share);
   int timing_begin(hipStream_t s);
@@ -391,6 +392,17 @@ class Xfer {
   }
   void prof_mark_first(hipStream_t s) {
     if (profiling_ && !prof_first_set_) prof_first_set_ = hipEventRecord(prof_first_, s) == hipSuccess;
+  }
+  // The event that the launch of a call of one launch completes: its end is the first
+  // result as well, where no call of the window had one before.  (The launch could
+  // take its start along, too, but then it takes the submitting thread 14 us longer.)
+  hipEvent_t prof_launch_end() const {
+    return !profiling_ ? nullptr : prof_first_set_ ? prof_end_ : prof_first_;
+  }
+  void prof_launch_marked() {
+    if (!profiling_) return;
+    prof_end_is_first_ = !prof_first_set_;
+    prof_first_set_ = prof_end_set_ = true;
   }
   void prof_mark_end(hipStream_t s, bool one_result) {
     if (!profiling_) return;
