@@ -59,6 +59,30 @@ constexpr uint32_t chunks_per_fragment(uint64_t frag, uint64_t n_blocks, bool al
   return static_cast<uint32_t>(chunks);
 }
 
+// A segment whose host image is one gapless range is cut along the link's packets
+// of 256 bytes instead (kUnitLines): chunk c is what lies of the range in the 16
+// bytes from 16 c - lead on, `lead` being the range's start modulo 256; the chunks
+// that stick out are shifted inwards.  A chunk may hold the end of one fragment and
+// the head of the next, `tail` being the bytes of the first (16: all).  Needs
+// frag >= 16 and a range of at most kMaxLinesRange (the starts of a whole last tile
+// stay in 32 bits).
+constexpr uint64_t kMaxLinesRange = 0xFFFFFFFFull - (64 << 10);
+constexpr uint32_t kLinkPacket = 256;
+constexpr uint32_t line_chunk_count(uint32_t range) { return (range + (kLinkPacket - 1) + 15u) >> 4; }
+struct LineChunk {
+  uint32_t start;  // in the range
+  uint32_t pos;    // list position of its first byte
+  uint32_t tail;
+  bool any;        // something of the range lies in it
+};
+constexpr LineChunk line_chunk(uint32_t c, uint32_t lead, uint32_t range, uint32_t frag) {
+  const uint32_t raw = 16u * c;
+  const uint32_t in = raw > lead ? raw - lead : 0u;
+  const uint32_t start = in < range - 16u ? in : range - 16u;
+  const uint32_t pos = start / frag;
+  const uint32_t left = (pos + 1) * frag - start;
+  return {start, pos, left < 16u ? left : 16u, raw + 16u > lead && in < range};
+}
 // Workgroups that a unit of a zero-copy launch needs to keep the link full: of
 // full tiles `full_tiles`, more of smaller ones, at most `most`.  Saves and units
 // in chunks take a whole multiple for every started share of a tile; a load of

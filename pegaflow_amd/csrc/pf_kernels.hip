@@ -407,7 +407,8 @@ __device__ __forceinline__ UnitFields unit_fields(UnitPtr up, uint64_t bias) {
 // workgroups, saved / loaded in 477 / 501, in turn in 450 / 451).  Units in chunks
 // of which more than `most_odd` tiles are left after whole rounds stay at workgroup
 // 0: 16 layers of 777 blocks of 1000 bytes (96 tiles, 64 workgroups) loaded in 458
-// us, in turn in 464.
+// us, in turn in 464.  Units cut along the link's packets always pass it (the same
+// saved in 452 us, with every unit beginning at workgroup 0 in 463).
 struct RowTurn {
   uint32_t at = 0;  // workgroup whose turn it is
   __device__ __forceinline__ uint32_t take(uint32_t n_tiles, uint32_t wg, uint32_t grid_x,
@@ -511,6 +512,75 @@ __device__ __forceinline__ void block_chunks_unit(const UnitFields& f, uint32_t 
   }
 }
 
+// Saves of fragments off the 16-byte grid into a host image without gaps, cut along
+// the link's packets (line_chunk): every wavefront writes whole ones, and a chunk that
+// holds the end of one fragment and the head of the next is put together from both.
+// With chunks of one fragment (block_chunks_unit) both ends of a fragment share a
+// packet with a neighbour, and the link carries its parts one by one.  Measured on
+// MI355X, GB/s queued, chunks of one fragment, along lines of 64 bytes, along packets
+// of 256: 16 layers of 1000-byte fragments, 25 MB, 52.3 / 55.0 / 55.8, 600 bytes 50.5 /
+// 53.9 / 54.7, 4100 bytes 53.7 / 55.2 / 55.9, 40 004 bytes (32 workgroups) 53.3 / 55.4 /
+// 55.9; 2 MB of 516 bytes 43.2 / 51.7 / 52.1, of 20 bytes 17.4 / 40.2 / 40.4.  Loads gain
+// nothing by it (25 MB of 1000 bytes 451 us either way, 1 MB 26.4 instead of 23.9): both
+// parts of a shared packet are read anyway, and the chunks of two fragments have to be
+// stored in pieces.
+template <int U>
+__device__ __forceinline__ void block_lines_unit(const UnitFields& f, uint32_t grid_x, RowTurn& turn) {
+  typedef unsigned __int128 u128;
+  const uint32_t frag = static_cast<uint32_t>(f.frag_bytes);
+  const uint32_t range = f.n_blocks * frag;  // the host keeps it within kMaxLinesRange
+  const uint32_t n_chunks = line_chunk_count(range);
+  const uint32_t tiles_per_seg = (n_chunks + U * kLanes - 1) / (U * kLanes);
+  const uint32_t n_tiles = tiles_per_seg * f.n_seg;
+  for (uint32_t t = turn.take(n_tiles, blockIdx.x, grid_x, grid_x); t < n_tiles; t += grid_x) {
+    const uint32_t seg = t >= tiles_per_seg ? 1u : 0u;
+    const uint32_t first = (seg ? t - tiles_per_seg : t) * (U * kLanes) + threadIdx.x;
+    const uint64_t near_seg = f.near_base + (seg ? f.kv_stride : 0);
+    const uint64_t far_seg = seg ? f.far_base1 : f.far_base0;
+    const uint32_t lead = static_cast<uint32_t>(far_seg) & (kLinkPacket - 1);
+    const __amdgpu_buffer_rsrc_t image = tile_descriptor(far_seg, range);
+    const uint32_t left = n_chunks - (first - threadIdx.x);  // > 0
+    with_steps<U>(min(wave_steps<kLanes>(left, threadIdx.x), static_cast<uint32_t>(U)), [&](auto steps) {
+      constexpr int K = decltype(steps)::value;
+      LineChunk c[K];
+      uint32_t word[K], next_word[K];
+      u32x4 v[K], w[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        c[k] = line_chunk(first + k * kLanes, lead, range, frag);
+        word[k] = f.ids[f.ids16 ? c[k].pos >> 1 : c[k].pos];
+        next_word[k] = 0;
+        if (c[k].tail < 16) next_word[k] = f.ids[f.ids16 ? (c[k].pos + 1) >> 1 : c[k].pos + 1];
+      }
+      auto near_of = [&](uint32_t pos, uint32_t id_word) {
+        const uint64_t id = f.ids16 ? ((pos & 1u) ? id_word >> 16 : id_word & 0xFFFFu) : id_word;
+        return near_seg + id * f.block_stride;
+      };
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t at = c[k].tail < 16 ? frag - 16u : c[k].start - c[k].pos * frag;
+        v[k] = load16_any(near_of(c[k].pos, word[k]) + at);
+        w[k] = v[k];
+        if (c[k].tail < 16) w[k] = load16_any(near_of(c[k].pos + 1, next_word[k]));
+      }
+      wait_for_loads();
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (c[k].tail < 16) {
+          v[k] = __builtin_bit_cast(u32x4, (__builtin_bit_cast(u128, v[k]) >> (8 * (16 - c[k].tail))) |
+                                               (__builtin_bit_cast(u128, w[k]) << (8 * c[k].tail)));
+        }
+        if (!c[k].any) continue;
+        if (((lead + c[k].start) & 15u) == 0) {
+          store16_sc1_nt(image, c[k].start, v[k]);
+        } else {
+          store16_any(far_seg + c[k].start, v[k]);
+        }
+      }
+    });
+  }
+}
+
 // The tiles of a unit over mapped host memory, by workgroup `wg` of the `grid_x` of
 // its row.  VEC_ONLY: the unit is known to be of the form kUnitVec, with one range
 // of host memory per segment and 32-bit ids.
@@ -576,6 +646,12 @@ __device__ __forceinline__ void block_units_body(UnitPtr units, uint32_t n_units
     if (f.form == kUnitChunks) {
       block_chunks_unit<U, TO_FAR>(f, grid_x, turn);
       continue;
+    }
+    if constexpr (TO_FAR) {
+      if (f.form == kUnitLines) {
+        block_lines_unit<U>(f, grid_x, turn);
+        continue;
+      }
     }
     unit_tiles<U, kLanes, TO_FAR, false>(f, turn, blockIdx.x, grid_x);
   }

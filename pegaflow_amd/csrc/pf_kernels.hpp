@@ -48,6 +48,7 @@ enum UnitForm : uint32_t {
   kUnitAny = 0,     // tiles of one fragment, no alignment assumed
   kUnitVec = 1,     // tiles of one fragment, every address and stride 16-byte aligned
   kUnitChunks = 2,  // zero-copy only: 16-byte chunks of consecutive fragments share a tile
+  kUnitLines = 3,   // zero-copy saves into gapless ranges: chunks along the link's packets (line_chunk)
 };
 
 // Bytes one workgroup moves per tile for the given unroll (256 lanes x 16 B x U).

@@ -1156,7 +1156,9 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
           u.frag_bytes, u.n_blocks, p.vec_ok, save,
           p.page_dev ? 1 : u.far_stride | u.far_base[0] | u.far_base[1], span);
       if (chunks != 0) {
-        u.form = kUnitChunks;
+        // Gapless images of a save take chunks along the link's packets.
+        const bool lines = save && !p.vec_ok && p.dense && span <= kMaxLinesRange;
+        u.form = lines ? kUnitLines : kUnitChunks;
         u.tiles_per_frag = chunks;
       }
     }
@@ -1252,9 +1254,11 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     return PF_OK;
   };
   auto tiles_of = [&](const BlockUnit& u) -> uint64_t {
-    const uint64_t per_seg = static_cast<uint64_t>(u.n_blocks) * u.tiles_per_frag;
+    uint64_t per_seg = static_cast<uint64_t>(u.n_blocks) * u.tiles_per_frag;
     const uint64_t chunks_per_tile = tile / 16;
-    return (u.form == kUnitChunks ? (per_seg + chunks_per_tile - 1) / chunks_per_tile : per_seg) * u.n_seg;
+    if (u.form == kUnitLines) per_seg = line_chunk_count(u.n_blocks * static_cast<uint32_t>(u.frag_bytes));
+    const bool whole_tiles = u.form == kUnitVec || u.form == kUnitAny;
+    return (whole_tiles ? per_seg : (per_seg + chunks_per_tile - 1) / chunks_per_tile) * u.n_seg;
   };
   // Skipped (empty) layers fire their event at the position of the next
   // planned layer; track the caller index we have fired up to.

@@ -1142,3 +1142,41 @@ def test_share_of_the_link_matches_oracle(name, copy_stream, stream):
         pool.close()
         for c in cases:
             c.close()
+
+
+@pytest.mark.parametrize("seg", [16, 17, 23, 31, 36, 100, 1000, 1016, 4097, 20004])
+def test_gapless_images_off_the_grid_match_oracle(seg, xfer, stream):
+    """Zero-copy saves into gapless images that begin anywhere in a 256-byte packet of the
+    link (chunks along the packets) and their loads: one block, a few, a list that travels
+    as 16-bit ids (1001), the lists of two tiles and a bit; bytes around the image."""
+    rng = np.random.default_rng(seg)
+    for n, segments, lead in [(1, 1, 0), (1, 2, 255), (2, 2, 17), (3, 1, 48), (67, 2, 1), (1001, 1, 136),
+                              (33000 // seg + 2, 2, 36), (33000 // seg + 2, 1, 199)]:
+        case = Case(rng, num_blocks=n + 5, seg=seg, segments=segments, n_ids=n, base_off=4 if lead & 1 else 0)
+        pool = PinnedMemory(4096 + segments * n * seg)
+        at = 1024 + lead
+        layer = _dense_layer(case, case.product_layout(), pool, case.ids)
+        layer.host = tuple(h + at for h in layer.host)
+        layer.host_device = tuple(h + at for h in layer.host_device)
+        try:
+            case.dev.copy_from_host(case.cache0)
+            pool.as_numpy()[:] = SENT
+            xfer.save([layer], stream, ZC)
+            stream.synchronize()
+            want = np.full(pool.as_numpy().size, SENT, dtype=np.uint8)
+            segs = [want[at + s * n * seg: at + (s + 1) * n * seg] for s in range(2)]
+            cache = case.cache0.copy()
+            O.transfer_layer(case.oracle_layout(cache), case.ids, segs[0], segs[1] if segments == 2 else None,
+                             host_is_src=False)
+            assert np.array_equal(pool.as_numpy(), want), (n, segments, lead)
+            layer.block_ids = rng.choice(case.num_blocks, n, replace=False).astype(np.uint32)
+            case.dev.fill(SENT)
+            xfer.load([layer], stream, ZC)
+            stream.synchronize()
+            cache = np.full_like(case.cache0, SENT)
+            O.transfer_layer(case.oracle_layout(cache), layer.block_ids, segs[0], segs[1] if segments == 2 else None,
+                             host_is_src=True)
+            assert np.array_equal(case.dev.copy_to_host(), cache), (n, segments, lead)
+        finally:
+            case.close()
+            pool.close()
