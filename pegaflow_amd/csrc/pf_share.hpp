@@ -18,7 +18,9 @@ namespace pf {
 // MI355X, calls back to back, save / load in us without a share, with b / 58 and
 // with this: one layer of 20 MB 393.7 / 398.7, 390.4 / 393.2, 390.2 / 392.5; 105 MB
 // in two 1904 / 1899, 1881 / 1868, 1876 / 1868; 524 MB in twelve 9432 / 9406, 9313 /
-// 9248, 9240 / 9230.
+// 9248, 9240 / 9230.  Link copies on a stream of their own run under the launches as
+// it is: there a share only adds a third user of the link (a save and a load at once
+// fell from 88 to 35 GB/s together in one repetition of nine).
 constexpr uint64_t kShareBase = 64 << 10;
 constexpr uint64_t kSharePart = 44;
 constexpr uint64_t link_share_bytes(uint64_t launch_bytes) {

@@ -536,7 +536,10 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     int st = ensure_slot(sl, max_chunk_bytes);
     if (st != PF_OK) return st;
   }
-  // The last pages of a chunk are its share of the link (pf_share.hpp).
+  // The last pages of a chunk are its share of the link (pf_share.hpp), where the
+  // link copies take turns with the launches.
+  const bool on_side = use_side_stream(chunks.size(), n * pack.page_bytes);
+  may_share = may_share && !on_side;
   std::vector<uint64_t> shared_pages(chunks.size(), 0);
   uint64_t min_frag = UINT64_MAX;
   for (const LayerPlan& p : plans) {
@@ -637,7 +640,6 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   }
 
   // Before anything of this call is on `s`: the check wants the stream idle.
-  const bool on_side = use_side_stream(chunks.size(), n * pack.page_bytes);
   if (on_side) {
     const int side_status = ensure_side_stream(s);
     if (side_status != PF_OK) return side_status;
@@ -923,9 +925,16 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (plans[u.layer].staged) plans[u.layer].units.emplace_back(u.first, u.count);
     }
   }
+  // A second stream pays off when the link copies of one fill can overlap the
+  // gather of the next: count the fills.
+  size_t fills = 0;
+  for (size_t ge : group_end) fills += ge != 0 ? 1 : 0;
+  uint64_t staged_bytes = 0;
+  for (const LayerPlan& p : plans) staged_bytes += p.staged ? p.layer_bytes : 0;
+  const bool on_side = use_side_stream(fills, staged_bytes);
   // The share of every fill that crosses the link with its launch (pf_share.hpp),
-  // by the fill's first unit.  Calls that asked for the staged path keep every byte
-  // on it.
+  // by the fill's first unit.  Not where the link copies run beside the launches
+  // anyway, and calls that asked for the staged path keep every byte on it.
   struct FillShare {
     size_t staged_end = 0;      // one past the last unit of which a part takes the slot
     uint64_t staged_frags = 0;  // fragments of that last unit in the slot
@@ -944,7 +953,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       max_blocks = std::max(max_blocks, unit_refs[k].count);
     }
     sh.staged_frags = unit_refs[sh.staged_end - 1].count * plans[unit_refs[sh.staged_end - 1].plan].n_seg;
-    if (path != PF_PATH_AUTO || max_blocks > kMaxSharedTileBlocks) continue;
+    if (path != PF_PATH_AUTO || on_side || max_blocks > kMaxSharedTileBlocks) continue;
     const ShareCut cut = plan_link_share(sh.staged_end - ui, link_share_bytes(fill_bytes), [&](size_t k) {
       const LayerPlan& p = plans[unit_refs[ui + k].plan];
       return ShareUnit{unit_refs[ui + k].count, p.n_seg, p.frag_bytes, p.vec_ok};
@@ -1198,13 +1207,6 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
   }
 
   // ---- 4. enqueue ---------------------------------------------------------
-  // A second stream pays off when the link copies of one fill can overlap the
-  // gather of the next: count the fills.
-  size_t fills = 0;
-  for (size_t ge : group_end) fills += ge != 0 ? 1 : 0;
-  uint64_t staged_bytes = 0;
-  for (const LayerPlan& p : plans) staged_bytes += p.staged ? p.layer_bytes : 0;
-  const bool on_side = use_side_stream(fills, staged_bytes);
   // Before anything of this call is on `s`: the check wants the stream idle.
   if (on_side) {
     const int side_status = ensure_side_stream(s);
