@@ -201,6 +201,7 @@ class SealedBlock {
   size_t num_slots() const { return image_ ? image_->num_slots() : slots_.size(); }
   const SaveImage* image() const { return image_.get(); }  // null: a list of slots
   uint32_t position() const { return position_; }
+  long image_owners() const { return image_.use_count(); }  // blocks of the save still about
 
  private:
   std::vector<RawBlock> slots_;

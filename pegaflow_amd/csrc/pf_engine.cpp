@@ -393,17 +393,25 @@ Engine::SealedEntry* Engine::find_sealed(uint32_t ns, std::string_view hash, uin
   return it == sealed_.end() ? nullptr : &it->second;
 }
 
-bool Engine::evict_one() {
+size_t Engine::evict(bool all) {
   // mu_ held by the caller.  Least recently used first; blocks that are
   // leased or being loaded (someone else holds a reference) stay.
-  for (SealedEntry* e = lru_.newer; e != &lru_; e = e->newer) {
-    if (e->block.use_count() > 1) continue;
-    lru_unlink(e);
-    auto it = sealed_.find(*e->key);
-    if (it != sealed_.end()) sealed_.erase(it);
-    return true;
+  size_t gone = 0;
+  for (SealedEntry* e = lru_.newer; e != &lru_;) {
+    SealedEntry* next = e->newer;
+    if (e->block.use_count() == 1) {
+      // The buffers of a save go with the last of its blocks: until then there is
+      // no more room than before, and the caller need not try.
+      const bool gives_back = e->block->image() == nullptr || e->block->image_owners() == 1;
+      lru_unlink(e);
+      auto it = sealed_.find(*e->key);
+      if (it != sealed_.end()) sealed_.erase(it);
+      ++gone;
+      if (gives_back && !all) break;
+    }
+    e = next;
   }
-  return false;
+  return gone;
 }
 
 size_t Engine::sweep_expired_locked() {
@@ -435,7 +443,7 @@ std::shared_ptr<PinnedAllocation> Engine::allocate(uint64_t size, NumaNode numa)
   for (;;) {
     if (auto a = pool_->allocate(size, numa)) return a;
     std::lock_guard<std::mutex> lock(mu_);
-    if (evict_one()) continue;
+    if (evict(false) != 0) continue;
     // Nothing evictable is left: blocks pinned by leases whose time is up
     // (a worker that died between query and load) are given back first.
     if (swept || sweep_expired_locked() == 0) return nullptr;
@@ -472,9 +480,7 @@ size_t Engine::gc_stale_inflight(std::chrono::milliseconds max_age) {
 
 size_t Engine::evict_all() {
   std::lock_guard<std::mutex> lock(mu_);
-  size_t n = 0;
-  while (evict_one()) ++n;
-  return n;
+  return evict(true);
 }
 
 // offload.rs:182-282.

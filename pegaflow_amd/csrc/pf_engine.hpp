@@ -190,7 +190,8 @@ class Engine {
   std::shared_ptr<InstanceContext> get_instance(const std::string& id, std::string* err);
   // storage/mod.rs:294-330: allocate, evicting oldest sealed blocks on pressure.
   std::shared_ptr<PinnedAllocation> allocate(uint64_t size, NumaNode numa);
-  bool evict_one();
+  // Drop blocks until some memory is given back, or all that can go; how many went.
+  size_t evict(bool all);
   int alloc_page_first_targets(const LayerTopology& topo, struct SaveLayerCtx* ctxs, size_t n,
                                NumaNode numa, std::vector<std::shared_ptr<PinnedAllocation>>* pages,
                                std::vector<LayerTransferData>* out, std::string* err);

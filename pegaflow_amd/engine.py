@@ -16,6 +16,11 @@ from . import _lib
 from ._lib import check
 from .transfer import LayerTransferData, TransferMode
 
+try:
+    from . import _calls  # built beside libpegahip.so (csrc/py/pf_calls.cpp)
+except ImportError as exc:
+    raise ImportError(f"pegaflow_amd/_calls.so is missing: build it with `make -C pegaflow_amd/csrc` ({exc})") from exc
+
 LOAD_STATE_PENDING = 0
 LOAD_STATE_SUCCESS = 1
 LOAD_STATE_ERROR = -1
@@ -62,6 +67,9 @@ TASK_PATH_NAMES = ((_lib.PF_TASK_PATH_STAGED, "staged"), (_lib.PF_TASK_PATH_ZERO
                    (_lib.PF_TASK_PATH_DESCRIPTORS, "descriptors"))
 
 
+PHASES = ("resolve", "queue", "convert", "plan", "staging_alloc", "enqueue", "sync", "device_first", "device")
+
+
 @dataclass
 class TaskResult:
     """What a settled task reports: bytes and duration (what the reference's
@@ -86,6 +94,22 @@ class TaskResult:
                    tuple(name for bit, name in TASK_PATH_NAMES if r.paths & bit),
                    r.staged_groups, r.zero_copy_launches, r.link_copies, phases)
 
+    @classmethod
+    def from_call(cls, done, nbytes, elapsed_ms, paths, staged_groups, zero_copy_launches, link_copies,
+                  phases) -> "TaskResult":
+        return cls(bool(done), nbytes, elapsed_ms, tuple(name for bit, name in TASK_PATH_NAMES if paths & bit),
+                   staged_groups, zero_copy_launches, link_copies, dict(zip(PHASES, phases)))
+
+
+_addresses = {}
+
+
+def _address(name: str) -> int:
+    """Address of a function of the library, for `_calls`."""
+    if name not in _addresses:
+        _addresses[name] = C.cast(getattr(_lib.load(), name), C.c_void_p).value
+    return _addresses[name]
+
 
 class Task:
     """A submitted load or save; ``wait`` raises if the task failed."""
@@ -96,6 +120,11 @@ class Task:
         self._keep = keep
 
     def wait(self, timeout_ms: int = -1) -> TaskResult:
+        made = _calls.wait(_address("pf_task_wait"), _handle(self), timeout_ms)
+        if made is not None:
+            status, *fields = made
+            check(status)
+            return TaskResult.from_call(*fields)
         r = _lib.PfTaskResult()
         check(self._lib.pf_task_wait(self.handle, timeout_ms, C.byref(r)))
         return TaskResult.from_c(r)
@@ -110,6 +139,11 @@ class Task:
             self.close()
         except Exception:
             pass
+
+
+def _handle(owner) -> int:
+    """The handle of an open engine or task as `_calls` takes it; 0 when it is closed."""
+    return (owner.handle.value or 0) if owner.handle is not None else 0
 
 
 def _pack_layer_transfers(layers: Sequence[LayerTransferData]):
@@ -358,12 +392,21 @@ class PegaEngine:
 
     def batch_save_kv_blocks(self, instance_id: str, tp_rank: int, pp_rank: int, device_id: int,
                              saves: Sequence[LayerSave] | PackedSaves) -> None:
+        status = _calls.save(_address("pf_engine_batch_save"), _handle(self), instance_id, tp_rank, pp_rank,
+                             device_id, saves)
+        if status is not None:
+            check(status)
+            return
         packed = saves if isinstance(saves, PackedSaves) else PackedSaves(saves)
         check(self._lib.pf_engine_batch_save(self.handle, instance_id.encode(), tp_rank, pp_rank,
                                              device_id, packed.array, packed.n))
 
     def query_prefix(self, instance_id: str, hashes: Sequence[bytes]) -> tuple[int, int]:
         """-> (hit blocks, lease id); lease 0 when nothing hit."""
+        made = _calls.query(_address("pf_engine_query_prefix"), _handle(self), instance_id, hashes)
+        if made is not None:
+            check(made[0])
+            return made[1], made[2]
         ptrs, lens, _bufs = _pack_hashes(hashes)
         hits, lease = C.c_uint64(), C.c_uint64()
         check(self._lib.pf_engine_query_prefix(self.handle, instance_id.encode(), ptrs, lens,
@@ -377,6 +420,12 @@ class PegaEngine:
                                          layer_groups: Sequence[Sequence[str]], lease: int,
                                          dest_block_ids_by_group: Sequence[Sequence[int | None]],
                                          load_state: LoadState | None = None) -> Task:
+        shm = load_state.shm_name if load_state is not None else None
+        made = _calls.load(_address("pf_engine_batch_load"), _handle(self), instance_id, tp_rank, device_id,
+                           layer_groups, lease, dest_block_ids_by_group, shm)
+        if made is not None:
+            check(made[0])
+            return Task(C.c_void_p(made[1]))
         g = len(layer_groups)
         keep = []
         group_ptrs = (C.POINTER(C.c_char_p) * max(g, 1))()
@@ -395,10 +444,9 @@ class PegaEngine:
             dests[i], owner = _pack_destinations(ids)
             keep.append(owner)
         t = C.c_void_p()
-        shm = load_state.shm_name.encode() if load_state is not None else None
         check(self._lib.pf_engine_batch_load(self.handle, instance_id.encode(), tp_rank, device_id,
-                                             g, group_ptrs, sizes, lease, dests, n_blocks, shm,
-                                             C.byref(t)))
+                                             g, group_ptrs, sizes, lease, dests, n_blocks,
+                                             shm.encode() if shm is not None else None, C.byref(t)))
         return Task(t, keep)
 
     def query_group_membership(self, instance_id: str, group: int,

@@ -1,0 +1,205 @@
+"""The engine's calls through pegaflow_amd._calls against the ctypes packing of the
+same arguments: what reaches the C function, for every form a caller may use.  The
+functions called are recorders of the test's own; no library, no GPU."""
+
+import ctypes as C
+import dataclasses
+
+import numpy as np
+import pytest
+
+from pegaflow_amd import _calls, _lib
+from pegaflow_amd import engine as E
+
+P8, P32, P64, PI64 = (C.POINTER(t) for t in (C.c_uint8, C.c_uint32, C.c_uint64, C.c_int64))
+SAVE = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_char_p, C.c_uint64, C.c_uint64, C.c_int, C.POINTER(_lib.PfLayerSave),
+                   C.c_uint64)
+QUERY = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_char_p, C.POINTER(P8), P32, C.c_uint64, P64, P64)
+LOAD = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_char_p, C.c_uint64, C.c_int, C.c_uint64, C.POINTER(C.POINTER(C.c_char_p)),
+                   P64, C.c_uint64, C.POINTER(PI64), C.c_uint64, C.c_char_p, C.POINTER(C.c_void_p))
+WAIT = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int, C.POINTER(_lib.PfTaskResult))
+
+
+def address(fn):
+    return C.cast(fn, C.c_void_p).value
+
+
+def hashes_at(ptrs, lens, n):
+    return [C.string_at(ptrs[i], lens[i]) for i in range(n)]
+
+
+class Bytes(bytes):
+    pass
+
+
+class Name(str):
+    pass
+
+
+HASHES = [[], [b"a"], (b"ab", b"", bytes(range(40))), [b"x" * 32] * 5]
+ODD_HASHES = [[bytearray(b"ab")], [b"a", Bytes(b"b")], iter([b"a"]), [memoryview(b"abc")], np.array([b"a"]), ["a"],
+              [b"a", None], None]
+
+
+@pytest.mark.parametrize("hashes", HASHES + ODD_HASHES, ids=lambda h: type(h).__name__)
+def test_query(hashes):
+    seen = []
+
+    def fn(engine, instance, ptrs, lens, n, hits, lease):
+        seen.append((engine, instance, hashes_at(ptrs, lens, n)))
+        hits[0], lease[0] = 7, 2**63 + 1
+        return 0
+
+    made = _calls.query(address(QUERY(fn)), 0x1234, "inst", hashes)
+    if any(hashes is h for h in ODD_HASHES):
+        assert made is None and not seen
+        return
+    assert made == (0, 7, 2**63 + 1)
+    ptrs, lens, _keep = E._pack_hashes(hashes)
+    assert seen == [(0x1234, b"inst", hashes_at(ptrs, lens, len(hashes)))] == [(0x1234, b"inst", list(hashes))]
+
+
+@dataclasses.dataclass
+class Odd:
+    layer_name: object
+    block_ids: object
+    block_hashes: object
+
+
+def _saves():
+    ids, hashes = [4, 0, 2**64 - 1], [b"h0", b"h1", b"h2" * 20]
+    return {
+        "one": [E.LayerSave("l0", ids, hashes)],
+        "shared": [E.LayerSave(f"läyer.{i}", ids, hashes) for i in range(40)],
+        "own": tuple(E.LayerSave(f"l{i}", [i, i + 1], (b"%d" % i, b"x")) for i in range(12)),
+        "mixed": [E.LayerSave("a", ids, hashes), E.LayerSave("b", (1,), [b"q"]), E.LayerSave("c", ids, hashes)],
+        "empty": [],
+        "no_blocks": [E.LayerSave("l", [], []), E.LayerSave("m", (), ())],
+    }
+
+
+def _odd_saves():
+    h = [b"h"]
+    return {
+        "array": [E.LayerSave("l", np.array([3]), h)],
+        "length": [E.LayerSave("l", [1, 2], h)],
+        "negative": [E.LayerSave("l", [-1], h)],
+        "large": [E.LayerSave("l", [2**64], h)],
+        "bool": [E.LayerSave("l", [True], h)],
+        "float": [E.LayerSave("l", [1.0], h)],
+        "later": [E.LayerSave("l", [1], h), E.LayerSave("l", [None], h)],
+        "name": [E.LayerSave(Name("l"), [1], h)],
+        "surrogate": [E.LayerSave("\ud800", [1], h)],
+        "hashes": [E.LayerSave("l", [1], [Bytes(b"h")])],
+        "no_attributes": [object()],
+        "generator": (s for s in _saves()["one"]),
+        "packed": E.PackedSaves(_saves()["one"]),
+    }
+
+
+def _record_saves(seen):
+    def fn(engine, instance, tp, pp, device, layers, n):
+        rows = [(layers[i].layer_name, layers[i].block_ids[:layers[i].n_blocks],
+                 hashes_at(layers[i].block_hashes, layers[i].block_hash_lens, layers[i].n_blocks),
+                 bool(layers[i].block_ids), bool(layers[i].block_hashes), bool(layers[i].block_hash_lens))
+                for i in range(n)]
+        seen.append((engine, instance, tp, pp, device, rows))
+        return 3
+    return SAVE(fn)
+
+
+@pytest.mark.parametrize("name", sorted(_saves()))
+def test_save(name):
+    saves, seen = _saves()[name], []
+    fn = _record_saves(seen)
+    assert _calls.save(address(fn), 5, "inst", 1, 2, 3, saves) == 3
+    packed = E.PackedSaves(saves)
+    assert fn(5, b"inst", 1, 2, 3, packed.array, packed.n) == 3
+    assert seen[0] == seen[1] and len(seen[0][5]) == len(saves)
+
+
+@pytest.mark.parametrize("name", sorted(_odd_saves()))
+def test_saves_left_to_ctypes(name):
+    seen = []
+    fn = _record_saves(seen)
+    assert _calls.save(address(fn), 5, "inst", 1, 2, 3, _odd_saves()[name]) is None and not seen
+    assert _calls.save(address(fn), 5, "inst", np.int64(1), 2, 3, _saves()["one"]) is None and not seen
+
+
+def test_saves_that_change_while_they_are_read():
+    ids, hashes, seen = [1, 2], [b"a", b"b"], []
+
+    class Grows:
+        layer_name = "l"
+        block_hashes = hashes
+
+        @property
+        def block_ids(self):
+            saves.append(self)
+            return ids
+
+    class Empties(Grows):
+        @property
+        def block_ids(self):
+            saves.clear()
+            return ids
+
+    fn = _record_saves(seen)
+    saves = [Grows()]
+    assert _calls.save(address(fn), 5, "inst", 0, 0, 0, saves) == 3 and len(seen[0][5]) == 1
+    saves = [Empties(), Empties()]
+    assert _calls.save(address(fn), 5, "inst", 0, 0, 0, saves) is None and len(seen) == 1
+
+
+def _record_loads(seen):
+    def fn(engine, instance, tp, device, groups, names, sizes, lease, dests, n, shm, task):
+        seen.append((engine, instance, tp, device, [[names[g][i] for i in range(sizes[g])] for g in range(groups)],
+                     lease, [dests[g][:n] for g in range(groups)], shm))
+        task[0] = 0xABCDEF
+        return 0
+    return LOAD(fn)
+
+
+@pytest.mark.parametrize("dests", [[[]], [[3]], [(3, None, 5)], [[None, None], [-7, 2**63 - 1]],
+                                   [[1, 2], (3, None), [9, 9]]], ids=str)
+@pytest.mark.parametrize("shm", [None, "pega_load_1"])
+def test_load(dests, shm):
+    groups = [["a", "lé"], ("b",), []][:len(dests)]
+    seen = []
+    fn = _record_loads(seen)
+    assert _calls.load(address(fn), 9, "inst", 1, 2, groups, 2**64 - 3, dests, shm) == (0, 0xABCDEF)
+    want = [[-1 if v is None else v for v in d] for d in dests]
+    assert seen == [(9, b"inst", 1, 2, [[n.encode() for n in g] for g in groups], 2**64 - 3, want,
+                     shm.encode() if shm else None)]
+    for d, w in zip(dests, want):
+        packed, _owner = E._pack_destinations(d)
+        assert [packed[i] for i in range(len(w))] == w
+
+
+@pytest.mark.parametrize("groups, dests", [
+    ([], []), ([["a"]], []), ([["a"]], [[1.0]]), ([["a"]], [[True]]), ([["a"]], [np.array([1])]),
+    ([["a"]], [[2**63]]), ([["a"], ["b"]], [[1], [1, 2]]), ([[Name("a")]], [[1]]), ([[b"a"]], [[1]]), (["a"], [[1]]),
+    ([["a"]], [range(3)]), ([["a"]], [None])], ids=str)
+def test_loads_left_to_ctypes(groups, dests):
+    seen = []
+    assert _calls.load(address(_record_loads(seen)), 9, "inst", 1, 2, groups, 4, dests, None) is None and not seen
+
+
+@pytest.mark.parametrize("status, timeout", [(0, -1), (2, 50)])
+def test_wait(status, timeout):
+    seen = []
+
+    def fn(task, timeout_ms, out):
+        seen.append((task, timeout_ms))
+        for i, (field, ctype) in enumerate(_lib.PfTaskResult._fields_):
+            setattr(out[0], field, ctype(i + 1).value)
+        out[0].paths = 5
+        return status
+
+    made = _calls.wait(address(WAIT(fn)), 77, timeout)
+    r = _lib.PfTaskResult()
+    assert fn(77, timeout, C.pointer(r)) == status
+    assert made[0] == status and seen == [(77, timeout)] * 2
+    assert E.TaskResult.from_call(*made[1:]) == E.TaskResult.from_c(r)
+    assert _calls.wait(address(WAIT(fn)), 77, 1.5) is None
+    assert _calls.wait(0, 77, 1) is None
