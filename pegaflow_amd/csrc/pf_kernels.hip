@@ -752,7 +752,7 @@ __device__ __forceinline__ bool link_share(const LinkShare& share, uint32_t plan
   constexpr int kUnroll = kShareTileBytes / (LT * 16);
   RowTurn turn;
   for (uint32_t k = 0; k < share.n_units; ++k) {
-    unit_tiles<kUnroll, LT, TO_FAR, true>(unit_fields(share.units + k, 0), turn, wg, share.workgroups);
+    unit_tiles<kUnroll, LT, TO_FAR, true>(unit_fields(share.units + k, 0), turn, share.first + wg, share.all);
   }
   return true;
 }

@@ -93,7 +93,11 @@ constexpr uint32_t kMaxTileUnits = 32767;
 struct LinkShare {
   const BlockUnit* units = nullptr;
   uint32_t n_units = 0;
-  uint32_t workgroups = 0;  // 0 = nothing to move
+  uint32_t workgroups = 0;  // of this launch; 0 = nothing to move
+  // A fill that goes out as several launches spreads its share over them: this launch
+  // has the workgroups from `first` on of `all`.
+  uint32_t first = 0;
+  uint32_t all = 0;
 };
 // Positions a unit of a launch with a share may have: the share's workgroups are
 // rows or planes of the same grid.

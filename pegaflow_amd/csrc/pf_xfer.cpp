@@ -665,7 +665,8 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
     // With the first launch of a chunk, that of the largest slices.
     LinkShare share;
     if (shared_pages[ci] != 0) {
-      share = {units_dev + n_units + ci * n_plans, static_cast<uint32_t>(n_plans), share_workgroups(min_frag, save)};
+      const uint32_t groups = share_workgroups(min_frag, save);
+      share = {units_dev + n_units + ci * n_plans, static_cast<uint32_t>(n_plans), groups, 0, groups};
     }
     auto launch = [&](bool to_far) -> int {
       int rc = timing_begin(s);
@@ -1317,7 +1318,8 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     const size_t ue = group_end[ui];
     const FillShare& fill_share = shares[ui];
     const size_t us = fill_share.staged_end;
-    const LinkShare share{units_dev + unit_refs.size() + fill_share.first, fill_share.count, fill_share.workgroups};
+    const LinkShare share{units_dev + unit_refs.size() + fill_share.first, fill_share.count,
+                          fill_share.workgroups, 0, fill_share.workgroups};
     Slot& sl = slots_[unit_slot[ui]];
     // The link copies of the group, coalesced: pieces that follow one another
     // both in staging and in the host image cross as one copy (a copy costs
@@ -1398,8 +1400,7 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
         size_t begin, end;
       };
       std::vector<Run> runs;
-      uint64_t runs_started = 0, most_tiles = 0;
-      size_t largest_run = 0;  // carries the share
+      uint64_t runs_started = 0;
       for (size_t k = ui; k < us;) {
         size_t e = k;
         uint64_t run_useful = 0, run_rows = 0, run_tiles = 0, run_seg = 0;
@@ -1416,10 +1417,6 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
           run_seg = ns;
           ++e;
         }
-        if (run_useful > most_tiles) {
-          most_tiles = run_useful;
-          largest_run = runs.size();
-        }
         runs.push_back({k, e});
         runs_started += run_rows * run_tiles * run_seg;
         k = e;
@@ -1434,9 +1431,13 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
       if (in_runs) {
         for (size_t ri = 0; ri < runs.size(); ++ri) {
           const Run& run = runs[ri];
+          // (The runs of a fill are of a size: eight units each, most of the time.)
+          LinkShare part = share;
+          part.first = static_cast<uint32_t>(ri) * share.workgroups;
+          part.all = static_cast<uint32_t>(runs.size()) * share.workgroups;
           rc = launch_block_tiles_rows(units_dev + run.begin, units_host + run.begin,
                                        static_cast<uint32_t>(run.end - run.begin), to_far, s,
-                                       &launched, ri == largest_run ? share : LinkShare());
+                                       &launched, part);
           if (rc != PF_OK) return rc;
           // (Only a launch beyond the grid limits is refused; what went out
           // before it is then simply done again by the form below.)
