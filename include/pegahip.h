@@ -334,8 +334,9 @@ typedef struct pf_xfer_config {
                                        1,2,4,8; 0 = default (4) */
   uint32_t copy_stream;             /* staged path: where the link copies run.
                                        0 = default (side stream when a call has more than
-                                       one staging fill and they hold 64 MiB or more each
-                                       on average), 1 = a side stream of the engine (the
+                                       one staging fill, they hold 64 MiB or more each on
+                                       average and their launches cannot carry a share of the
+                                       link: PF_PATH_STAGED, fragments off the 16-byte grid), 1 = a side stream of the engine (the
                                        copy of one unit overlaps the gather of the next),
                                        2 = the caller's stream (in order, no second queue) */
   uint64_t auto_staged_min_call_bytes; /* PF_PATH_AUTO also stages every dense layer (of 32 KiB or

@@ -377,7 +377,9 @@ class Xfer {
   // / 54.5 against 54.5 / 53.9; 8 saves of 21 MB 33.7 / 51.7 against 52.4 /
   // 51.8; 6 loads of 64 MB 55.4 / 55.2 against 55.2 / 54.9; 4 of 131 MB 56.0 /
   // 55.9 against 55.6 / 55.5.  So calls of smaller fills go in order: alone they
-  // give up at most 1 % by it, back to back they gain a fifth and more.
+  // give up at most 1 % by it, back to back they gain a fifth and more.  (Of the
+  // others only those go to the side stream whose launches cannot have a share of
+  // the link, see run_impl.)
   bool use_side_stream(size_t fills, uint64_t staged_bytes) const {
     if ((timing_ && !timing_in_place_) || copy_stream_ == 2) return false;
     if (copy_stream_ == 1) return true;
