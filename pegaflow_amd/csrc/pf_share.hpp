@@ -12,17 +12,18 @@ namespace pf {
 // therefore also moves a share of the fill straight between the cache and host
 // memory, with a few workgroups of its own, and the link copy is shorter by it.  A
 // launch of b bytes takes 4-6 us and b / 3.05 TB/s, in which the link moves b / 53
-// and 250-350 KB; with a little more than the first and less than the second the
-// share ends with the launch at every size.  (A longer share gains nothing: the
-// launch then waits for it instead of the link copy for the launch.)  Measured on
-// MI355X, calls back to back, save / load in us without a share, with b / 58 and
-// with this: one layer of 20 MB 393.7 / 398.7, 390.4 / 393.2, 390.2 / 392.5; 105 MB
-// in two 1904 / 1899, 1881 / 1868, 1876 / 1868; 524 MB in twelve 9432 / 9406, 9313 /
-// 9248, 9240 / 9230.  Link copies on a stream of their own run under the launches as
-// it is: there a share only adds a third user of the link (a save and a load at once
-// fell from 88 to 35 GB/s together in one repetition of nine).
+// and 250-350 KB: the share ends with the launch of a full slot and a little before
+// that of a small one.  (A longer share gains nothing: the launch then waits for it
+// instead of the link copy for the launch.)  Measured on MI355X, calls back to back,
+// save / load in us without a share, with 64 KiB and b / 44, b / 52, b / 60: one layer
+// of 20 MB 393.9 / 395.6, 390.5 / 389.4, 390.1 / 388.9, 389.9 / 389.0; 524 MB in twelve
+// 9437 / 9409, 9247 / 9194, 9254 / 9228, 9277 / 9252; 1.3 GB in four 23 352 / 23 223,
+// 23 106 / 23 001, 23 107 / 23 004, 23 135 / 23 053.  Link copies on a stream of their
+// own run under the launches as it is: there a share only adds a third user of the
+// link (a save and a load at once fell from 88 to 35 GB/s together in one repetition
+// of nine).
 constexpr uint64_t kShareBase = 64 << 10;
-constexpr uint64_t kSharePart = 44;
+constexpr uint64_t kSharePart = 52;
 constexpr uint64_t link_share_bytes(uint64_t launch_bytes) {
   return kShareBase + launch_bytes / kSharePart;
 }
