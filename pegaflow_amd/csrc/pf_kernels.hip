@@ -1297,7 +1297,8 @@ template <bool HOST_IS_SRC>
 void launch_packing(const uint64_t* table, uint64_t n, uint64_t n_link, uint64_t max_size,
                     uint32_t link_workgroups, hipStream_t s, uint32_t max_workgroups) {
   const RowsGrid g = rows_grid(n, max_size, max_workgroups);
-  const uint32_t link_groups = n_link == 0 ? 0 : (link_workgroups + g.y - 1) / g.y;
+  // (Rows of the share are a tile at most: those of the grid's first layer move it.)
+  const uint32_t link_groups = n_link == 0 ? 0 : link_workgroups;
   const dim3 grid(g.x + link_groups, g.y, 1), block(kLanes, 1, 1);
   const Rows3<true> rows{table};
   const Rows3<false> link{table + 3 * n};

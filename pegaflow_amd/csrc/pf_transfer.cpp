@@ -26,6 +26,39 @@ static uint32_t host_link_workgroups(uint64_t total_bytes, uint64_t n) {
   return static_cast<uint32_t>(scaled < 64 ? scaled : 64);
 }
 
+// Rows of a launch over mapped host memory are cut into pieces of this size (0: left
+// whole) where they are of unlike length and the longest is a good part of what one
+// workgroup has to move: a workgroup takes whole rows, and the last long one would
+// have the link to itself.  Ranges that merge into runs of 1 to 64 fragments are like
+// that (direct backend, out and back in us: 67 fragments of 93 754 bytes 443 -> 247,
+// 600 of 16 KiB 414 -> 367, 1302 of 4 KiB 240 -> 206).  Rows of one length are balanced
+// well enough as long as half of the workgroups keep the link busy, and cutting them
+// costs a row to fetch per piece (40 rows of 128 KiB 197 -> 204).
+constexpr uint64_t kLinkTile = 16384;
+static uint64_t link_row_piece(uint64_t total_bytes, uint64_t n, uint64_t max_size, uint32_t workgroups) {
+  constexpr uint64_t kPiecesPerWorkgroup = 16, kMostTiles = 16;
+  if (max_size <= kLinkTile || n == 0 || max_size <= 2 * (total_bytes / n) ||
+      max_size * 4 <= total_bytes / workgroups) {
+    return 0;
+  }
+  const uint64_t tiles = total_bytes / (workgroups * kPiecesPerWorkgroup) / kLinkTile;
+  return kLinkTile * std::clamp<uint64_t>(tiles, 1, kMostTiles);
+}
+static uint64_t pieces_of(uint64_t size, uint64_t piece) {
+  return piece == 0 || size <= piece ? 1 : (size + piece - 1) / piece;
+}
+// Writes the piece(s) of one row; returns the row behind them.
+static uint64_t write_row(uint64_t* table, uint64_t row, uint64_t dst, uint64_t src, uint64_t size,
+                          uint64_t piece) {
+  const uint64_t n = pieces_of(size, piece);
+  for (uint64_t k = 0; k < n; ++k, ++row) {
+    table[3 * row + 0] = dst + k * piece;
+    table[3 * row + 1] = src + k * piece;
+    table[3 * row + 2] = k + 1 < n ? piece : size - k * piece;
+  }
+  return row;
+}
+
 // ---------------------------------------------------------------------------
 // merge
 // ---------------------------------------------------------------------------
@@ -304,7 +337,8 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     uint64_t bytes;
     std::vector<uint32_t> members;  // indices into `ranges`
     size_t packed = 0;              // members that go through staging; the others are
-    uint64_t link_bytes = 0;        // the packing launch's share of the link (pf_share.hpp)
+    uint64_t link_bytes = 0;        // the packing launch's share of the link (pf_share.hpp),
+    uint64_t link_rows = 0;         // in rows of a tile
   };
   std::vector<Run> runs;
   std::vector<std::pair<uint64_t, size_t>> open;  // host allocation -> index of its open run
@@ -341,7 +375,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       if (open.size() >= 64) open.erase(open.begin());  // bound the linear search
       open.emplace_back(r.host_allocation, runs.size());
     }
-    runs.push_back(Run{r.host, r.size, {static_cast<uint32_t>(i)}, 0, 0});
+    runs.push_back(Run{r.host, r.size, {static_cast<uint32_t>(i)}, 0, 0, 0});
   }
   std::vector<uint32_t> isolated;
   bool isolated_mapped = true;
@@ -357,7 +391,6 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       isolated.push_back(run.members[0]);
       isolated_mapped = isolated_mapped && ranges[run.members[0]].host_device != 0;
     } else {
-      staged_pieces += run.members.size();
       max_run_bytes = std::max(max_run_bytes, run.bytes + 16);
       for (uint32_t m : run.members) max_staged_piece = std::max(max_staged_piece, ranges[m].size);
       const ShareCut cut = plan_link_share(run.members.size(), link_share_bytes(run.bytes), [&](size_t k) {
@@ -366,6 +399,10 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       });
       run.packed = cut.unit;
       run.link_bytes = cut.bytes;
+      for (size_t k = run.packed; k < run.members.size(); ++k) {
+        run.link_rows += pieces_of(ranges[run.members[k]].size, kLinkTile);
+      }
+      staged_pieces += run.packed + run.link_rows;
     }
   }
   const bool isolated_by_kernel = isolated_mapped && isolated.size() > kFewRanges;
@@ -383,7 +420,18 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       if (e != hipSuccess) return fail_hip(e, what);
     }
   }
-  const uint64_t table_rows = staged_pieces + (isolated_by_kernel ? isolated.size() : 0);
+  uint64_t isolated_rows = 0, max_isolated = 0, isolated_bytes = 0, isolated_piece = 0;
+  uint32_t isolated_workgroups = 0;
+  if (isolated_by_kernel) {
+    for (uint32_t i : isolated) {
+      max_isolated = std::max(max_isolated, ranges[i].size);
+      isolated_bytes += ranges[i].size;
+    }
+    isolated_workgroups = host_link_workgroups(isolated_bytes, isolated.size());
+    isolated_piece = link_row_piece(isolated_bytes, isolated.size(), max_isolated, isolated_workgroups);
+    for (uint32_t i : isolated) isolated_rows += pieces_of(ranges[i].size, isolated_piece);
+  }
+  const uint64_t table_rows = staged_pieces + isolated_rows;
   if (table_rows == 0) return PF_OK;
   if (table_rows > 0x7FFFFFFFull) {
     return fail(PF_ERR_INVALID_ARGUMENT, "descriptor batch of %llu exceeds the kernel limit",
@@ -423,16 +471,11 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
   const uint64_t* table_dev = static_cast<const uint64_t*>(slab->dev);
   uint64_t row = 0;
   // Rows of the isolated ranges first, then run by run.
-  uint64_t max_isolated = 0, isolated_bytes = 0;
   if (isolated_by_kernel) {
     for (uint32_t i : isolated) {
       const Range& r = ranges[i];
-      table[3 * row + 0] = host_is_src ? r.device : r.host_device;
-      table[3 * row + 1] = host_is_src ? r.host_device : r.device;
-      table[3 * row + 2] = r.size;
-      max_isolated = std::max(max_isolated, r.size);
-      isolated_bytes += r.size;
-      ++row;
+      row = write_row(table, row, host_is_src ? r.device : r.host_device, host_is_src ? r.host_device : r.device,
+                      r.size, isolated_piece);
     }
   }
   const uint64_t staging_base = reinterpret_cast<uint64_t>(staging_);
@@ -445,10 +488,8 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       const Range& r = ranges[run.members[k]];
       const uint64_t far = k < run.packed ? staging_base + pad + static_cast<uint64_t>(r.host - run.host_begin)
                                           : r.host_device;
-      table[3 * row + 0] = host_is_src ? r.device : far;
-      table[3 * row + 1] = host_is_src ? far : r.device;
-      table[3 * row + 2] = r.size;
-      ++row;
+      row = write_row(table, row, host_is_src ? r.device : far, host_is_src ? far : r.device, r.size,
+                      k < run.packed ? 0 : kLinkTile);
     }
   }
   // A short table of ranges that all go through the mapped-memory kernel is
@@ -468,10 +509,10 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
   if (isolated_by_kernel) {
     st = upload_table();
     if (st != PF_OK) return st;
-    st = launch_desc_copy(table_dev, isolated.size(), max_isolated, host_is_src, s,
-                          host_link_workgroups(isolated_bytes, isolated.size()));
+    st = launch_desc_copy(table_dev, isolated_rows, isolated_piece ? isolated_piece : max_isolated, host_is_src, s,
+                          isolated_workgroups);
     if (st != PF_OK) return st;
-    row = isolated.size();
+    row = isolated_rows;
   }
   // One staging buffer, everything in stream order: pack, then copy (save),
   // or copy, then unpack (load); the next run waits for the previous one.
@@ -489,7 +530,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
     // Many pieces of at most one tile: two rows per workgroup, so that the second
     // row's descriptor is on its way while the first is copied (65 536 pieces of
     // 4 KiB: 92 us instead of 98).
-    const uint64_t pieces = run.packed, shared = run.members.size() - run.packed;
+    const uint64_t pieces = run.packed, shared = run.link_rows;
     const uint32_t pack_workgroups =
         max_staged_piece <= 16384 && pieces >= 8192 ? static_cast<uint32_t>((pieces + 1) / 2) : 0;
     st = launch_desc_pack(table_dev + 3 * row, pieces, shared, max_staged_piece, host_is_src, s,
@@ -499,7 +540,7 @@ int MemcpyBackend::submit_piece(const CopyDesc* copies, uint64_t n, bool host_is
       PF_HIP(hipMemcpyDtoHAsync(run.host_begin, reinterpret_cast<hipDeviceptr_t>(in_staging),
                                 run.bytes - run.link_bytes, s));
     }
-    row += run.members.size();
+    row += pieces + shared;
   }
   if (staged_pieces != 0) {
     PF_HIP(hipEventRecord(staging_done_, s));
@@ -524,11 +565,6 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
     return fail(PF_ERR_INVALID_ARGUMENT, "descriptor batch of %llu exceeds the kernel limit",
                 static_cast<unsigned long long>(n));
   }
-  const uint64_t bytes = n * 3 * sizeof(uint64_t);
-  SlabPool::Slab* slab = nullptr;
-  int st = slabs_.acquire(bytes, &slab);
-  if (st != PF_OK) return st;
-  uint64_t* table = static_cast<uint64_t*>(slab->host);
   uint64_t max_size = 0, total_size = 0;
   for (uint64_t i = 0; i < n; ++i) {
     const CopyDesc& c = copies[i];
@@ -540,10 +576,29 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
                   "device-visible host address",
                   static_cast<unsigned long long>(i));
     }
-    table[3 * i + 0] = host_is_src ? c.device : c.host_device;
-    table[3 * i + 1] = host_is_src ? c.host_device : c.device;
-    table[3 * i + 2] = c.size;
     max_size = std::max<uint64_t>(max_size, c.size);
+  }
+  const uint32_t workgroups = host_link_workgroups(total_size, n);
+  const uint64_t piece = link_row_piece(total_size, n, max_size, workgroups);
+  uint64_t rows = n;
+  if (piece != 0) {
+    rows = 0;
+    for (uint64_t i = 0; i < n; ++i) rows += pieces_of(copies[i].size, piece);
+    if (rows > 0x7FFFFFFFull) {
+      return fail(PF_ERR_INVALID_ARGUMENT, "descriptor batch of %llu bytes exceeds the kernel limit",
+                  static_cast<unsigned long long>(total_size));
+    }
+  }
+  const uint64_t bytes = rows * 3 * sizeof(uint64_t);
+  SlabPool::Slab* slab = nullptr;
+  int st = slabs_.acquire(bytes, &slab);
+  if (st != PF_OK) return st;
+  uint64_t* table = static_cast<uint64_t*>(slab->host);
+  uint64_t row = 0;
+  for (uint64_t i = 0; i < n; ++i) {
+    const CopyDesc& c = copies[i];
+    row = write_row(table, row, host_is_src ? c.device : c.host_device, host_is_src ? c.host_device : c.device,
+                    c.size, piece);
   }
   // A short table is read where it was written, in mapped host memory: the
   // upload would cost more than the rows' trip over the link, which the kernel
@@ -555,8 +610,7 @@ int KernelBackend::submit_impl(const CopyDesc* copies, uint64_t n, bool host_is_
     st = SlabPool::upload(slab, 0, bytes, s);
     if (st != PF_OK) return st;
   }
-  st = launch_desc_copy(table_dev, n, max_size, host_is_src, s,
-                        host_link_workgroups(total_size, n));
+  st = launch_desc_copy(table_dev, rows, piece ? piece : max_size, host_is_src, s, workgroups);
   if (st != PF_OK) return st;
   return slabs_.release_after(slab, s);
 }

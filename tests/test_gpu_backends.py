@@ -530,3 +530,30 @@ def test_random_descriptor_batches_match_oracle(backends, stream, seed):
 
     for b in backends:
         _run_both_directions(b, stream, descs, dev_bytes, host_bytes, rows, seed=seed)
+
+
+@pytest.mark.parametrize("fragment, lengths, backend", [
+    (16384, [40, 1, 1, 3, 17, 2], "kernel"),                # a long row among short ones: cut into tiles
+    (93754, [30, 1, 2, 5, 1], "direct"),                    # off the grid, merged ranges of unlike length
+    (16385, [20] + [1] * 30, "direct"),                     # pieces of one byte behind whole tiles
+    (70000, [50, 1, 9] + [1, 4] * 60 + [60], "direct"),     # 21 MB: packed, the last range longer than the share
+    (40000, [3, 1] * 150, "direct"),                        # 24 MB: packed, pieces of the share among them
+])
+def test_rows_of_unlike_length_over_the_link(stream, gpu, fragment, lengths, backend):
+    from pegaflow_amd.transfer import desc_array
+    sizes = np.array(lengths, dtype=np.uint64) * np.uint64(fragment)
+    host_off = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.uint64) + np.uint64(48)
+    gap = np.uint64(80)
+    order = np.random.default_rng(fragment).permutation(len(sizes))
+    dev_off = np.zeros(len(sizes), dtype=np.uint64)
+    dev_off[order] = np.concatenate([[0], np.cumsum(sizes[order] + gap)[:-1]]).astype(np.uint64)
+    rows = [(int(d), int(h), int(s)) for d, h, s in zip(dev_off, host_off, sizes)]
+
+    def descs(dev, host):
+        return desc_array(dev.ptr + dev_off, host.host_ptr + host_off, host.device_ptr + host_off, sizes, 0, 1)
+
+    b = KernelBackend() if backend == "kernel" else MemcpyBackend()
+    try:
+        _run_both_directions(b, stream, descs, int(sizes.sum() + gap * len(sizes)), int(sizes.sum()) + 96, rows, seed=7)
+    finally:
+        b.close()
