@@ -128,6 +128,22 @@ bool begin(PyObject* const* args, Py_ssize_t n, Py_ssize_t want, Fn* fn, void** 
   return true;
 }
 
+// Runs `call` without the interpreter's lock; false, with an error set, when it threw
+// (the C functions do not, short of memory they cannot get).
+template <typename Call>
+bool unlocked(Call call) {
+  bool done = true;
+  Py_BEGIN_ALLOW_THREADS
+  try {
+    call();
+  } catch (...) {
+    done = false;
+  }
+  Py_END_ALLOW_THREADS
+  if (!done) PyErr_SetString(PyExc_RuntimeError, "the engine call threw an exception");
+  return done;
+}
+
 // save(fn, engine, instance_id, tp_rank, pp_rank, device_id, saves) -> status or None
 PyObject* save(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
   decltype(&pf_engine_batch_save) fn = nullptr;
@@ -202,10 +218,11 @@ PyObject* save(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
     layers[i] = {name, ids[a].ids.data(), hashes[b].hashes.ptrs.data(), hashes[b].hashes.lens.data(), count};
   }
   int status = 0;
-  Py_BEGIN_ALLOW_THREADS
-  status = fn(static_cast<pf_engine_t>(engine), instance, tp, pp, static_cast<int>(device), layers.data(),
-              static_cast<uint64_t>(n));
-  Py_END_ALLOW_THREADS
+  const bool done = unlocked([&] {
+    status = fn(static_cast<pf_engine_t>(engine), instance, tp, pp, static_cast<int>(device), layers.data(),
+                static_cast<uint64_t>(n));
+  });
+  if (!done) return nullptr;
   return PyLong_FromLong(status);
 } catch (const std::bad_alloc&) {
   return PyErr_NoMemory();
@@ -223,10 +240,11 @@ PyObject* query(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
   const uint64_t n = static_cast<uint64_t>(size_of(args[3]));
   uint64_t hits = 0, lease = 0;
   int status = 0;
-  Py_BEGIN_ALLOW_THREADS
-  status = fn(static_cast<pf_engine_t>(engine), instance, hashes.ptrs.data(), hashes.lens.data(), n, &hits,
-              &lease);
-  Py_END_ALLOW_THREADS
+  const bool done = unlocked([&] {
+    status = fn(static_cast<pf_engine_t>(engine), instance, hashes.ptrs.data(), hashes.lens.data(), n, &hits,
+                &lease);
+  });
+  if (!done) return nullptr;
   return Py_BuildValue("iKK", status, static_cast<unsigned long long>(hits),
                        static_cast<unsigned long long>(lease));
 } catch (const std::bad_alloc&) {
@@ -272,11 +290,12 @@ PyObject* load(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
   }
   pf_task_t task = nullptr;
   int status = 0;
-  Py_BEGIN_ALLOW_THREADS
-  status = fn(static_cast<pf_engine_t>(engine), instance, tp, static_cast<int>(device),
-              static_cast<uint64_t>(g), name_ptrs.data(), sizes.data(), lease, id_ptrs.data(),
-              static_cast<uint64_t>(n), shm, &task);
-  Py_END_ALLOW_THREADS
+  const bool done = unlocked([&] {
+    status = fn(static_cast<pf_engine_t>(engine), instance, tp, static_cast<int>(device),
+                static_cast<uint64_t>(g), name_ptrs.data(), sizes.data(), lease, id_ptrs.data(),
+                static_cast<uint64_t>(n), shm, &task);
+  });
+  if (!done) return nullptr;
   return Py_BuildValue("iK", status, static_cast<unsigned long long>(reinterpret_cast<uintptr_t>(task)));
 } catch (const std::bad_alloc&) {
   return PyErr_NoMemory();
@@ -292,9 +311,9 @@ PyObject* wait(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!begin(args, nargs, 3, &fn, &task) || !integer(args[2], &timeout)) return not_here();
   pf_task_result r = {};
   int status = 0;
-  Py_BEGIN_ALLOW_THREADS
-  status = fn(static_cast<pf_task_t>(task), static_cast<int>(timeout), &r);
-  Py_END_ALLOW_THREADS
+  if (!unlocked([&] { status = fn(static_cast<pf_task_t>(task), static_cast<int>(timeout), &r); })) {
+    return nullptr;
+  }
   return Py_BuildValue("iiKdIIII(ddddddddd)", status, r.done, static_cast<unsigned long long>(r.bytes),
                        r.elapsed_ms, r.paths, r.staged_groups, r.zero_copy_launches, r.link_copies,
                        r.resolve_ms, r.queue_ms, r.convert_ms, r.plan_ms, r.staging_alloc_ms, r.enqueue_ms,
