@@ -4,6 +4,7 @@
 #include <cstring>
 
 #include "pf_common.hpp"
+#include "pf_ranges.hpp"
 #include "pf_share.hpp"
 
 namespace pf {
@@ -233,40 +234,6 @@ MemcpyBackend::~MemcpyBackend() {
 }
 
 namespace {
-
-// A merged range that keeps what the staged forms need.
-struct Range {
-  uint64_t device;
-  uint8_t* host;
-  uint64_t host_device;
-  uint64_t size;
-  uint64_t host_allocation;
-};
-
-// The reference's merge rule (memcpy.rs:25-55), keeping the device-visible
-// host address and the host allocation of the descriptor that opened a range.
-std::vector<Range> merge_ranges(const CopyDesc* copies, uint64_t n) {
-  std::vector<Range> out;
-  out.reserve(n);
-  uint64_t run_first = 0;
-  for (uint64_t i = 0; i < n; ++i) {
-    const CopyDesc& c = copies[i];
-    if (!out.empty()) {
-      Range& run = out.back();
-      const CopyDesc& first = copies[run_first];
-      if (first.device_allocation == c.device_allocation &&
-          first.host_allocation == c.host_allocation && run.device + run.size == c.device &&
-          run.host + run.size == static_cast<uint8_t*>(c.host)) {
-        run.size += c.size;
-        continue;
-      }
-    }
-    run_first = i;
-    out.push_back({c.device, static_cast<uint8_t*>(c.host), c.host_device, c.size,
-                   c.host_allocation});
-  }
-  return out;
-}
 
 hipError_t copy_range(const Range& r, bool host_is_src, hipStream_t s) {
   return host_is_src

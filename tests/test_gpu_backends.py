@@ -408,6 +408,30 @@ def test_direct_backend_moves_the_tail_of_a_run_over_the_link(stream, gpu, size,
         b.close()
 
 
+@pytest.mark.parametrize("mapped", [(1, 0), (0, 1)], ids=["second_unmapped", "first_unmapped"])
+@pytest.mark.parametrize("pairs", [1500, 3000])
+def test_direct_backend_merges_across_mappings(stream, gpu, pairs, mapped):
+    """Descriptors that follow one another on both sides, of which one has no
+    device-visible address, below and above the 16 MiB from which runs are packed: the
+    merged range goes by its host address (pf_ranges.hpp)."""
+    from pegaflow_amd.transfer import desc_array
+    size = 4096
+    order = np.array(xorshift_shuffle(pairs), dtype=np.uint64)
+    dev_off = (order[:, None] * np.uint64(2 * size + 64) + np.array([0, size], dtype=np.uint64)).ravel()
+    host_off = np.arange(2 * pairs, dtype=np.uint64) * np.uint64(size)
+    visible = np.tile(np.array(mapped, dtype=np.uint64), pairs)
+    rows = [(int(d), int(h), size) for d, h in zip(dev_off, host_off)]
+
+    def descs(dev, host):
+        return desc_array(dev.ptr + dev_off, host.host_ptr + host_off, (host.device_ptr + host_off) * visible, size, 0, 1)
+
+    b = MemcpyBackend()
+    try:
+        _run_both_directions(b, stream, descs, pairs * (2 * size + 64), 2 * pairs * size, rows, seed=pairs)
+    finally:
+        b.close()
+
+
 def test_direct_backend_mixed_batch(stream, gpu):
     """One batch holding a large range, a host-dense run of odd-sized unaligned
     pieces, isolated small ranges without a device-visible host address (so
