@@ -13,6 +13,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <cxxabi.h>
+
 #include <cstdint>
 #include <new>
 #include <vector>
@@ -28,16 +30,21 @@ PyObject* g_block_hashes;
 // Objects that a call needs while it runs without the interpreter's lock.
 class Kept {
  public:
+  // A thread that wants the lock back from an interpreter that is ending is ended there
+  // itself, and unwound: it does not have the lock, and its objects stay.
   ~Kept() {
+    if (unlocked_) return;
     for (PyObject* o : objects_) Py_DECREF(o);
   }
   void add(PyObject* borrowed) {
     objects_.push_back(borrowed);
     Py_INCREF(borrowed);
   }
+  void set_unlocked(bool unlocked) { unlocked_ = unlocked; }
 
  private:
   std::vector<PyObject*> objects_;
+  bool unlocked_ = false;
 };
 
 bool is_sequence(PyObject* o) { return PyList_CheckExact(o) || PyTuple_CheckExact(o); }
@@ -131,15 +138,19 @@ bool begin(PyObject* const* args, Py_ssize_t n, Py_ssize_t want, Fn* fn, void** 
 // Runs `call` without the interpreter's lock; false, with an error set, when it threw
 // (the C functions do not, short of memory they cannot get).
 template <typename Call>
-bool unlocked(Call call) {
+bool unlocked(Kept& kept, Call call) {
   bool done = true;
+  kept.set_unlocked(true);
   Py_BEGIN_ALLOW_THREADS
   try {
     call();
+  } catch (const abi::__forced_unwind&) {
+    throw;  // the thread is being ended
   } catch (...) {
     done = false;
   }
   Py_END_ALLOW_THREADS
+  kept.set_unlocked(false);
   if (!done) PyErr_SetString(PyExc_RuntimeError, "the engine call threw an exception");
   return done;
 }
@@ -218,7 +229,7 @@ PyObject* save(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
     layers[i] = {name, ids[a].ids.data(), hashes[b].hashes.ptrs.data(), hashes[b].hashes.lens.data(), count};
   }
   int status = 0;
-  const bool done = unlocked([&] {
+  const bool done = unlocked(kept, [&] {
     status = fn(static_cast<pf_engine_t>(engine), instance, tp, pp, static_cast<int>(device), layers.data(),
                 static_cast<uint64_t>(n));
   });
@@ -240,7 +251,7 @@ PyObject* query(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
   const uint64_t n = static_cast<uint64_t>(size_of(args[3]));
   uint64_t hits = 0, lease = 0;
   int status = 0;
-  const bool done = unlocked([&] {
+  const bool done = unlocked(kept, [&] {
     status = fn(static_cast<pf_engine_t>(engine), instance, hashes.ptrs.data(), hashes.lens.data(), n, &hits,
                 &lease);
   });
@@ -290,7 +301,7 @@ PyObject* load(PyObject*, PyObject* const* args, Py_ssize_t nargs) try {
   }
   pf_task_t task = nullptr;
   int status = 0;
-  const bool done = unlocked([&] {
+  const bool done = unlocked(kept, [&] {
     status = fn(static_cast<pf_engine_t>(engine), instance, tp, static_cast<int>(device),
                 static_cast<uint64_t>(g), name_ptrs.data(), sizes.data(), lease, id_ptrs.data(),
                 static_cast<uint64_t>(n), shm, &task);
@@ -311,7 +322,8 @@ PyObject* wait(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!begin(args, nargs, 3, &fn, &task) || !integer(args[2], &timeout)) return not_here();
   pf_task_result r = {};
   int status = 0;
-  if (!unlocked([&] { status = fn(static_cast<pf_task_t>(task), static_cast<int>(timeout), &r); })) {
+  Kept kept;
+  if (!unlocked(kept, [&] { status = fn(static_cast<pf_task_t>(task), static_cast<int>(timeout), &r); })) {
     return nullptr;
   }
   return Py_BuildValue("iiKdIIII(ddddddddd)", status, r.done, static_cast<unsigned long long>(r.bytes),

@@ -4,6 +4,9 @@ functions called are recorders of the test's own; no library, no GPU."""
 
 import ctypes as C
 import dataclasses
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -203,3 +206,34 @@ def test_wait(status, timeout):
     assert E.TaskResult.from_call(*made[1:]) == E.TaskResult.from_c(r)
     assert _calls.wait(address(WAIT(fn)), 77, 1.5) is None
     assert _calls.wait(0, 77, 1) is None
+
+
+ENDS_BESIDE_A_CALL = """
+import ctypes, sys, threading, time
+from pegaflow_amd import _calls
+
+class Layer:
+    layer_name, block_ids, block_hashes = "l", [1], [b"h"]
+    def __del__(self, print=print):
+        print("released", flush=True)
+
+class Late:  # goes with the modules, while other threads cannot have the interpreter's lock any more
+    def __del__(self, sleep=time.sleep):
+        sleep(1.0)
+
+usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
+saves = [Layer()]
+threading.Thread(target=lambda: _calls.save(usleep, 500000, "inst", 0, 0, 0, saves), daemon=True).start()
+time.sleep(0.2)
+saves.clear()  # the call has the last reference
+sys.late = Late()
+print("ending", flush=True)
+"""
+
+
+def test_interpreter_that_ends_beside_a_call():
+    """A daemon thread inside a call is ended where it takes the interpreter's lock again:
+    the objects that the call held stay, because they cannot be given back without it."""
+    proc = subprocess.run([sys.executable, "-c", ENDS_BESIDE_A_CALL], capture_output=True, text=True, timeout=60,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert proc.returncode == 0 and proc.stdout == "ending\n", (proc.returncode, proc.stdout, proc.stderr)
