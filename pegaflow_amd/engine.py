@@ -7,6 +7,7 @@ offload.rs:293-659)."""
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 from dataclasses import dataclass
 from typing import Sequence
 
@@ -16,10 +17,12 @@ from . import _lib
 from ._lib import check
 from .transfer import LayerTransferData, TransferMode
 
-try:
-    from . import _calls  # built beside libpegahip.so (csrc/py/pf_calls.cpp)
-except ImportError as exc:
-    raise ImportError(f"pegaflow_amd/_calls.so is missing: build it with `make -C pegaflow_amd/csrc` ({exc})") from exc
+# The calls of a request without ctypes (csrc/py/pf_calls.cpp), where the module was
+# built for this interpreter; every call has its ctypes form beside it.
+if importlib.util.find_spec(f"{__package__}._calls") is not None:
+    from . import _calls
+else:
+    _calls = None
 
 LOAD_STATE_PENDING = 0
 LOAD_STATE_SUCCESS = 1
@@ -120,7 +123,7 @@ class Task:
         self._keep = keep
 
     def wait(self, timeout_ms: int = -1) -> TaskResult:
-        made = _calls.wait(_address("pf_task_wait"), _handle(self), timeout_ms)
+        made = _calls and _calls.wait(_address("pf_task_wait"), _handle(self), timeout_ms)
         if made is not None:
             status, *fields = made
             check(status)
@@ -392,8 +395,8 @@ class PegaEngine:
 
     def batch_save_kv_blocks(self, instance_id: str, tp_rank: int, pp_rank: int, device_id: int,
                              saves: Sequence[LayerSave] | PackedSaves) -> None:
-        status = _calls.save(_address("pf_engine_batch_save"), _handle(self), instance_id, tp_rank, pp_rank,
-                             device_id, saves)
+        status = _calls and _calls.save(_address("pf_engine_batch_save"), _handle(self), instance_id, tp_rank,
+                                        pp_rank, device_id, saves)
         if status is not None:
             check(status)
             return
@@ -403,7 +406,7 @@ class PegaEngine:
 
     def query_prefix(self, instance_id: str, hashes: Sequence[bytes]) -> tuple[int, int]:
         """-> (hit blocks, lease id); lease 0 when nothing hit."""
-        made = _calls.query(_address("pf_engine_query_prefix"), _handle(self), instance_id, hashes)
+        made = _calls and _calls.query(_address("pf_engine_query_prefix"), _handle(self), instance_id, hashes)
         if made is not None:
             check(made[0])
             return made[1], made[2]
@@ -421,8 +424,8 @@ class PegaEngine:
                                          dest_block_ids_by_group: Sequence[Sequence[int | None]],
                                          load_state: LoadState | None = None) -> Task:
         shm = load_state.shm_name if load_state is not None else None
-        made = _calls.load(_address("pf_engine_batch_load"), _handle(self), instance_id, tp_rank, device_id,
-                           layer_groups, lease, dest_block_ids_by_group, shm)
+        made = _calls and _calls.load(_address("pf_engine_batch_load"), _handle(self), instance_id, tp_rank,
+                                      device_id, layer_groups, lease, dest_block_ids_by_group, shm)
         if made is not None:
             check(made[0])
             return Task(C.c_void_p(made[1]))

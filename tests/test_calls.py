@@ -5,8 +5,11 @@ functions called are recorders of the test's own; no library, no GPU."""
 import ctypes as C
 import dataclasses
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
+import types
 
 import numpy as np
 import pytest
@@ -206,6 +209,58 @@ def test_wait(status, timeout):
     assert E.TaskResult.from_call(*made[1:]) == E.TaskResult.from_c(r)
     assert _calls.wait(address(WAIT(fn)), 77, 1.5) is None
     assert _calls.wait(0, 77, 1) is None
+
+
+def test_module_is_found_by_the_interpreter_it_was_built_for_alone(tmp_path):
+    """The file carries the interpreter's tag; a package that holds one of another
+    interpreter, or none, is imported without it."""
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert os.path.basename(_calls.__file__) == "_calls" + suffix
+    package = tmp_path / "pegaflow_amd"
+    package.mkdir()
+    for name in os.listdir(os.path.dirname(E.__file__)):
+        if name.endswith(".py"):
+            shutil.copy(os.path.join(os.path.dirname(E.__file__), name), package)
+    (package / "_calls.cpython-399-x86_64-linux-gnu.so").write_bytes(b"of another interpreter")
+    proc = subprocess.run([sys.executable, "-c", "import pegaflow_amd.engine as e; print(e._calls)"], cwd=tmp_path,
+                          capture_output=True, text=True, timeout=60, env={**os.environ, "PYTHONPATH": str(tmp_path)})
+    assert proc.returncode == 0 and proc.stdout == "None\n", (proc.stdout, proc.stderr)
+
+
+@pytest.mark.parametrize("native", [True, False], ids=["module", "ctypes"])
+def test_calls_of_an_engine_with_and_without_the_module(native, monkeypatch):
+    saves, loads, queries = [], [], []
+
+    def query(engine, instance, ptrs, lens, n, hits, lease):
+        queries.append((engine, instance, hashes_at(ptrs, lens, n)))
+        hits[0], lease[0] = 2, 9
+        return 0
+
+    def wait(task, timeout_ms, out):
+        assert (task, timeout_ms) == (0xABCDEF, 70)
+        out[0].done, out[0].bytes, out[0].paths = 1, 4096, _lib.PF_TASK_PATH_STAGED
+        return 0
+
+    record_save = _record_saves(saves)
+    lib = types.SimpleNamespace(
+        pf_engine_batch_save=SAVE(lambda *a: record_save(*a) - 3), pf_engine_query_prefix=QUERY(query),
+        pf_engine_batch_load=_record_loads(loads), pf_task_wait=WAIT(wait), pf_task_destroy=lambda t: 0,
+        pf_engine_destroy=lambda e: 0)
+    monkeypatch.setattr(E._lib, "load", lambda: lib)
+    monkeypatch.setattr(E, "_addresses", {})
+    if not native:
+        monkeypatch.setattr(E, "_calls", None)
+    eng = object.__new__(E.PegaEngine)
+    eng._lib, eng.handle = lib, C.c_void_p(5)
+    eng.batch_save_kv_blocks("inst", 1, 2, 3, [E.LayerSave("l0", [4, 0], [b"a", b"b"])])
+    assert saves == [(5, b"inst", 1, 2, 3, [(b"l0", [4, 0], [b"a", b"b"], True, True, True)])]
+    assert eng.query_prefix("inst", [b"a", b"b"]) == (2, 9) and queries == [(5, b"inst", [b"a", b"b"])]
+    task = eng.batch_load_kv_blocks_multi_layer("inst", 1, 3, [["l0"]], 9, [[6, None]])
+    assert loads == [(5, b"inst", 1, 3, [[b"l0"]], 9, [[6, -1]], None)]
+    result = task.wait(70)
+    assert (result.done, result.bytes, result.paths) == (True, 4096, ("staged",))
+    task.close()
+    eng.handle = None
 
 
 ENDS_BESIDE_A_CALL = """
