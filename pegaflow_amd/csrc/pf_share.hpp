@@ -68,6 +68,12 @@ ShareCut plan_link_share(size_t n_units, uint64_t want, UnitAt unit_at) {
   return cut;
 }
 
+// The same where pages are packed whole: pages at the end of a chunk of `count`.
+constexpr uint64_t link_share_pages(uint64_t count, uint64_t page_bytes) {
+  const uint64_t pages = link_share_bytes(count * page_bytes) / page_bytes;
+  return pages < count ? pages : 0;
+}
+
 // A workgroup of a share moves a tile of one fragment at a time.  Full tiles keep
 // the link busy with 16 workgroups on the way out, whose stores nobody waits for,
 // and with 32 on the way in; more of them slow the rest of the launch (524 MB saved

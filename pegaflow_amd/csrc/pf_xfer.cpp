@@ -548,8 +548,7 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   }
   for (size_t ci = 0; may_share && ci < chunks.size(); ++ci) {
     const uint64_t count = chunks[ci].count;
-    const uint64_t pages = link_share_bytes(count * pack.page_bytes) / pack.page_bytes;
-    if (pages < count && count <= kMaxSharedTileBlocks) shared_pages[ci] = pages;
+    if (count <= kMaxSharedTileBlocks) shared_pages[ci] = link_share_pages(count, pack.page_bytes);
   }
   if (on_side && may_share) {
     on_side = std::count(shared_pages.begin(), shared_pages.end(), 0u) != 0;
@@ -582,7 +581,7 @@ int Xfer::run_page_pack(std::vector<LayerPlan>& plans, const PagePack& pack, uin
   std::vector<size_t> plan_order(n_plans);
   for (size_t pi = 0; pi < n_plans; ++pi) plan_order[pi] = pi;
   auto tiles_of_plan = [&](size_t pi) {
-    return (plans[pi].frag_bytes + kStagedTileBytes - 1) / kStagedTileBytes;
+    return staged_tiles(plans[pi].frag_bytes);
   };
   std::stable_sort(plan_order.begin(), plan_order.end(),
                    [&](size_t a, size_t b) { return tiles_of_plan(a) > tiles_of_plan(b); });
@@ -1389,78 +1388,31 @@ int Xfer::run_impl(const pf_layer_blocks* layers, uint64_t n_layers, int path, b
     };
     auto launch_group = [&](bool to_far) -> int {
       if (us - ui == 1) return launch_tiles(units_host[ui], to_far, s, share);
-      // Workgroups the one-launch form would start: the rows form (up to
-      // kRowsLaunchUnits units) starts every row with the tiles of the largest
-      // fragment and the segments of the widest unit; the units-inner form also
-      // gives every unit the rows of the longest.
-      auto tiles_of = [](const BlockUnit& u) {
-        return (u.frag_bytes + kStagedTileBytes - 1) / kStagedTileBytes;
-      };
       uint32_t max_blocks = 0, max_seg = 0;
-      uint64_t max_frag = 0, max_tiles = 0, total_rows = 0;
+      uint64_t max_frag = 0;
       for (size_t k = ui; k < us; ++k) {
         const BlockUnit& u = units_host[k];
         max_blocks = std::max(max_blocks, u.n_blocks);
         max_seg = std::max(max_seg, u.n_seg);
         max_frag = std::max(max_frag, u.frag_bytes);
-        max_tiles = std::max(max_tiles, tiles_of(u));
-        total_rows += u.n_blocks;
       }
       const size_t n_group = us - ui;
       const bool rows_form = n_group <= kRowsLaunchUnits;
-      const uint64_t started =
-          (rows_form ? total_rows : static_cast<uint64_t>(max_blocks) * n_group) * max_tiles * max_seg;
-      // Units too unlike for one grid leave it full of workgroups that find no
-      // tile.  Those are cheap but not free (they start and end at ~6 000 per
-      // microsecond), and so is every further launch (~8 us of ramp, tail and
-      // hand-over): the fill is cut into runs of units that keep three quarters
-      // of their grids busy, and goes out as one rows launch per run when that
-      // saves more idle workgroups than the launches cost.  A task over cache
-      // groups of unlike size (8 full-attention layers of 625 blocks among 40
-      // sliding-window layers of 8: 82 % of the units-inner grid idle) does:
-      // gather 240 -> 136 us, scatter 241 -> 140 us.  Layers of 72 KiB and of
-      // 8 KiB blocks in turn (44 % idle) do not: one launch 170 us, a launch
-      // per layer 242 us.
-      struct Run {
-        size_t begin, end;
-      };
-      std::vector<Run> runs;
-      uint64_t runs_started = 0;
-      for (size_t k = ui; k < us;) {
-        size_t e = k;
-        uint64_t run_useful = 0, run_rows = 0, run_tiles = 0, run_seg = 0;
-        while (e < us && e - k < kRowsLaunchUnits) {
-          const BlockUnit& u = units_host[e];
-          const uint64_t nu = run_useful + static_cast<uint64_t>(u.n_blocks) * tiles_of(u) * u.n_seg;
-          const uint64_t nr = run_rows + u.n_blocks;
-          const uint64_t nt = std::max(run_tiles, tiles_of(u));
-          const uint64_t ns = std::max<uint64_t>(run_seg, u.n_seg);
-          if (e > k && nu * 4 < nr * nt * ns * 3) break;
-          run_useful = nu;
-          run_rows = nr;
-          run_tiles = nt;
-          run_seg = ns;
-          ++e;
-        }
-        runs.push_back({k, e});
-        runs_started += run_rows * run_tiles * run_seg;
-        k = e;
-      }
-      constexpr uint64_t kIdleWorkgroupsPerUs = 6000, kLaunchUs = 8;
-      const bool in_runs = runs.size() > 1 && started > runs_started &&
-                           (started - runs_started) / kIdleWorkgroupsPerUs >
-                               (runs.size() - 1) * kLaunchUs;
+      const std::vector<LaunchRun> runs = plan_launch_runs(n_group, [&](size_t k) {
+        const BlockUnit& u = units_host[ui + k];
+        return LaunchUnit{u.n_blocks, u.n_seg, u.frag_bytes};
+      });
       int rc = timing_begin(s);
       if (rc != PF_OK) return rc;
       bool launched = false;
-      if (in_runs) {
+      if (!runs.empty()) {
         for (size_t ri = 0; ri < runs.size(); ++ri) {
-          const Run& run = runs[ri];
+          const LaunchRun& run = runs[ri];
           // (The runs of a fill are of a size: eight units each, most of the time.)
           LinkShare part = share;
           part.first = static_cast<uint32_t>(ri) * share.workgroups;
           part.all = static_cast<uint32_t>(runs.size()) * share.workgroups;
-          rc = launch_block_tiles_rows(units_dev + run.begin, units_host + run.begin,
+          rc = launch_block_tiles_rows(units_dev + ui + run.begin, units_host + ui + run.begin,
                                        static_cast<uint32_t>(run.end - run.begin), to_far, s,
                                        &launched, part);
           if (rc != PF_OK) return rc;

@@ -1068,34 +1068,55 @@ def test_tiles_of_unlike_units_are_dealt_out_once(stream, workgroups):
 
 # Staged calls of AUTO move a share of every fill over the link with the gather /
 # scatter launch (pf_share.hpp).  Layers (blocks, fragment, segments) by where the
-# fill is cut and by the launch that carries the share.
+# fill is cut and by the launch that carries the share; test_share_rule.py checks on
+# the CPU that each is cut and launched as it is meant to be.
 SHARES = {
     "tail_of_v": [(80, 32768, 2)],                                   # 5 MiB: ordered rows on the load
     "tail_of_k_and_v": [(60, 32768, 2), (5, 16384, 2)],
     "one_segment": [(40, 73728, 1)],
     "whole_layers": [(60, 32768, 2), (1, 32768, 2), (1, 16384, 1), (2, 4096, 2)],
     "whole_layer_to_the_fragment": [(61, 16384, 1), (1, 65536, 1)],  # 64 KiB and a little are wanted
+    "whole_layer_alone": [(30, 65536, 1), (4, 16384, 1)],            # no fragment of the first fits any more
     "short_tiles": [(300, 1040, 2), (100, 12304, 2)],
     "fragments_of_1k": [(1500, 1024, 1)],
     "fragment_larger_than_the_share": [(3, 262144, 2)],
     "last_layer_off_the_grid": [(60, 32768, 2), (50, 1000, 2)],
     "off_the_grid_before": [(50, 1000, 2), (60, 32768, 2)],
     "units_inner": [(7 + i, 16384, 1 + i % 2) for i in range(12)],
-    "unlike_lengths_in_runs": [(600, 16384, 2)] + [(2, 16384, 2)] * 11,
+    "unlike_lengths_in_runs": [(2, 16384, 2)] * 11 + [(600, 16384, 2)],
     "rows_folded": [(40000, 64, 1), (40000, 64, 1)],
     "most_rows_of_one_unit": [(65279, 64, 1)],
     "too_many_rows": [(65500, 64, 1)],
 }
 
 
-@pytest.mark.parametrize("copy_stream", [1, 2], ids=["side_stream", "in_order"])
+# Calls of several fills of a staging slot of 80 MiB, where the copy stream is left to
+# the call (copy_stream 0): in order when every fill can have a share, otherwise on the
+# side stream with the shares taken back.
+SHARE_SLOT = 80 << 20
+LARGE_SHARES = {
+    "every_fill_shares": [(1280, 32768, 2), (1100, 32768, 2)],
+    "one_fill_cannot_share": [(1280, 32768, 2), (1100, 32776, 2)],
+    "runs_in_the_second_fill": [(1280, 32768, 2)] + [(2, 16384, 2)] * 11 + [(600, 16384, 2)],
+}
+
+
+@pytest.mark.parametrize("copy_stream", [0, 2], ids=["default", "in_order"])
 @pytest.mark.parametrize("name", sorted(SHARES))
 def test_share_of_the_link_matches_oracle(name, copy_stream, stream):
-    rng = np.random.default_rng(zlib.crc32(name.encode()))
-    cases = [Case(rng, num_blocks=n + 9, seg=seg, segments=segments, n_ids=n) for n, seg, segments in SHARES[name]]
+    _share_roundtrip(SHARES[name], BlockTransfer(auto_staged_min_bytes=1, copy_stream=copy_stream), stream)
+
+
+@pytest.mark.parametrize("name", sorted(LARGE_SHARES))
+def test_shares_of_several_large_fills_match_oracle(name, stream):
+    _share_roundtrip(LARGE_SHARES[name], BlockTransfer(staging_slot_bytes=SHARE_SLOT, auto_staged_min_bytes=1), stream)
+
+
+def _share_roundtrip(spec, x, stream):
+    rng = np.random.default_rng(zlib.crc32(repr(spec).encode()))
+    cases = [Case(rng, num_blocks=n + 9, seg=seg, segments=segments, n_ids=n) for n, seg, segments in spec]
     sizes = [len(c.ids) * c.seg * c.segments for c in cases]
     pool = PinnedMemory(sum(sizes) + 4096)
-    x = BlockTransfer(auto_staged_min_bytes=1, copy_stream=copy_stream)
 
     def layers(lists):
         out, at = [], 0
@@ -1137,6 +1158,53 @@ def test_share_of_the_link_matches_oracle(name, copy_stream, stream):
                              host_is_src=True)
             assert np.array_equal(c.dev.copy_to_host(), cache), (c.args, len(ids))
             at += size
+    finally:
+        x.close()
+        pool.close()
+        for c in cases:
+            c.close()
+
+
+# Page-first calls of AUTO that share whole pages: slices of a page, and the pages of
+# every chunk (slots of SHARE_SLOT bytes).
+PAGE_SHARES = {
+    "unlike_slices": ([16384] * 4 + [4096] * 4, [100]),              # two launches a chunk, the first with the share
+    "every_chunk_shares": ([71680] * 20, [58, 58]),
+    "last_chunk_cannot_share": ([71680] * 20, [58, 58, 30]),         # 64 MiB a chunk: the others are taken back
+}
+
+
+@pytest.mark.parametrize("name", sorted(PAGE_SHARES))
+def test_share_of_whole_pages_matches_oracle(name, stream):
+    sizes, chunks = PAGE_SHARES[name]
+    rng = np.random.default_rng(zlib.crc32(name.encode()))
+    n = sum(chunks)
+    offsets, page, pool, idx, page_host, page_dev, ids, cases = _paged_setup(rng, sizes, num_blocks=n + 9, n=n)
+    x = BlockTransfer(staging_slot_bytes=SHARE_SLOT, auto_staged_min_bytes=1)
+    opool = np.full(pool.size, SENT, dtype=np.uint8)
+    opages = (opool.ctypes.data + idx * page).astype(np.uint64)
+    try:
+        layers = []
+        for li, c in enumerate(cases):
+            c.dev.copy_from_host(c.cache0)
+            oc = c.cache0.copy()  # keep the oracle's "device" image alive across the call
+            O.transfer_layer_paged(c.oracle_layout(oc), ids, opages, int(offsets[li]), host_is_src=False)
+            layers.append(LayerBlocks(layout=c.product_layout(), block_ids=ids, page_host=page_host,
+                                      page_host_device=page_dev, page_offset=int(offsets[li]), page_len=page,
+                                      layer_name=f"layer_{li}"))
+        x.save(layers, stream, TransferPath.AUTO)
+        stream.synchronize()
+        assert x.last_path == ST and np.array_equal(pool.as_numpy(), opool)
+        dest = rng.choice(n + 9, n, replace=False).astype(np.uint32)
+        for layer, c in zip(layers, cases):
+            c.dev.fill(SENT)
+            layer.block_ids = dest
+        x.load(layers, stream, TransferPath.AUTO)
+        stream.synchronize()
+        for li, c in enumerate(cases):
+            oc = np.full_like(c.cache0, SENT)
+            O.transfer_layer_paged(c.oracle_layout(oc), dest, opages, int(offsets[li]), host_is_src=True)
+            assert np.array_equal(c.dev.copy_to_host(), oc), li
     finally:
         x.close()
         pool.close()
