@@ -69,6 +69,41 @@ def measured_traffic(workload, alg_bytes_per_launch):
     return int(round(total)), f"profiles/{name}"
 
 
+SHARE_BASE, SHARE_PART = 64 << 10, 52   # csrc/pf_share.hpp: link_share_bytes
+SIDE_STREAM_FILL = 64 << 20             # csrc/pf_xfer.hpp: kSideStreamFillBytes
+
+
+def link_share(fill_bytes, piece):
+    """Bytes of a staging fill that its gather or scatter launch moves over the link
+    itself, in whole pieces (fragments, or pages where pages are packed whole)."""
+    share = (SHARE_BASE + fill_bytes // SHARE_PART) // piece * piece
+    return share if share < fill_bytes else 0
+
+
+def link_shares(fills, piece, copy_stream):
+    """The same of every fill of an AUTO call: none where the link copies run on a
+    side stream, as they do by choice of the call when large fills cannot all share."""
+    shares = [link_share(b, piece) for b in fills]
+    large = len(fills) > 1 and sum(fills) // len(fills) >= SIDE_STREAM_FILL
+    on_side = copy_stream == 1 or (copy_stream == 0 and large and 0 in shares)
+    return [0] * len(fills) if on_side else shares
+
+
+def staging_fills(w, n_layers, slot_bytes, group_bytes):
+    """Bytes of every staging fill of one direction of a workload."""
+    from pegaflow_amd.transfer import plan_staged_fills
+    if w["page_first"]:
+        page = n_layers * w["seg"]
+        per_slot = max(slot_bytes // page, 1)
+        return [min(per_slot, w["n"] - i) * page for i in range(0, w["n"], per_slot)]
+    block = (2 if w["split"] else 1) * w["seg"]
+    units, n_fills = plan_staged_fills([w["n"]] * n_layers, [block] * n_layers, slot_bytes, group_bytes)
+    fills = [0] * n_fills
+    for u in units:
+        fills[u.fill] += u.count * block
+    return fills
+
+
 WORKLOADS = {
     # BASELINE configs[1] (save) + configs[2] (load)
     "llama8b": dict(label="configs[1]+configs[2]: Llama-3.1-8B KV [2,8192,16,8,128] bf16",
@@ -818,8 +853,9 @@ def run_workload(args, workload, sections, torch, np):
     # `achieved` comes from the events around every launch of the timed steps
     # (above).  A second, untimed pass times the launches running alone (the link
     # copies share the kernels' stream in that mode) and splits them by direction.
-    # The launches of AUTO also move ~2 % of their bytes over the link and end with
-    # it; the second pass takes the path whose launches move bytes through HBM alone.
+    # The launches of AUTO also move ~2 % of their bytes over the link and take 7 %
+    # longer by it; the second pass takes the path whose launches move bytes through
+    # HBM alone.
     alone_path = TransferPath.STAGED if used_path == "staged" else path
     xfer.set_kernel_timing(1)
     xfer.save(save_layers, stream, alone_path)
@@ -835,12 +871,19 @@ def run_workload(args, workload, sections, torch, np):
     assert launches == alone_launches, (launches, alone_launches)
     bytes_per_launch = 2 * payload / max(launches, 1)          # payload bytes one launch moves
     # staged: every payload byte is read once and written once in HBM -> 2 x
-    # payload algorithmic bytes per launch; zero-copy: the kernel touches HBM
-    # once per payload byte and is bounded by the host link, not by HBM
+    # payload algorithmic bytes per launch, but for the launch's share of the link,
+    # which touches HBM once; zero-copy: the kernel touches HBM once per payload
+    # byte and is bounded by the host link, not by HBM
     staged_path = used_path == "staged"
-    alg_bytes = (2 if staged_path else 1) * bytes_per_launch
+    share = 0
+    if staged_path and path == TransferPath.AUTO:
+        fills = staging_fills(w, n_layers, (args.slot_mb or 512) << 20, args.group_mb << 20)
+        piece = n_layers * seg if w["page_first"] else seg
+        share = 2 * sum(link_shares(fills, piece, args.copy_stream)) / max(launches, 1)
+    alone_alg_bytes = (2 if staged_path else 1) * bytes_per_launch
+    alg_bytes = alone_alg_bytes - share
     achieved = alg_bytes / (live_launch_ms / 1e3) / 1e9
-    traffic, traffic_source = (measured_traffic(workload, alg_bytes) if staged_path
+    traffic, traffic_source = (measured_traffic(workload, alone_alg_bytes) if staged_path
                                else (None, "zero-copy launches are not profiled for HBM traffic"))
     # What a pair of events reads with nothing between them on that stream: the
     # part of avg_launch_us that is the bracket itself, not the kernel (reported,
@@ -862,12 +905,13 @@ def run_workload(args, workload, sections, torch, np):
                             f"{args.steps} timed steps",
                 "launches": launches, "avg_launch_us": round(live_launch_ms * 1e3, 2),
                 "empty_event_pair_us": round(empty_pair_us[len(empty_pair_us) // 2], 2),
-                "alg_bytes_per_launch": int(alg_bytes),
+                "alg_bytes_per_launch": int(alg_bytes), "link_share_bytes_per_launch": int(share),
                 "launches_alone": {
                     "avg_launch_us": round(alone_launch_ms * 1e3, 2),
-                    "achieved": round(alg_bytes / (alone_launch_ms / 1e3) / 1e9, 1),
-                    "save_kernel_gbps": round(alg_bytes * k_save_n / (k_save_ms / 1e3) / 1e9, 1),
-                    "load_kernel_gbps": round(alg_bytes * k_load_n / (k_load_ms / 1e3) / 1e9, 1)},
+                    "alg_bytes_per_launch": int(alone_alg_bytes),   # `traffic` is of these launches
+                    "achieved": round(alone_alg_bytes / (alone_launch_ms / 1e3) / 1e9, 1),
+                    "save_kernel_gbps": round(alone_alg_bytes * k_save_n / (k_save_ms / 1e3) / 1e9, 1),
+                    "load_kernel_gbps": round(alone_alg_bytes * k_load_n / (k_load_ms / 1e3) / 1e9, 1)},
                 "plain_copy_same_tile_gbps": round(hbm_copy_gbps, 1)}
     if staged_path:
         roofline["plain_copy_over_layers_gbps"] = {"from_caches": round(plain_gather_form, 1),

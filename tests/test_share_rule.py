@@ -8,6 +8,7 @@ import subprocess
 
 import pytest
 
+import bench
 from pegaflow_amd.transfer import plan_staged_fills
 from tests.test_gpu_blocks import LARGE_SHARES, PAGE_SHARES, SHARE_SLOT, SHARES
 
@@ -92,3 +93,27 @@ def test_page_cases_share_in_the_chunks_that_they_name(planner):
             assert sum(chunks) * page >= len(chunks) * (64 << 20)
     assert pages == {"unlike_slices": ["pages 2"], "every_chunk_shares": ["pages 1"] * 2,
                      "last_chunk_cannot_share": ["pages 1", "pages 1", "pages 0"]}
+
+
+def test_bytes_that_the_bench_charges_to_its_launches(planner):
+    """bench.py leaves the share out of what a launch moves through HBM: the same shares
+    as the planner's, for every fill of its workloads."""
+    for name, w in bench.WORKLOADS.items():
+        fills = bench.staging_fills(w, w["layers"], 512 << 20, 0)
+        segments = 2 if w["split"] else 1
+        assert sum(fills) == w["layers"] * w["n"] * segments * w["seg"]
+        if w["page_first"]:
+            page = w["layers"] * w["seg"]
+            want = [int(planner("pages", b // page, page).split()[1]) * page for b in fills]
+            shares = [bench.link_share(b, page) for b in fills]
+        else:
+            want = [int(planner("fill", f"{b // (segments * w['seg'])}:{w['seg']}:{segments}:1").split()[1]) for b in fills]
+            shares = [bench.link_share(b, w["seg"]) for b in fills]
+        assert shares == want, name
+        assert bench.link_shares(fills, 1, 1) == [0] * len(fills)
+    # The last chunk of 25 pages cannot share one: with the stream left to the call none does.
+    w = bench.WORKLOADS["dsv3_mla"]
+    page = w["layers"] * w["seg"]
+    fills = bench.staging_fills(w, w["layers"], 512 << 20, 0)
+    assert bench.link_share(fills[0], page) == 2 * page and fills[-1] == 25 * page
+    assert bench.link_shares(fills, page, 0) == [0] * 18 and sum(bench.link_shares(fills, page, 2)) == 17 * 2 * page
