@@ -335,9 +335,11 @@ typedef struct pf_xfer_config {
   uint32_t copy_stream;             /* staged path: where the link copies run.
                                        0 = default (side stream when a call has more than
                                        one staging fill, they hold 64 MiB or more each on
-                                       average and their launches cannot carry a share of the
-                                       link: PF_PATH_STAGED, fragments off the 16-byte grid), 1 = a side stream of the engine (the
-                                       copy of one unit overlaps the gather of the next),
+                                       average and their launches cannot all carry a share of
+                                       the link: PF_PATH_STAGED, fragments off the 16-byte grid,
+                                       pages larger than 64 KiB + 1/52 of a fill), 1 = a side
+                                       stream of the engine (the copy of one unit overlaps the
+                                       gather of the next),
                                        2 = the caller's stream (in order, no second queue) */
   uint64_t auto_staged_min_call_bytes; /* PF_PATH_AUTO also stages every dense layer (of 32 KiB or
                                        more) of a call whose dense layers add up to this much;
@@ -707,10 +709,13 @@ typedef struct pf_engine_config {
                                         one stream, between its gather / scatter kernels.
                                         1 = each worker moves them on a second stream of its
                                         own, so that the copy of one staging fill overlaps the
-                                        kernel of the next: a save or a load running alone gains
-                                        the kernels' time (Llama-3.1-8B shape: save 55.5 -> 56.2,
-                                        load 55.3 -> 56.0 GB/s; a save and a load at once 94.6 ->
-                                        88-93 together).  That is four streams per registered
+                                        kernel of the next.  In order the kernels move a share of
+                                        the link meanwhile, which gains as much (Llama-3.1-8B
+                                        shape, in order / copy streams: save 56.6 / 56.5, load
+                                        56.8 / 56.6 GB/s; a save and a load at once 95.2 / 85-97
+                                        together); copy streams are ahead only for fragments off
+                                        the 16-byte grid, which cannot share.  They make
+                                        four streams per registered
                                         context, and a process's streams share few hardware
                                         queues (GPU_MAX_HW_QUEUES, 4 by default): the pool looks
                                         for queues that no stream of the opposite direction

@@ -11,10 +11,12 @@ namespace pf {
 // link has nothing to do while the launch moves the fill through HBM.  The launch
 // therefore also moves a share of the fill straight between the cache and host
 // memory, with a few workgroups of its own, and the link copy is shorter by it.  A
-// launch of b bytes takes 4-6 us and b / 3.05 TB/s, in which the link moves b / 53
-// and 250-350 KB: the share ends with the launch of a full slot and a little before
-// that of a small one.  (A longer share gains nothing: the launch then waits for it
-// instead of the link copy for the launch.)  Measured on MI355X, calls back to back,
+// launch of b bytes alone takes 4-6 us and b / 3.05 TB/s, in which the link moves b / 53
+// and 250-350 KB; the share is about that much.  It does not ride along for nothing:
+// with it the launch of a full slot of 512 MiB takes 186 us instead of 176 (16 KiB
+// fragments: 193 instead of 178) for a link copy that is 10.4 MB = 181 us shorter.
+// (A longer share gains nothing: the launch then waits for it instead of the link copy
+// for the launch.)  Measured on MI355X, calls back to back,
 // save / load in us without a share, with 64 KiB and b / 44, b / 52, b / 60: one layer
 // of 20 MB 393.9 / 395.6, 390.5 / 389.4, 390.1 / 388.9, 389.9 / 389.0; 524 MB in twelve
 // 9437 / 9409, 9247 / 9194, 9254 / 9228, 9277 / 9252; 1.3 GB in four 23 352 / 23 223,

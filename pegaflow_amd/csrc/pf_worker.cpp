@@ -775,8 +775,9 @@ void GpuWorkerPool::run(Worker* w, bool is_load, NumaNode numa, std::promise<Tas
       // worker keeps to one stream: with a side stream per engine the link
       // copies of the two directions were seen on one hardware queue (a
       // process gets 4 by default) and a save and a load together shared
-      // 56 GB/s.  One stream per worker costs 1.4 % when one direction is
-      // active alone (see also prime_copy_overlap).
+      // 56 GB/s.  In order the launches carry a share of the link, so that one
+      // stream per worker costs nothing when one direction is active alone
+      // either (see also prime_copy_overlap).
       pf_xfer_config cfg;
       std::memset(&cfg, 0, sizeof(cfg));
       // With side_copy_streams the pool gives each worker a second stream for

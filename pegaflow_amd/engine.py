@@ -346,8 +346,9 @@ class PegaEngine:
         with TransferMode.KERNEL get zero-copy workers, the reference's meaning
         of that mode, instead of the per-task choice.  ``side_copy_streams``:
         every worker moves its link copies on a second stream of its own (they
-        then overlap its gather / scatter kernels: 1-2 % for a direction running
-        alone) instead of in order on its one stream; four streams per context,
+        then overlap its gather / scatter kernels) instead of in order on its one
+        stream, where the kernels carry a share of the link (as fast, but for
+        fragments off the 16-byte grid); four streams per context,
         for processes with one context per GPU (pf_engine_config)."""
         self._lib = _lib.load()
         cfg = _lib.PfEngineConfig(pool_size, int(use_hugepages), int(numa_aware), pool_shards,
