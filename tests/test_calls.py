@@ -274,11 +274,11 @@ class Layer:
 
 class Late:  # goes with the modules, while other threads cannot have the interpreter's lock any more
     def __del__(self, sleep=time.sleep):
-        sleep(1.0)
+        sleep(1.5)
 
 usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
 saves = [Layer()]
-threading.Thread(target=lambda: _calls.save(usleep, 500000, "inst", 0, 0, 0, saves), daemon=True).start()
+threading.Thread(target=lambda: _calls.save(usleep, 900000, "inst", 0, 0, 0, saves), daemon=True).start()
 time.sleep(0.2)
 saves.clear()  # the call has the last reference
 sys.late = Late()
